@@ -20,6 +20,18 @@ __device__ __forceinline__ float split_rne(float y, float C) {
   return c - (c - y);
 }
 
+// The same rounding in two operations, for P = 2^(23 - m) with m <= 10: c = y * (1 - P), then fma(y, P, c), where
+// y * P is exact and the sum too (c is y * (1 - P) rounded at y's m-bit step, or at half of it for y just above a
+// power of two, which rounds to that power either way).  Equal to the bit form for every finite y whose c is finite
+// and every y of 24 significant bits (an exhaustive check for m = 1..10); zeros come out as +0.  Both operations are
+// full rate when P is a literal or in a VGPR; with P in an SGPR the fma issues at half rate, no better than
+// split_rne.
+__device__ __forceinline__ float fma_rne(float y, float P) {
+#pragma clang fp contract(off)
+  const float c = y * (1.0f - P);
+  return __builtin_fmaf(y, P, c);
+}
+
 // An operand matrix: row stride and problem stride in elements.
 struct Operand {
   const float* p;

@@ -300,6 +300,18 @@ def test_split_rne_equals_bit_rne_on_bf16_lane_values():
     assert_bits_equal(_split_rne(sub, 7), sub, "split bf16 subnormal")
 
 
+@pytest.mark.parametrize("m", [1, 4, 5, 6, 7, 9, 10])
+def test_fma_rne_equals_bit_rne(m):
+    """fma_rne (csrc/reducer_common.h): c = y * (1 - 2^(23-m)), then fma(y, 2^(23-m), c), equals bit RNE at m
+    fraction bits for every 24-bit significand; both operations commute with powers of two and with the sign.  The
+    fma is formed in float64, where y * 2^(23-m) + c of two float32 values 23 - m binades apart is exact."""
+    y = (np.arange(1 << 23, 1 << 24, dtype=np.float64) / (1 << 23)).astype(np.float32)
+    P = 2.0 ** (23 - m)
+    c = y * np.float32(1.0 - P)
+    got = (y.astype(np.float64) * P + c.astype(np.float64)).astype(np.float32)
+    assert_bits_equal(got, _bit_rne(y, m), f"fma m={m}")
+
+
 @pytest.mark.parametrize("fmt,e,m,top", [("MXFP8_E4M3", 4, 3, 448.0), ("MXFP8_E5M2", 5, 2, 57344.0),
                                          ("MXFP6_E3M2", 3, 2, 28.0), ("MXFP6_E2M3", 2, 3, 7.5), ("MXFP4", 2, 1, 6.0)])
 def test_microsoft_even_is_clamped_ocp_rne(fmt, e, m, top):

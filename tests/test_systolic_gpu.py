@@ -558,3 +558,27 @@ def test_batched_hint_and_epilogue_errors(cuda):
     with pytest.raises(Exception, match="z0 \\+ count below 2\\^31"):
         systolic_batched(ops, lay, 2, 64, 40, 50, C, ar, HW_FINAL,
                          epilogue=_lib.SystolicEpilogue(scale=1.0, m=1, z_per_b=1, z0=2 ** 31 - 2))
+
+
+@pytest.mark.parametrize("ladder", [HW_FINAL, [(4, 5)] * 15 + [(8, 7)], [(4, 4)] * 16, [(4, 9)] * 16],
+                         ids=["hw_final", "e4m5_bf16", "e4m4", "e4m9"])
+@pytest.mark.parametrize("K,M,N", [(192, 40, 72), (192, 1024, 1024)], ids=["tiles32", "tiles64"])
+def test_scales_past_the_short_tile_add(cuda, ladder, K, M, N):
+    """Blocks whose scales leave the short tile add's range (2^46 and more, zero, 1e-38, 2^-60) before and after
+    blocks inside it: a sum that a large scale has made large must keep the long rounding in the blocks that
+    follow.  Against the general kernel, which is checked against the oracle above."""
+    from mxq import matmul
+    rng = np.random.default_rng(K + M)
+    ops = []
+    for n, lift in ((M, 1.0), (N, 0.5)):
+        P, _ = _codes(rng, K, n, scale=lift)
+        X = np.exp2(rng.integers(-3, 3, (K // 32, n))).astype(np.float32)
+        X[1, : n // 2] = np.float32(2.0 ** 46)
+        X[1, n // 2] = np.float32(2.0 ** 63)
+        X[3, 1::5] = np.float32(1e-38)
+        X[4, ::7] = 0.0
+        X[4, 1::7] = np.float32(2.0 ** -60)
+        ops += [torch.from_numpy(P).cuda(), torch.from_numpy(X).cuda()]
+    got = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder).cpu().numpy()
+    want = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder, force_general=True).cpu().numpy()
+    assert_bits_equal(got, want, f"{ladder[0]} {M}x{N}")
