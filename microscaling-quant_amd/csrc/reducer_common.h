@@ -26,10 +26,22 @@ __device__ __forceinline__ float split_rne(float y, float C) {
 // and every y of 24 significant bits (an exhaustive check for m = 1..10); zeros come out as +0.  Both operations are
 // full rate when P is a literal or in a VGPR; with P in an SGPR the fma issues at half rate, no better than
 // split_rne.
-__device__ __forceinline__ float fma_rne(float y, float P) {
+__device__ __forceinline__ float fma_rne(float y, float P, float one_less_P) {
 #pragma clang fp contract(off)
-  const float c = y * (1.0f - P);
+  const float c = y * one_less_P;
   return __builtin_fmaf(y, P, c);
+}
+__device__ __forceinline__ float fma_rne(float y, float P) { return fma_rne(y, P, 1.0f - P); }
+
+// A block's scales allow the short tile add when each is zero or a power of two with |x| in [xs_lo, xs_hi]
+// (bit patterns, from the host): a reduction's sum S, of at most 8 significant bits, then times a scale product is
+// exact and normal, so bf16(S * scale) = S * scale and the tile add is one fma and one rounding to bf16.  That
+// rounding (fma_rne) also needs |C + S * scale| below 2^112: it is while no scale has been above xs_hi, so one that
+// is (bit 1) denies the short add to every later block too.
+__device__ __forceinline__ uint32_t scale_denies(float x, uint32_t lo, uint32_t hi) {
+  const uint32_t u = f2u(x) & 0x7FFFFFFFu;
+  const bool exact = u == 0u || ((u & 0x007FFFFFu) == 0u && u >= lo && u <= hi);
+  return (exact ? 0u : 1u) | (u > hi ? 2u : 0u);
 }
 
 // An operand matrix: row stride and problem stride in elements.

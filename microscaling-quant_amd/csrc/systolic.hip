@@ -183,17 +183,6 @@ struct LaneConsts {
   }
 };
 
-// A block's scales allow the short tile add when each is zero or a power of two with |x| in [xs_lo, xs_hi]
-// (bit patterns, from the host): the sum S, of at most 8 significant bits, then times a scale product is exact and
-// normal, so bf16(S * scale) = S * scale and the tile add is one fma and one rounding to bf16.  That rounding
-// (fma_rne) also needs |C + S * scale| below 2^112: it is while no scale has been above xs_hi, so one that is
-// (bit 1) denies the short add to every later block too.
-__device__ __forceinline__ uint32_t scale_denies(float x, uint32_t lo, uint32_t hi) {
-  const uint32_t u = f2u(x) & 0x7FFFFFFFu;
-  const bool exact = u == 0u || ((u & 0x007FFFFFu) == 0u && u >= lo && u <= hi);
-  return (exact ? 0u : 1u) | (u > hi ? 2u : 0u);
-}
-
 // Scales a thread's staged A rows by 2^a_exp[lane of the row] on the way to LDS.  A thread always stages the
 // same rows of a stage (stages start at multiples of 32 and SIZE | 32), so the exponents are fixed per thread.
 template <int W, int NT, int SIZE>

@@ -24,9 +24,9 @@
 //                        first level A's rows are staged times 2^(6 + m_1), so a product is in units of that
 //                        level's subnormal step and lane(p) = rint(trunc(a' b)) (the flush under half a step is
 //                        subsumed).  Every add is one float32 add, exact on e4 levels (integers below 2^24), and
-//                        RNE at the level's m (Veltkamp's split, split_rne), which needs no units (m never falls,
+//                        RNE at the level's m (fma_rne, two operations), which needs no units (m never falls,
 //                        so a later level's grid is never coarser than its inputs'); on bf16 levels the float32
-//                        add of two 8-bit values rounds once more, harmlessly (24 >= 2 * 8 + 1).  3 + 4 VALU
+//                        add of two 8-bit values rounds once more, harmlessly (24 >= 2 * 8 + 1).  3 + 3 VALU
 //                        operations per product, all full-rate but the rint.
 //   k_anchor_fast        MXGEMMINI, no emin, equal level widths within each tree (no regridding: a tree is the
 //                        exact integer sum of its terms on one grid), bf16 tree lanes.  Pass 1 takes the anchor
@@ -355,25 +355,31 @@ __device__ __forceinline__ bool fast_verdict(const TreeArgs& a, uint32_t max_a, 
   return ok;
 }
 
-// The block's scales of a thread's TM x TN outputs (zero outside C), with the largest |scale| bit pattern.
+// The block's scales of a thread's TM x TN outputs (zero outside C), with the largest |scale| bit pattern; returns
+// what scale_denies says of them.
 template <int TM, int TN>
-__device__ __forceinline__ void block_scales(const TreeArgs& a, int64_t g, int64_t mr, int64_t nc,
-                                             float (&scale)[TM][TN], uint32_t& max_x) {
+__device__ __forceinline__ uint32_t block_scales(const TreeArgs& a, int64_t g, int64_t mr, int64_t nc,
+                                                 float (&scale)[TM][TN], uint32_t& max_x, uint32_t xs_lo,
+                                                 uint32_t xs_hi) {
   float xa[TM], xb[TN];
+  uint32_t denies = 0u;
 #pragma unroll
   for (int x = 0; x < TM; ++x) {
     xa[x] = mr + x < a.M ? a.XA[g * a.M + mr + x] : 0.0f;
     max_x = umax(max_x, f2u(xa[x]) & 0x7FFFFFFFu);
+    denies |= scale_denies(xa[x], xs_lo, xs_hi);
   }
 #pragma unroll
   for (int y = 0; y < TN; ++y) {
     xb[y] = nc + y < a.N ? a.XB[g * a.N + nc + y] : 0.0f;
     max_x = umax(max_x, f2u(xb[y]) & 0x7FFFFFFFu);
+    denies |= scale_denies(xb[y], xs_lo, xs_hi);
   }
 #pragma unroll
   for (int x = 0; x < TM; ++x)
 #pragma unroll
     for (int y = 0; y < TN; ++y) scale[x][y] = xa[x] * xb[y];
+  return denies;
 }
 
 template <int TM, int TN>
@@ -401,17 +407,23 @@ __device__ __forceinline__ void lds_row(const float (*src)[W], int r, int c, flo
 
 // Per-level constants of the fast adder tree, built on the host (make_fast_levels).
 struct FastLevels {
-  float split[5];     // split_rne's constant 2^(23 - m) + 1 at each level's m (bf16: 7)
+  float pow[5];       // fma_rne's constant P = 2^(23 - m) at each level's m (bf16: 7)
+  float low[5];       // and 1 - P
   float a_scale;      // A's rows are staged times this: 2^(6 + m_1) for an e4 first level, else 1
   float out_scale;    // root -> value: 1 / a_scale
   uint32_t pmask;     // product truncation to prod_m fraction bits
   float flush_thr;    // bf16 first level: |product| below this becomes +0
   float prod_max;     // bound on max|a| * max|b|: no e4 level overflows, no product saturates
+  uint32_t xs_lo, xs_hi;   // scale magnitudes (bit patterns) that allow the short tile add
 };
 
 // BM = 64: 4 x 4 outputs per thread; BM = 32: 2 x 4, for problems with too few 64 x 64 tiles to fill the chip.
+// Bound by VALU issue: 16 products, 15 level sums and their roundings a reduction.  Each level's nearest even is
+// fma_rne with its power of two held in a VGPR (from an SGPR the fma issues at half rate), and a block whose scales
+// allow it (scale_denies) adds its tile with one fma and one rounding.  512 x 4096 outputs, K = 4096, levels e4m4,
+// e4m5, e4m6, bf16: 1.107 ms a call, 1.195 with the three-operation split and a separate product, sum and roundings.
 template <int SIZE, int BM, bool FIRST_E4>
-__global__ void __launch_bounds__(256) k_adder_fast(const TreeArgs args, const FastLevels fl) {
+__global__ void __launch_bounds__(256, BM == 32 ? 4 : SIZE == 32 ? 2 : 3) k_adder_fast(const TreeArgs args, const FastLevels fl) {
   constexpr int BN = FBN, TM = BM / 16, TN = 4, NT = 256, L = ilog2(SIZE);
   static_assert((1 << L) == SIZE && KT % SIZE == 0 && L <= 5, "size: a power of two dividing 32");
   static_assert((BM / TM) * (BN / TN) == NT, "256 threads");
@@ -440,13 +452,20 @@ __global__ void __launch_bounds__(256) k_adder_fast(const TreeArgs args, const F
     la.store(sm.a[to], va);
     lb.store(sm.b[to], vb);
   };
+  float pw[L];                                      // the levels' powers of two, pinned to VGPRs
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    pw[l] = fl.pow[l];
+    asm volatile("" : "+v"(pw[l]));
+  }
   int buf = 0;
   la.load(args.A, M, K, M, 0, m0, va);
   lb.load(args.B, N, K, N, 0, n0, vb);
   stage(0);
   __syncthreads();
   float scale[TM][TN];
-  int in_block = 0;
+  bool short_add = false, large = false;            // this block's scales allow the short tile add; one was above
+  int in_block = 0;                                 // xs_hi (scale_denies)
   int64_t g = 0;
   for (int64_t k0 = 0; k0 < K; k0 += KT) {
     const bool more = k0 + KT < K;
@@ -457,7 +476,12 @@ __global__ void __launch_bounds__(256) k_adder_fast(const TreeArgs args, const F
     const int kend = (int)((K - k0 < KT) ? (K - k0) : KT);
     // rows past K are zero in LDS: zero products, which is what the reference adds past a K tail
     for (int r0 = 0; r0 < kend; r0 += SIZE) {
-      if (in_block == 0) block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x);
+      if (in_block == 0) {
+        const uint32_t denies =
+            block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x, fl.xs_lo, fl.xs_hi);
+        large = large || __any((denies & 2u) != 0u) != 0;
+        short_add = __all(denies == 0u) != 0 && !large;
+      }
       float pend[L][TM][TN];
       float root[TM][TN];
 #pragma unroll
@@ -476,7 +500,7 @@ __global__ void __launch_bounds__(256) k_adder_fast(const TreeArgs args, const F
 #pragma unroll
             for (int l = 0; l < L; ++l) {
               if (carry) {
-                if ((i >> l) & 1) v = split_rne(pend[l][x][y] + v, fl.split[l]);
+                if ((i >> l) & 1) v = fma_rne(pend[l][x][y] + v, pw[l], fl.low[l]);
                 else {
                   pend[l][x][y] = v;
                   carry = false;
@@ -486,13 +510,20 @@ __global__ void __launch_bounds__(256) k_adder_fast(const TreeArgs args, const F
             if (carry) root[x][y] = v;
           }
       }
+      // the roots stand here: sunk into the branches below, the sums keep every operand of the reduction in registers
+      // until there (185 VGPRs instead of 123 at 2 x 4 outputs)
+#pragma unroll
+      for (int x = 0; x < TM; ++x)
+#pragma unroll
+        for (int y = 0; y < TN; ++y) asm volatile("" : "+v"(root[x][y]));
       // tile_add: C (a bf16 value, never -0) plus bf16(root * scale), one rounding to bf16
 #pragma unroll
       for (int x = 0; x < TM; ++x)
 #pragma unroll
         for (int y = 0; y < TN; ++y) {
           const float r = FIRST_E4 ? root[x][y] * fl.out_scale : root[x][y];
-          C[x][y] = bf16_rne(C[x][y] + bf16_rne(r * scale[x][y]));
+          if (short_add) C[x][y] = fma_rne(__builtin_fmaf(r, scale[x][y], C[x][y]), 65536.0f);
+          else C[x][y] = bf16_rne(C[x][y] + bf16_rne(r * scale[x][y]));
         }
       in_block += SIZE;
       if (in_block == bs) {
@@ -599,7 +630,7 @@ __global__ void __launch_bounds__(256) k_anchor_fast(const TreeArgs args, const 
     // rows past K are zero in LDS (zero codes): their products are zeros and never set the anchor, as the
     // reference's missing products
     for (int r0 = 0; r0 < kend; r0 += size) {
-      if (in_block == 0) block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x);
+      if (in_block == 0) block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x, 1u, 0u);
       float c[TM][TN];
 #pragma unroll
       for (int x = 0; x < TM; ++x)
@@ -780,17 +811,30 @@ bool adder_fast_levels(const int32_t* e, const int32_t* m, int levels, const mxq
   }
   float prod_max = ar.sat_limit;                                     // no product saturates
   if (first_e4) prod_max = std::min(prod_max, adder_e4_bound(ne, mmin));
+  prod_max = std::min(prod_max, pow2_host(64));                      // the levels' roundings multiply by up to 2^22
   if (!(prod_max > 0.0f)) return false;
   *fl = FastLevels{};
   for (int l = 0; l < levels; ++l) {
     const int mm = e[l] == 8 ? 7 : m[l];
-    fl->split[l] = (float)((1u << (23 - mm)) + 1u);
+    fl->pow[l] = (float)(1u << (23 - mm));
+    fl->low[l] = 1.0f - fl->pow[l];
   }
   fl->a_scale = first_e4 ? pow2_host(6 + m[0]) : 1.0f;
   fl->out_scale = first_e4 ? pow2_host(-(6 + m[0])) : 1.0f;
   fl->pmask = ~((1u << (23 - ar.prod_m)) - 1u);
   fl->flush_thr = first_e4 ? 0.0f : ar.flush_thr;
   fl->prod_max = prod_max;
+  // The short tile add (scale_denies): a root of at most 8 significant bits, a multiple of level 1's step (e4) or of
+  // a kept product's last bit (bf16), below 2^top, times scales of 2^-L .. 2^H is exact in bf16 and normal when
+  // 2L <= 126 + log2 of that step, and leaves C below 2^112 when top + 2H <= 98: as the systolic kernels' lanes.
+  fl->xs_lo = 1u;                                                    // empty range: always the rounded tile add
+  fl->xs_hi = 0u;
+  const int low = first_e4 ? -(6 + m[0]) : (int)std::floor(std::log2((double)ar.flush_thr)) - ar.prod_m;
+  const int top = (int)std::ceil(std::log2((double)prod_max)) + levels + 1;
+  if ((bf16 || prev <= 7) && 126 + low >= 0 && top <= 98) {
+    fl->xs_lo = (uint32_t)(127 - std::min(59, (126 + low) / 2)) << 23;
+    fl->xs_hi = (uint32_t)(127 + std::max(0, std::min(45, (98 - top) / 2))) << 23;
+  }
   return true;
 }
 

@@ -296,3 +296,27 @@ def test_trees_against_reference_fixtures(cuda, case):
     else:
         Y = matmul.adder_tree(*ops, ar, kw.pop("schedule"), **kw)
     assert_bits_equal(Y.cpu().numpy(), z[f"{name}_Y"], f"{tree} tree {name}")
+
+
+@pytest.mark.parametrize("size,levels", [(16, [(4, 4), (4, 5), (4, 6), (8, 7)]), (16, [(8, 7)] * 4), (8, [(4, 7)] * 3),
+                                         (4, [(4, 9)] * 2), (32, [(4, 4)] * 4 + [(8, 7)])],
+                         ids=["readme", "bf16", "e4m7", "e4m9", "size32"])
+@pytest.mark.parametrize("K,M,N", [(192, 40, 72), (192, 2048, 4096)], ids=["tiles32", "tiles64"])
+def test_adder_scales_past_the_short_tile_add(cuda, size, levels, K, M, N):
+    """Blocks whose scales leave the short tile add's range before and after blocks inside it, against the general
+    kernel (checked against the oracle above)."""
+    from mxq import matmul
+    rng = np.random.default_rng(size + M)
+    ops = []
+    for n, lift in ((M, 1.0), (N, 0.25)):
+        P, _ = _codes(rng, K, n, scale=lift)
+        X = np.exp2(rng.integers(-3, 3, (K // 32, n))).astype(np.float32)
+        X[1, : n // 2] = np.float32(2.0 ** 46)
+        X[1, n // 2] = np.float32(2.0 ** 63)
+        X[3, 1::5] = np.float32(1e-38)
+        X[4, ::7] = 0.0
+        X[4, 1::7] = np.float32(2.0 ** -60)
+        ops += _t(P, X)
+    got = matmul.adder_tree(*ops, matmul.MXGEMMINI(), levels, size).cpu().numpy()
+    want = matmul.adder_tree(*ops, matmul.MXGEMMINI(), levels, size, force_general=True).cpu().numpy()
+    assert_bits_equal(got, want, f"{levels} {M}x{N}")
