@@ -582,3 +582,54 @@ def test_scales_past_the_short_tile_add(cuda, ladder, K, M, N):
     got = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder).cpu().numpy()
     want = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder, force_general=True).cpu().numpy()
     assert_bits_equal(got, want, f"{ladder[0]} {M}x{N}")
+
+
+SMALL_LADDERS = {
+    "hw_final": (("MXGEMMINI",), HW_FINAL, 16), "e4m4": (("MXGEMMINI",), [(4, 4)] * 16, 16),
+    "e4m5_bf16_8": (("MXGEMMINI",), [(4, 5)] * 7 + [(8, 7)], 8), "e4m9_4": (("MXGEMMINI",), [(4, 9)] * 4, 4),
+    "bf16": (("MXGEMMINI",), [(8, 7)] * 16, 16), "e5m6": (("MXGEMMINI",), [(5, 6)] * 16, 16),
+    "e5m5_e7m10_32": (("MXGEMMINI",), [(5, 5)] * 16 + [(7, 10)] * 16, 32),
+    "mxquant_hw": (("MXQUANT", 4, 3), HW_FINAL, 16), "mxquant_e6m9": (("MXQUANT", 5, 10), [(6, 9)] * 16, 16),
+    "mxquant_falling_8": (("MXQUANT", 4, 3), [(5, 6)] * 4 + [(4, 3)] * 4, 8),
+    "mxquant_float_4": (("MXQUANT", 8, 7), [(8, 10)] * 4, 4), "mxquant_e5m6_32": (("MXQUANT", 5, 2), [(5, 6)] * 32, 32),
+}
+
+
+@pytest.mark.parametrize("name", SMALL_LADDERS)
+@pytest.mark.parametrize("K,M,N", [(1, 1, 1), (96, 1, 17), (4099, 1, 70), (2080, 3, 33), (333, 8, 130), (1000, 17, 64),
+                                   (160, 70, 515), (64, 520, 2050)])
+def test_few_outputs(cuda, name, K, M, N):
+    """The kernel for few outputs, at the edges of its tiles (1, 4, 8 and 16 rows, 16 to 64 columns), rounds (of up to
+    4096 rows of K) and K tails, for every datapath it has, against the general kernel (checked against the oracle
+    above)."""
+    from mxq import matmul
+    ar_args, ladder, size = SMALL_LADDERS[name]
+    ar = getattr(matmul, ar_args[0])(*ar_args[1:])
+    rng = np.random.default_rng(K + M + N)
+    ops = [torch.from_numpy(np.ascontiguousarray(x)).cuda()
+           for x in (*_codes(rng, K, M, mode="rne"), *_codes(rng, K, N, scale=0.02))]
+    got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
+    want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
+    assert_bits_equal(got, want, f"{name} {M}x{N}, K={K}")
+
+
+@pytest.mark.parametrize("name", ["hw_final", "e4m4", "e5m6", "mxquant_hw", "mxquant_e6m9"])
+def test_few_outputs_fall_back(cuda, name):
+    """Codes and scales the fast datapaths refuse (specials, products past the overflow bound, odd scales), in some
+    workgroups' operands and not in others'."""
+    from mxq import matmul
+    ar_args, ladder, size = SMALL_LADDERS[name]
+    ar = getattr(matmul, ar_args[0])(*ar_args[1:])
+    rng = np.random.default_rng(11)
+    P_A, X_A = _codes(rng, 200, 9)
+    P_B, X_B = _codes(rng, 200, 150)
+    P_B[:, 64:80] *= 200.0
+    P_B[17, 100] = np.inf
+    P_B[199, 130] = np.nan
+    X_B[:, 20:30] = np.float32(2.0 ** 70)
+    X_B[2, 32:48] = np.float32(3e-39)
+    X_A[1, 3] = np.float32(1.5)
+    ops = [torch.from_numpy(x).cuda() for x in (P_A, X_A, P_B, X_B)]
+    got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
+    want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
+    assert_bits_equal(got, want, name)
