@@ -9,39 +9,30 @@
 //
 // Operands are strided and batched: element (r, c) of problem z of an operand sits at base + z*batch + r*ld + c.
 //
-// A fast kernel, then the general one:
-//   k_systolic_fast MXGEMMINI with size in {4, 8, 16, 32}, lanes (4, m <= 9) of non-decreasing m, optionally a
-//                   last (8, 7) lane, prod_m <= every e4 lane's m (checked on the host).  A's rows are staged
-//                   into LDS times 2^(6 + m) of their lane, so an e4 lane works in units of its subnormal step
-//                   2^-(6+m):
-//                      p = rint(trunc(a' * b))      float32 multiply, mask the dropped significand bits,
-//                                                   round to an integer = lane(p) (the flush below
-//                                                   2^prod_floor is under half a step, so it is subsumed)
-//                      S = rne_m(S + p)             the sum is an exact integer below 2^24; RNE at m fraction
-//                                                   bits (fma_rne under HW_FINAL, whose constants are literals,
-//                                                   else Veltkamp's split, split_rne) is the lane rounding
-//                                                   (identity below 2^(m+1))
-//                   6 VALU operations per emulated MAC under HW_FINAL, else 7, all but the rint full-rate on
-//                   gfx950; the sum is rescaled by 2 when m steps up.  The bf16 lane and the tile add are one float32 add of two
-//                   values of at most 8 significant bits followed by RNE to bf16, which equals the reference's
-//                   exact add with one rounding (double rounding through 24 bits is harmless for 8-bit
-//                   operands: 24 >= 2*8 + 1).
-//                   While it computes, each workgroup keeps the largest |a|, |b| and scale it has read.  Its
-//                   results are exact when those are finite, max|a| < 2^100 and max|a| * max|b| stays under
-//                   the ladder's overflow bound; then it writes its tile and a 0 flag, otherwise only a 1 flag.
-//   k_systolic_fast64  the same check and results for ladders ending in a bf16 lane on 64 x 64 tiles, when the
-//                   operands need no bounds checks (hints and the epilogue as above): 64-row stages loaded
-//                   straight into LDS, the lanes in value units (a product rounded to its lane's step by adding
-//                   and subtracting a constant, full rate, no staging scale or rescale), eight waves.  7
-//                   operations per MAC under HW_FINAL, all full rate: with the two-operation rounding and the
-//                   fused short tile add 512 x 4096 outputs over K = 4096 take 0.954 ms, with the three-operation
-//                   split and a separate product, sum and bit rounding 1.066.
-//   k_systolic_small  (systolic_small_impl.h) products of few outputs, whose waves share K, and the ladders of wide
-//                   lanes and MXQUANT's, which the kernels above do not take.
-//   k_systolic_gen  the full per-step rule for any codes, any lanes (e <= 8), MXGEMMINI or MXQUANT, NaN, Inf,
-//                   saturation and overflow included.  After a fast kernel its flagged form
-//                   (k_systolic_gen_flagged) computes only the tiles whose flag is 1; alone (no fast case, or
-//                   forced) it computes everything.
+// The fast datapaths (systolic_common.h: Datapath), for MXGEMMINI's e4 ladders (HW_FINAL's constants as literals), its
+// ladders of wider lanes and MXQUANT's, are exact when the codes and scales they read are finite, max|a| < 2^100 and
+// max|a| * max|b| is under the ladder's bound.  Their kernels:
+//   k_systolic_tile   (systolic_tile_impl.h) tiles of 64 x 64 or 32 x 32 outputs.  While it computes, each workgroup
+//                     keeps the largest |a|, |b| and scale it has read; if they allow it writes its tile and a 0 flag,
+//                     otherwise only a 1 flag.
+//   k_systolic_small  (systolic_small_impl.h) products of few outputs, whose waves share K; a workgroup whose operands
+//                     are refused computes its outputs by the general rule itself.
+//   k_systolic_fast   e4 ladders with blocks of other sizes than 32, in units of the lane's subnormal step:
+//                     MXGEMMINI with size in {4, 8, 16, 32}, lanes (4, m <= 9) of non-decreasing m, optionally a
+//                     last (8, 7) lane, prod_m <= every e4 lane's m (checked on the host).  A's rows are staged into
+//                     LDS times 2^(6 + m) of their lane, so
+//                        p = rint(trunc(a' * b))      float32 multiply, mask the dropped significand bits, round to
+//                                                     an integer = lane(p) (the flush below 2^prod_floor is under
+//                                                     half a step, so it is subsumed)
+//                        S = rne_m(S + p)             the sum is an exact integer below 2^24; RNE at m fraction bits
+//                     and the sum is rescaled by 2 when m steps up.  The bf16 lane and the tile add are one float32
+//                     add of two values of at most 8 significant bits followed by RNE to bf16, which equals the
+//                     reference's exact add with one rounding (double rounding through 24 bits is harmless for
+//                     8-bit operands: 24 >= 2*8 + 1).  Its check and flags are k_systolic_tile's.
+//   k_systolic_gen    the full per-step rule for any codes, any lanes (e <= 8), MXGEMMINI or MXQUANT, NaN, Inf,
+//                     saturation and overflow included.  After a tile kernel its flagged form
+//                     (k_systolic_gen_flagged) computes only the tiles whose flag is 1; alone (no fast datapath, or
+//                     forced) it computes everything.
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -56,11 +47,6 @@ using namespace mxq_red;
 using namespace mxq_sys;
 
 constexpr int64_t kInnerLd = int64_t(1) << 26;     // row strides below this keep 32 * ld in a 32-bit offset
-// The fast kernel's tiles: 64 x 64, 32 x 64 or 32 x 32 outputs, the largest that still gives the chip at least
-// 4 workgroups per CU (4 waves per SIMD, as many as the 32 x 64 and 64 x 64 instances' registers allow).  With
-// the full-rate lane rounding a wave's chains keep the VALU busy at that occupancy, and a larger tile does less
-// staging per MAC: on 512 x 4096 outputs (K = 4096) 32 x 64 tiles take 1.16 ms against 1.23 ms for 32 x 32
-// (2048 workgroups); on 4096 x 4096, 64 x 64 tiles.
 
 // Whether the rows of 32-row stage s may be left out of a reduction that ends before them, per 32-column
 // group: of A only where every code is +-0 (0 * b = +-0 adds nothing), and only if every block scale holding
@@ -647,286 +633,6 @@ __global__ void __launch_bounds__(256, 4) k_systolic_fast(const SysArgs args, co
   write_tile<TM, TN>(args, z, m0 + tm * TM, n0 + tn * TN, C);
 }
 
-// ------------------------------------------------------------------------- fast datapath, 64-row stages
-// k_systolic_fast64: k_systolic_fast's datapath on 64 x 64 tiles for operands that need no bounds checks,
-// eight waves a workgroup (4 x 2 outputs a thread).
-// Its operands lie whole inside the matrices (M, N and K multiples of 64, rows 16-byte aligned, blocks of 32),
-// so every stage of 64 rows moves straight from global memory into LDS (global_load_lds_dwordx4: no registers,
-// no LDS stores, 1 KB per instruction per wave) while the previous stage is reduced; one barrier per two
-// blocks.  The lanes work in value units: a product is rounded to its lane's subnormal step 2^-(6+m) by adding
-// and subtracting 1.5 * 2^(17-m) (exact: |p| stays far below 2^(16-m) whenever the tile's results are kept),
-// so A is staged as it is, no sum is rescaled between lanes, and every operation issues at full rate.  The
-// sums, roundings and tile adds are k_systolic_fast's, value for value.  The workgroup's operand maxima are
-// read back from LDS once per stage; its verdict and flag are k_systolic_fast's, and so are the caller's hints
-// (dispatch order, skipped tiles, the reduction's stop under k_end and the check of the rows past it) and the
-// epilogue.
-constexpr int KS64 = 64;                            // rows per stage
-
-template <int SIZE, bool BF16_LAST, bool HWF, int TN>
-__global__ void __launch_bounds__(64 * 64 / (4 * TN)) k_systolic_fast64(const SysArgs args, const FastLanes fl) {
-  constexpr int BM = 64, BN = 64, TM = 4, NBS = KS64 / KT;
-  constexpr int NT = (BM / TM) * (BN / TN), NWV = NT / 64;   // threads, waves
-  static_assert(TN == 4 || TN == 2 || TN == 1, "4 x 4, 4 x 2 or 4 x 1 outputs a thread (4, 8 or 16 waves)");
-  // (launched with TN = 2: on 512 x 4096 outputs, K = 4096, 1.062 ms a call against 1.112 with TN = 4 (two waves
-  // a SIMD at 172 VGPRs) and 1.243 with TN = 1 (79 VGPRs: one workgroup a CU), the same bits)
-  typedef __attribute__((address_space(3))) void* lds_t;
-  static_assert(!HWF || (SIZE == 16 && BF16_LAST), "HW_FINAL has 16 lanes, the last bf16");
-  const LaneConsts<HWF> lc{fl};
-  // the two stage buffers are distinct arrays, each named where it is used: the compiler can then tell the
-  // direct-to-LDS loads into one from the reads of the other, and does not wait for the loads before them
-  __shared__ __align__(16) float sa0[KS64][BM], sa1[KS64][BM];
-  __shared__ __align__(16) float sb0[KS64][BN], sb1[KS64][BN];
-  __shared__ __align__(16) float xs_a[2][NBS][BM];
-  __shared__ __align__(16) float xs_b[2][NBS][BN];
-  __shared__ uint32_t denies_w[2][NBS][NWV];        // per buffer, block and wave: scale_denies of its scales
-  __shared__ uint32_t red[4][NWV];
-  const int tn = threadIdx.x % (BN / TN), tm = threadIdx.x / (BN / TN);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // the tile: from the caller's dispatch order (k_tile_order: heaviest first) when there is one, else the grid's
-  int64_t z, ty, tx;
-  bool marked = false;                              // skipped, as the order entry says (order_skip)
-  if (args.order) {
-    uint32_t t = args.order[blockIdx.x + args.tiles_x * (blockIdx.y + args.tiles_y * (int64_t)blockIdx.z)];
-    if (args.order_skip) {
-      marked = (t >> 31) != 0u;
-      t &= 0x7FFFFFFFu;
-    }
-    const uint32_t zy = t / (uint32_t)args.tiles_x;
-    tx = t - zy * (uint32_t)args.tiles_x;
-    z = zy / (uint32_t)args.tiles_y;
-    ty = zy - (uint32_t)z * (uint32_t)args.tiles_y;
-  } else {
-    z = blockIdx.z;
-    ty = blockIdx.y;
-    tx = blockIdx.x;
-  }
-  const int64_t m0 = ty * BM, n0 = tx * BN;
-  const float* A = args.A.p + z * args.A.batch + m0;
-  const float* B = args.B.p + z * args.B.batch + n0;
-  const float* XA = args.XA.p + z * args.XA.batch + m0;
-  const float* XB = args.XB.p + z * args.XB.batch + n0;
-  const int64_t K = args.K;
-  // a wave instruction moves 64 lanes x 16 bytes = 4 rows of 64 floats; a stage is 16 such row quads per
-  // operand, 16 / NWV per wave
-  constexpr int INST = KS64 / 4 / NWV;
-  float xv[NBS];
-  // the scales' loads go first: a wait the compiler places before rewriting their registers then does not
-  // wait for the stage's direct-to-LDS loads too
-  auto load_stage = [&](int64_t k, float (&da)[KS64][BM], float (&db)[KS64][BN]) __attribute__((always_inline)) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < NBS; ++q) {
-      const int64_t g = k / KT + q;
-      xv[q] = t < BM ? XA[g * args.XA.ld + t] : (t < BM + BN ? XB[g * args.XB.ld + t - BM] : 0.0f);
-    }
-#pragma unroll
-    for (int j = 0; j < INST; ++j) {
-      const int r0 = (wave * INST + j) * 4;
-      const int64_t r = k + r0 + lane / 16;
-      const int c = 4 * (lane % 16);
-      __builtin_amdgcn_global_load_lds(A + r * args.A.ld + c, (lds_t)&da[r0][0], 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(B + r * args.B.ld + c, (lds_t)&db[r0][0], 16, 0, 0);
-    }
-  };
-  uint32_t max_a = 0u, max_b = 0u, max_x = 0u;
-  // the stage's scales into LDS with their short-add verdicts, then the barrier once this wave's loads landed
-  auto finish_stage = [&](int buf) __attribute__((always_inline)) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < NBS; ++q) {
-      uint32_t denies = 0u;
-      if (t < BM + BN) {
-        max_x = umax(max_x, f2u(xv[q]) & 0x7FFFFFFFu);
-        denies = scale_denies(xv[q], fl.xs_lo, fl.xs_hi);
-        if (t < BM) xs_a[buf][q][t] = xv[q];
-        else xs_b[buf][q][t - BM] = xv[q];
-      }
-      const uint32_t dw = (__any((denies & 1u) != 0u) ? 1u : 0u) | (__any((denies & 2u) != 0u) ? 2u : 0u);
-      if (lane == 0) denies_w[buf][q][wave] = dw;
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0): the direct-to-LDS loads of this wave landed
-    __syncthreads();
-  };
-
-  float C[TM][TN];
-#pragma unroll
-  for (int x = 0; x < TM; ++x)
-#pragma unroll
-    for (int y = 0; y < TN; ++y) C[x][y] = 0.0f;
-
-  bool large = false;                               // some scale so far was above xs_hi
-  // one stage: its operand maxima read back from LDS, then its blocks reduced into C
-  auto reduce_stage = [&](const float (&ca)[KS64][BM], const float (&cb)[KS64][BN], int buf)
-                          __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < KS64 * BM / 4 / NT; ++j) {
-      const float4 qa = reinterpret_cast<const float4*>(&ca[0][0])[threadIdx.x + NT * j];
-      const float4 qb = reinterpret_cast<const float4*>(&cb[0][0])[threadIdx.x + NT * j];
-      max_a = umax(max_a, umax(umax(f2u(qa.x) & 0x7FFFFFFFu, f2u(qa.y) & 0x7FFFFFFFu),
-                               umax(f2u(qa.z) & 0x7FFFFFFFu, f2u(qa.w) & 0x7FFFFFFFu)));
-      max_b = umax(max_b, umax(umax(f2u(qb.x) & 0x7FFFFFFFu, f2u(qb.y) & 0x7FFFFFFFu),
-                               umax(f2u(qb.z) & 0x7FFFFFFFu, f2u(qb.w) & 0x7FFFFFFFu)));
-    }
-#pragma unroll
-    for (int q = 0; q < NBS; ++q) {
-      uint32_t denies = 0u;
-#pragma unroll
-      for (int v = 0; v < NWV; ++v) denies |= denies_w[buf][q][v];
-      large = large || (denies & 2u) != 0u;
-      const bool short_add = denies == 0u && !large;
-      float scale[TM][TN];
-      {
-        const float4 xa = *reinterpret_cast<const float4*>(&xs_a[buf][q][tm * TM]);
-        float fb[TN];
-        if constexpr (TN == 4) {
-          const float4 xb = *reinterpret_cast<const float4*>(&xs_b[buf][q][tn * TN]);
-          fb[0] = xb.x; fb[1] = xb.y; fb[2] = xb.z; fb[3] = xb.w;
-        } else if constexpr (TN == 2) {
-          const float2 xb = *reinterpret_cast<const float2*>(&xs_b[buf][q][tn * TN]);
-          fb[0] = xb.x; fb[1] = xb.y;
-        } else {
-          fb[0] = xs_b[buf][q][tn];
-        }
-        const float fa[TM] = {xa.x, xa.y, xa.z, xa.w};
-#pragma unroll
-        for (int x = 0; x < TM; ++x)
-#pragma unroll
-          for (int y = 0; y < TN; ++y) scale[x][y] = fa[x] * fb[y];
-      }
-#pragma unroll
-      for (int r0 = KT * q; r0 < KT * q + KT; r0 += SIZE) {
-        float S[TM][TN];
-#pragma unroll
-        for (int i = 0; i < SIZE; ++i) {
-          const float4 a4 = *reinterpret_cast<const float4*>(&ca[r0 + i][tm * TM]);
-          const float a[TM] = {a4.x, a4.y, a4.z, a4.w};
-          float b[TN];
-          if constexpr (TN == 4) {
-            const float4 b4 = *reinterpret_cast<const float4*>(&cb[r0 + i][tn * TN]);
-            b[0] = b4.x; b[1] = b4.y; b[2] = b4.z; b[3] = b4.w;
-          } else if constexpr (TN == 2) {
-            const float2 b2 = *reinterpret_cast<const float2*>(&cb[r0 + i][tn * TN]);
-            b[0] = b2.x; b[1] = b2.y;
-          } else {
-            b[0] = cb[r0 + i][tn];
-          }
-          if (BF16_LAST && i == SIZE - 1) {
-            // bf16 lane: S plus the truncated product flushed below the threshold, RNE to bf16
-#pragma unroll
-            for (int x = 0; x < TM; ++x)
-#pragma unroll
-              for (int y = 0; y < TN; ++y) {
-                float t = u2f(f2u(a[x] * b[y]) & fl.pmask);
-                t = fabsf(t) < fl.flush_thr ? 0.0f : t;
-                S[x][y] = fma_rne(S[x][y] + t, 65536.0f);
-              }
-          } else {
-            const float mg = lc.magic(i);
-#pragma unroll
-            for (int x = 0; x < TM; ++x)
-#pragma unroll
-              for (int y = 0; y < TN; ++y) {
-#pragma clang fp contract(off)
-                const float p = (u2f(f2u(a[x] * b[y]) & fl.pmask) + mg) - mg;    // lane(p)
-                S[x][y] = i == 0 ? p : lc.rne(S[x][y] + p, i);
-              }
-          }
-        }
-        if (short_add) {
-#pragma unroll
-          for (int x = 0; x < TM; ++x)
-#pragma unroll
-            for (int y = 0; y < TN; ++y) C[x][y] = fma_rne(__builtin_fmaf(S[x][y], scale[x][y], C[x][y]), 65536.0f);
-        } else {
-#pragma unroll
-          for (int x = 0; x < TM; ++x)
-#pragma unroll
-            for (int y = 0; y < TN; ++y) C[x][y] = bf16_bits(C[x][y] + bf16_bits(S[x][y] * scale[x][y]));
-        }
-      }
-    }
-  };
-
-  // a tile made only of groups the caller does not need is written as +0 (through the epilogue), uncomputed
-  if (args.skip && (args.order_skip ? marked : tile_skipped(args, z, m0, n0, BM, BN))) {
-    if (threadIdx.x == 0) args.flags[(z * args.tiles_y + ty) * args.tiles_x + tx] = 0u;
-    if (!args.c_end || n0 < args.c_end[z * args.kend_groups + m0 / 64])
-      write_tile<TM, TN>(args, z, m0 + tm * TM, n0 + tn * TN, C);
-    return;
-  }
-  // the reduction stops past the caller's k_end for these columns of A: at ks32 (a multiple of 32, as
-  // k_systolic_fast and the general kernel's pieces take it), rounded up here to a whole 64-row stage; the rows
-  // read past ks32 join the operand maxima, and every row from ks32 on is checked below
-  const int64_t ks32 = tile_kstop(args, z, m0);
-  const int64_t kst = (ks32 + KS64 - 1) / KS64 * KS64 < K ? (ks32 + KS64 - 1) / KS64 * KS64 : K;
-  if (kst > 0) {
-    load_stage(0, sa0, sb0);
-    finish_stage(0);
-  }
-  for (int64_t k0 = 0; k0 < kst; k0 += 2 * KS64) {
-    // even stage: buffer 0 reduced while stage k0 + 64 lands in buffer 1; odd stage: the other way round
-    const bool more1 = k0 + KS64 < kst;
-    if (more1) load_stage(k0 + KS64, sa1, sb1);
-    reduce_stage(sa0, sb0, 0);
-    if (!more1) break;
-    finish_stage(1);
-    const bool more2 = k0 + 2 * KS64 < kst;
-    if (more2) load_stage(k0 + 2 * KS64, sa0, sb0);
-    reduce_stage(sa1, sb1, 1);
-    if (more2) finish_stage(0);
-  }
-
-  // rows from ks32 on: exact only if A holds +-0 there and B and every remaining block scale are finite
-  // (k_suffix_flags' bytes, as k_systolic_fast reads them); bit j for the tile's 32-column group j of A, then B
-  constexpr int GT = BM / 32 + BN / 32;
-  uint32_t bad = 0u;
-  if (ks32 < K) {
-    const int64_t s0 = ks32 / KT, ga = (args.M + 31) / 32, gb = (args.N + 31) / 32;
-    for (int64_t i = threadIdx.x; i < (args.stages - s0) * GT; i += NT) {
-      const int64_t st = s0 + i / GT;
-      const int j = (int)(i % GT);
-      bool b;
-      if (j < BM / 32) {
-        const int64_t g = m0 / 32 + j;
-        b = g < ga && args.suf_a[(z * args.stages + st) * ga + g];
-      } else {
-        const int64_t g = n0 / 32 + (j - BM / 32);
-        b = g < gb && args.suf_b[(z * args.stages + st) * gb + g];
-      }
-      bad |= b ? 1u << j : 0u;
-    }
-  }
-
-  for (int off = 32; off > 0; off >>= 1) {
-    max_a = umax(max_a, (uint32_t)__shfl_xor((int)max_a, off, 64));
-    max_b = umax(max_b, (uint32_t)__shfl_xor((int)max_b, off, 64));
-    max_x = umax(max_x, (uint32_t)__shfl_xor((int)max_x, off, 64));
-    bad |= (uint32_t)__shfl_xor((int)bad, off, 64);
-  }
-  if (lane == 0) {
-    red[0][wave] = max_a;
-    red[1][wave] = max_b;
-    red[2][wave] = max_x;
-    red[3][wave] = bad;
-  }
-  __syncthreads();
-  uint32_t wa = 0u, wb = 0u, wx = 0u, wbad = 0u;
-#pragma unroll
-  for (int v = 0; v < NWV; ++v) {
-    wa = umax(wa, red[0][v]);
-    wb = umax(wb, red[1][v]);
-    wx = umax(wx, red[2][v]);
-    wbad |= red[3][v];
-  }
-  const bool ok = wbad == 0u && wa < kFastAMaxBits && wb < 0x7F800000u && wx < 0x7F800000u &&
-                  u2f(wa) * u2f(wb) <= args.fast_prod_max;
-  // the flag: bit 0, the general kernel computes the tile; bits 1..GT, which groups' left-out rows failed their
-  // check (piece_kstop)
-  if (threadIdx.x == 0) args.flags[(z * args.tiles_y + ty) * args.tiles_x + tx] = ok ? 0u : 1u | (wbad << 1);
-  if (!ok) return;
-  write_tile<TM, TN>(args, z, m0 + tm * TM, n0 + tn * TN, C);
-}
-
 // ------------------------------------------------------------------------------- general datapath
 // The BM x BN outputs at (m0, n0) of problem z.
 // The reduction runs over rows [0, kstop) of A and B (kstop = K, or a multiple of 32 the fast kernel's check
@@ -1274,59 +980,81 @@ void launch_fast(int size, bool bf16_last, bool hwf, dim3 grid, hipStream_t st, 
   }
 }
 
-// Ladders with a last bf16 lane (HW_FINAL among them); without one the compiler's schedule of this kernel
-// spills, and k_systolic_fast takes them.
-void launch_fast64(int size, bool hwf, dim3 grid, hipStream_t st, const SysArgs& a, const FastLanes& fl) {
-  if (hwf) {
-    k_systolic_fast64<16, true, true, 2><<<grid, 512, 0, st>>>(a, fl);
-    return;
-  }
-  switch (size) {
-    case 4: k_systolic_fast64<4, true, false, 2><<<grid, 512, 0, st>>>(a, fl); break;
-    case 8: k_systolic_fast64<8, true, false, 2><<<grid, 512, 0, st>>>(a, fl); break;
-    case 16: k_systolic_fast64<16, true, false, 2><<<grid, 512, 0, st>>>(a, fl); break;
-    default: k_systolic_fast64<32, true, false, 2><<<grid, 512, 0, st>>>(a, fl); break;
-  }
-}
+// Which kernel computes a call, and its tile.
+struct Plan {
+  enum Kernel { kGeneral, kSmall, kTile, kFast } kernel;
+  SmallTile small;
+  int bm, bn;              // the tile kernels' tile
+};
 
-// Whether k_systolic_fast64 takes the launch: a ladder ending in a bf16 lane, at least one 64 x 64 tile per CU
-// (256), every 64-row stage inside the operands and 16-byte aligned, blocks of 32; hints and the epilogue as
-// k_systolic_fast takes them.
-// Measured against k_systolic_fast on MXGEMMINI HW_FINAL, the same bits: 512 x 4096 outputs, K = 4096: 1.06 ms
-// against 1.16 (32 x 64 tiles); 4096 x 4096 x 4096: 7.86 against 8.18; 1024 x 4096 x 4096: 2.04 against 2.45;
-// 256 x 4096 x 4096: 0.59 against 0.66; with 128 tiles (256 x 2048) half the CUs idle: 0.59 against 0.43.
-bool takes_fast64(const SysArgs& a, int64_t count) {
-  const int64_t tiles = mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count;
-  auto aligned = [](const Operand& o) {
-    return o.ld % 4 == 0 && o.batch % 4 == 0 && reinterpret_cast<uintptr_t>(o.p) % 16 == 0;
-  };
-  return a.lane_e[a.size - 1] == 8 && a.block_size == KT && a.K > 0 &&
-         a.M % 64 == 0 && a.N % 64 == 0 &&
-         a.K % KS64 == 0 && tiles >= 256 && aligned(a.A) && aligned(a.B);
-}
+// What a launch takes: `fill` and a `round` for every 256 workgroups (one a CU) begun, at least `alone`, which that many
+// of one wave a SIMD take; `start` whatever K is.  Microseconds, measured under HW_FINAL at K = 2048 over 8 x 256 to
+// 1024 x 4096 outputs, and at K = 128 to 704 for `start`; all but `start` are proportional to K.  `fixed` is the part of
+// a workgroup's time that does not grow with the datapath's instructions (from the same on MXQUANT).
+struct Shape {
+  Plan::Kernel kernel;
+  int rows, log_cols, waves;
+  double fill, round, alone, start, fixed;
+};
+constexpr Shape kShapes[] = {
+    {Plan::kTile, 64, 6, 8, 35, 237, 275, 14, 0.0},    // 256 x 4096: 280, 512 x 4096: 508, 333 x 5632: 733
+    {Plan::kTile, 32, 5, 4, 24, 66, 172, 12, 0.1},     // 64 x 4096: 170, 256 x 2048: 180, 333 x 5632: 519
+    {Plan::kSmall, 16, 6, 8, 28, 74, 103, 20, 0.23},   // 128 x 4096: 174, 192 x 4096: 252, 512 x 2048: 324
+    {Plan::kSmall, 8, 6, 8, 14, 45, 66, 12, 0.38},     // 64 x 4096: 104, 320 x 2048: 241
+    {Plan::kSmall, 8, 6, 16, 0, 54, 53, 20, 0.38},     // 32 x 4096: 59, 64 x 4096: 111
+    {Plan::kSmall, 8, 5, 16, 1, 33, 33, 8, 0.48},      // 16 x 4096: 36
+    {Plan::kSmall, 8, 5, 8, 8, 29, 40, 8, 0.48},       // (the ladders without the sixteen-wave tiles)
+    {Plan::kSmall, 4, 6, 16, 2, 36, 37, 8, 0.57},      // 16 x 4096: 39
+    {Plan::kSmall, 4, 5, 16, 1, 22, 23, 8, 0.57},      // 32 x 1024: 24
+    {Plan::kSmall, 4, 4, 16, 5, 15, 18, 8, 0.57},      // 32 x 1024: 31
+};
+// A MAC's cost on the tile kernels by datapath (512 x 4096 outputs), HW_FINAL's being 1.
+constexpr double kMacCost[] = {1.0, 1.29, 1.36, 2.27, 2.3, 2.02};
 
-// Whether k_systolic_small takes the launch, and its tile.  It does while the outputs are fewer than 256 tiles of
-// 64 x 64, where the tile kernels leave CUs idle (past that their lower overhead wins: 256 x 4096 outputs, K = 4096,
-// take 0.53 ms on k_systolic_fast64), for up to 16 rows, which leave half of those kernels' smallest tile empty
-// (1 x 32000, K = 2048: 65 us against 337), and always for datapaths that have no other fast kernel (`only`).  The
-// tile is the largest that still makes a workgroup for every CU, two for those of eight waves: larger ones read B less often,
-// smaller ones keep more CUs busy.  1 x 5632 outputs, K = 2048: 23 us with 32 columns, 35 with 16, 25 with 64;
-// 4 x 4096, K = 4096: 4 rows by 16, 32 and 64 columns 40, 45 and 75 us; 16 x 4096: 8 by 32 67, 4 by 64 72; 32 x 4096:
-// 8 by 64 109 (141 with eight waves); 64 x 4096: 214 and 199; 128 x 4096: 16 by 64 337.  Hints that leave rows of A
-// unread (a_live) or outputs unstored (c_end) go to the tile kernels.
-bool takes_small(const SysArgs& a, int64_t count, bool only, bool final_ladder, SmallTile* t) {
-  if (a.c_end || a.a_live || a.K < 1 || a.K >= (int64_t(1) << 30) || a.B.ld >= (int64_t(1) << 18)) return false;
-  if (!only && a.M > 16 && mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= 256) return false;
-  auto wgs = [&](int rows, int log_cw) {
-    return mxq::ceil_div(a.M, rows) * mxq::ceil_div(a.N, int64_t(1) << log_cw) * count;
-  };
-  if (a.M == 1 && final_ladder) *t = {1, wgs(1, 6) >= 256 ? 6 : wgs(1, 5) >= 128 ? 5 : 4, 16};
-  else if (a.M > 8 && final_ladder && wgs(16, 6) >= 512) *t = {16, 6, 8};
-  else if (a.M > 4 && wgs(8, 6) >= 400) *t = {8, 6, 8};
-  else if (a.M > 4 && wgs(8, 6) >= 256) *t = {8, 6, final_ladder ? 16 : 8};
-  else if (a.M > 4 && wgs(8, 5) >= 256) *t = {8, 5, final_ladder ? 16 : 8};
-  else *t = {4, wgs(4, 6) >= 256 ? 6 : wgs(4, 5) >= 256 ? 5 : 4, 16};
-  return mxq::ceil_div(a.M, t->rows) <= 65535;
+Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
+  // hints that leave rows of A unread (a_live) or outputs unstored (c_end) need a tile kernel, whose own limits are
+  // blocks of 32 and a lane's offset in 32 bits; k_systolic_small's are its 32-bit rows and lane offsets
+  const bool small_ok = !a.c_end && !a.a_live && a.K < (int64_t(1) << 30) && a.B.ld < (int64_t(1) << 18);
+  const bool tile_ok = a.block_size == KT && a.A.ld < (int64_t(1) << 28) && a.B.ld < (int64_t(1) << 28);
+  const bool every_small = kind == kE4Final || kind == kMxqFinal;
+  Plan p{};
+  if (a.M == 1 && every_small && small_ok) {
+    // one row: 32 columns a workgroup while that leaves half the CUs one (K = 2048, 5632 columns: 23 us, 35 with 16,
+    // 25 with 64), 64 when that makes one for every CU (32000 columns: 65, 85 with 32)
+    auto wgs = [&](int log_cw) { return mxq::ceil_div(a.N, int64_t(1) << log_cw) * count; };
+    p.kernel = Plan::kSmall;
+    p.small = {1, wgs(6) >= 256 ? 6 : wgs(5) >= 128 ? 5 : 4, 16};
+    return p;
+  }
+  double best = 0.0;
+  for (const Shape& sh : kShapes) {
+    const bool tile = sh.kernel == Plan::kTile;
+    if (tile ? !tile_ok : !small_ok) continue;
+    if (!tile && !every_small && !(sh.rows == 4 || (sh.rows == 8 && sh.waves == 8))) continue;
+    if (!tile && mxq::ceil_div(a.M, sh.rows) > 65535) continue;
+    const int64_t n = mxq::ceil_div(a.M, sh.rows) * mxq::ceil_div(a.N, int64_t(1) << sh.log_cols) * count;
+    double t = std::max(sh.alone, sh.fill + sh.round * (double)mxq::ceil_div(n, 256));
+    t *= (sh.fixed + (1.0 - sh.fixed) * kMacCost[kind]) * (double)a.K / 2048.0;
+    if (tile && a.k_end) t *= 0.6;                    // a causal mask's half, and the uneven rest of it
+    t += sh.start;
+    if (tile && (a.skip || a.k_end)) t += 20.0;       // the dispatch order's and the suffix check's launches
+    if (p.kernel == Plan::kGeneral || t < best) {
+      best = t;
+      p.kernel = sh.kernel;
+      p.small = {sh.rows, sh.log_cols, sh.waves};
+      p.bm = p.bn = sh.rows;
+    }
+  }
+  // e4 lanes with other blocks than 32 (or wider rows): k_systolic_fast while it has a workgroup for every CU
+  if (!tile_ok && kind <= kE4 &&
+      (!small_ok || (a.M > 16 && mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= 256))) {
+    // its tiles: 64 x 64, 32 x 64 or 32 x 32 outputs, the largest that gives every CU four workgroups
+    const int64_t want = 4 * 256;
+    p.kernel = Plan::kFast;
+    p.bm = mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= want ? 64 : 32;
+    p.bn = p.bm == 64 || mxq::ceil_div(a.M, 32) * mxq::ceil_div(a.N, 64) * count >= want ? 64 : 32;
+  }
+  return p;
 }
 
 bool lanes_valid(const int32_t* e, const int32_t* m, int size) {
@@ -1342,47 +1070,37 @@ int run_systolic(const SysArgs& base, const int32_t* lane_e, const int32_t* lane
   const mxq_arith_spec& ar = base.ar;
   SysArgs a = base;
   for (int i = 0; i < a.size; ++i) { a.lane_e[i] = (int8_t)lane_e[i]; a.lane_m[i] = (int8_t)lane_m[i]; }
-  // the largest fast tile that gives every CU at least 4 workgroups (else the smallest)
-  const int64_t want = 4 * 256;
-  if (mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= want) { a.fbm = 64; a.fbn = 64; }
-  else if (mxq::ceil_div(a.M, 32) * mxq::ceil_div(a.N, 64) * count >= want) { a.fbm = 32; a.fbn = 64; }
-  else { a.fbm = 32; a.fbn = 32; }
-  const bool fast_lanes = !force_general && a.K > 0 && lanes_fast(lane_e, lane_m, a.size, ar);
-  const bool hwf = is_hw_final(lane_e, lane_m, a.size);
+  // the datapath: its constants and its bound on max|a| * max|b|
+  int kind = -1;
+  FastLanes fl;
+  const bool bf16_last = lane_e[a.size - 1] == 8, hwf = is_hw_final(lane_e, lane_m, a.size);
   if (!force_general && a.K > 0) {
-    SmallTile t;
-    FastLanes fl;
     bool high = false;
-    mxq::KernelTimer timer("systolic_small", st);
-    if (fast_lanes) {
-      if (takes_small(a, count, false, hwf, &t)) {
-        a.fast_prod_max = fast_prod_bound(lane_e, lane_m, a.size);
-        launch_small_e4(hwf ? kE4Final : kE4, lane_e[a.size - 1] == 8, a, make_fast_lanes(lane_e, lane_m, a.size, ar), t,
-                        count, st);
-        return mxq::check_launch("mxq_systolic small");
-      }
+    if (lanes_fast(lane_e, lane_m, a.size, ar)) {
+      kind = hwf ? kE4Final : kE4;
+      fl = make_fast_lanes(lane_e, lane_m, a.size, ar);
+      a.fast_prod_max = fast_prod_bound(lane_e, lane_m, a.size);
     } else if (lanes_wide(lane_e, lane_m, a.size, ar, &fl, &a.fast_prod_max)) {
-      if (takes_small(a, count, true, false, &t)) {
-        launch_small_wide(a, fl, t, count, st);
-        return mxq::check_launch("mxq_systolic small");
-      }
+      kind = kWide;
     } else if (lanes_mxquant(lane_e, lane_m, a.size, ar, a.K, &fl, &a.fast_prod_max, &high)) {
-      const bool final_ladder = hwf && !high;
-      if (takes_small(a, count, true, final_ladder, &t)) {
-        launch_small_mxquant(final_ladder ? kMxqFinal : high ? kMxqHigh : kMxq, a, fl, t, count, st);
-        return mxq::check_launch("mxq_systolic small");
-      }
+      kind = high ? kMxqHigh : hwf ? kMxqFinal : kMxq;
     }
   }
-  const bool fast64 = fast_lanes && takes_fast64(a, count);
-  if (fast64) { a.fbm = 64; a.fbn = 64; }
-  a.tiles_x = mxq::ceil_div(a.N, a.fbn);
-  a.tiles_y = mxq::ceil_div(a.M, a.fbm);
-  a.fast_prod_max = 0.0f;
-  const dim3 grid_f((unsigned)a.tiles_x, (unsigned)a.tiles_y, (unsigned)count);
+  const Plan plan = kind < 0 ? Plan{} : plan_launch(a, count, kind);
+  if (plan.kernel == Plan::kSmall) {
+    mxq::KernelTimer timer("systolic_small", st);
+    if (kind <= kE4) launch_small_e4(kind, bf16_last, a, fl, plan.small, count, st);
+    else if (kind == kWide) launch_small_wide(a, fl, plan.small, count, st);
+    else launch_small_mxquant(kind, a, fl, plan.small, count, st);
+    return mxq::check_launch("mxq_systolic small");
+  }
   const dim3 grid_g((unsigned)mxq::ceil_div(a.N, 32), (unsigned)mxq::ceil_div(a.M, 32), (unsigned)count);
-  if (fast_lanes) {
-    a.fast_prod_max = fast_prod_bound(lane_e, lane_m, a.size);
+  if (plan.kernel != Plan::kGeneral) {
+    a.fbm = plan.bm;
+    a.fbn = plan.bn;
+    a.tiles_x = mxq::ceil_div(a.N, a.fbn);
+    a.tiles_y = mxq::ceil_div(a.M, a.fbm);
+    const dim3 grid_f((unsigned)a.tiles_x, (unsigned)a.tiles_y, (unsigned)count);
     // workspace: a flag per 32 x 32 tile (W), the dispatch order (W), the suffix bytes of A's and B's groups
     const int64_t W = mxq::ceil_div(a.M, 32) * mxq::ceil_div(a.N, 32) * count;
     const int64_t total = a.tiles_x * a.tiles_y * count;
@@ -1412,12 +1130,10 @@ int run_systolic(const SysArgs& base, const int32_t* lane_e, const int32_t* lane
     }
     {
       mxq::KernelTimer timer("systolic_fast", st);
-      if (fast64)
-        launch_fast64(a.size, hwf, grid_f, st, a,
-                      make_fast_lanes(lane_e, lane_m, a.size, ar));
-      else
-        launch_fast(a.size, lane_e[a.size - 1] == 8, hwf, grid_f, st, a,
-                    make_fast_lanes(lane_e, lane_m, a.size, ar));
+      if (plan.kernel == Plan::kFast) launch_fast(a.size, bf16_last, hwf, grid_f, st, a, fl);
+      else if (kind <= kE4) launch_tile_e4(kind, bf16_last, grid_f, a, fl, st);
+      else if (kind == kWide) launch_tile_wide(grid_f, a, fl, st);
+      else launch_tile_mxquant(kind, grid_f, a, fl, st);
     }
     if (int rc = mxq::check_launch("mxq_systolic fast")) return rc;
     mxq::KernelTimer timer("systolic_general", st);

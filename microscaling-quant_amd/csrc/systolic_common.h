@@ -315,6 +315,11 @@ struct Datapath {
     if (!short_add) return bf16_bits(t);
     return KIND == kWide ? fma_rne(t, 65536.0f) : t;
   }
+  // C after the tile of a block whose scales allow the short form: MXGEMMINI's exact product joins the sum in one fma.
+  __device__ __forceinline__ float tile_add(float C, float S, float scale) const {
+    if constexpr (kind_mxq(KIND) || KIND == kWide) return add(C, tile(S, scale, true), false);
+    return fma_rne(__builtin_fmaf(S, scale, C), 65536.0f);
+  }
   // C after the tile: one rounding to bf16 (two operations while no scale has been large), or the float32 sum.
   __device__ __forceinline__ float add(float C, float t, bool large) const {
 #pragma clang fp contract(off)
@@ -322,6 +327,11 @@ struct Datapath {
     return large ? bf16_bits(C + t) : fma_rne(C + t, 65536.0f);
   }
 };
+
+// The kernels' launches, a translation unit for each family of datapaths.
+void launch_tile_e4(int kind, bool bf16_last, dim3 grid, const SysArgs& a, const FastLanes& fl, hipStream_t st);
+void launch_tile_wide(dim3 grid, const SysArgs& a, const FastLanes& fl, hipStream_t st);
+void launch_tile_mxquant(int kind, dim3 grid, const SysArgs& a, const FastLanes& fl, hipStream_t st);
 
 // k_systolic_small's tile: rows x 2^log_cw outputs a workgroup of `waves` waves.
 struct SmallTile {

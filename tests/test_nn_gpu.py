@@ -537,3 +537,26 @@ def test_softmax_tail_against_full_scores(cuda, fmt):
             assert_bits_equal(X[:kw // 32, c0:c0 + 64], wX[:kw // 32, c0:c0 + 64], f"scales z{z} t{t}")
             if kw < T:
                 assert not wP[kw:, c0:c0 + 64].any() and not wlive[z, kw // 32:, t * 2:t * 2 + 2].any()
+
+
+@pytest.mark.parametrize("B,H,Hkv,Tq,Tk,D", [(1, 8, 8, 192, 224, 64), (2, 16, 4, 320, 1184, 64), (1, 32, 32, 512, 992, 128),
+                                             (1, 16, 16, 333, 700, 64)], ids=lambda v: str(v))
+@pytest.mark.parametrize("junk", [0.5, float("nan")])
+def test_attend_keys_ahead_of_the_queries(cuda, B, H, Hkv, Tq, Tk, D, junk):
+    """A causal mask whose 64-query groups end at keys that are no multiple of 64 (cached keys ahead of the prompt): P
+    V's reduction stops inside its stages, and P^T past the stop is never written, so what its memory held must not
+    reach the product.  Against the reference's call for every pair, on the general kernel."""
+    from mxq import Scheme, matmul, schedule
+    from mxq.nn import attend
+    hw = _hw(None)
+    by_pair = Scheme("by_pair", a=lambda V: hw.a(V), b=lambda V: hw.b(V),
+                     reduce=partial(matmul.systolic, arith=matmul.MXGEMMINI(), schedule=schedule.HW_FINAL,
+                                    force_general=True))
+    g = torch.Generator(device="cuda").manual_seed(Tk)
+    q, k, v = (torch.randn(B, n, t, D, generator=g, device="cuda") for n, t in ((H, Tq), (Hkv, Tk), (Hkv, Tk)))
+    mask = torch.triu(torch.full((Tq, Tk), torch.finfo(torch.float32).min, device="cuda"), Tk - Tq + 1)[None, None]
+    held = [torch.full((1 << n,), junk, device="cuda") for n in (16, 18, 20, 22, 24)]
+    del held                                    # the allocator hands this memory out again
+    got = attend(q, k, v, mask, D ** -0.5, hw, hw)
+    want = attend(q, k, v, mask, D ** -0.5, by_pair, by_pair)
+    assert_bits_equal(got.cpu().numpy(), want.cpu().numpy(), f"{H}/{Hkv} heads, {Tq} of {Tk}")

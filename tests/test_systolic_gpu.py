@@ -633,3 +633,23 @@ def test_few_outputs_fall_back(cuda, name):
     got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
     want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
     assert_bits_equal(got, want, name)
+
+
+@pytest.mark.parametrize("name", SMALL_LADDERS)
+@pytest.mark.parametrize("K,M,N", [(64, 2048, 2048), (200, 1000, 1030), (77, 2049, 1023), (33, 1030, 2001)],
+                         ids=lambda v: str(v))
+def test_tiles_of_any_shape(cuda, name, K, M, N):
+    """Grids of 64 x 64 and 32 x 64 tiles whose operands end inside a tile, a stage or a group of four columns, for
+    every datapath, against the general kernel."""
+    from mxq import matmul
+    ar_args, ladder, size = SMALL_LADDERS[name]
+    if name == "mxquant_falling_8":
+        K = K // 8 * 8                          # (the lanes of a cut reduction are the general kernel's)
+    ar = getattr(matmul, ar_args[0])(*ar_args[1:])
+    rng = np.random.default_rng(K + M + N)
+    ops = [torch.from_numpy(np.ascontiguousarray(x)).cuda()
+           for x in (*_codes(rng, K, M, mode="rne"), *_codes(rng, K, N, scale=0.02))]
+    ops[0][K // 2, 70] = 300.0                  # one column of tiles goes to the general kernel
+    got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
+    want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
+    assert_bits_equal(got, want, f"{name} {M}x{N}, K={K}")
