@@ -35,7 +35,32 @@ namespace {
 constexpr int H = 2;          // 64-row groups per workgroup
 constexpr int RB = 64 * H;    // rows per workgroup
 constexpr int NT = 256 * H;   // threads per workgroup: 4 waves per row group
+// The most rows k_softmax_row takes: at 2048 keys 8192 rows take it 113 us and k_softmax_pt 204, 16,384 rows 361
+// and 206; at 256 keys 17 and 39, 32 and 42.
+constexpr int64_t kRowKernelRows = 8192;
 static_assert(H == 2, "a workgroup pairs a front and a back row group");
+
+// The maximum of a row's elements (lane l's e[it] its element l + 64 it), the exponentials in their place and the
+// sum of those, in torch's order.
+template <int IT>
+__device__ __forceinline__ void exp_stats(float (&e)[IT], float& mx, float& sum) {
+  mx = e[0];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) mx = mx > e[it] ? mx : e[it];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float b = __shfl_xor(mx, off, 64);
+    mx = mx < b ? b : mx;
+  }
+  sum = 0.0f;
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    e[it] = expf(e[it] - mx);
+    sum += e[it];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum = sum + __shfl_xor(sum, off, 64);
+}
 
 // torch's statistics of one row: lane l's elements l + 64 it, keys at and past `stored` taken from `tail`
 // (a mask row, through the score step) when it is not NULL, else -Inf (no part in the maximum, +0 in the sum)
@@ -48,19 +73,7 @@ __device__ __forceinline__ void row_stats(const float* __restrict__ row, int T, 
     const int idx = lane + 64 * it;
     e[it] = idx < stored ? row[idx] : (tail && idx < T ? 0.0f * score_scale + tail[idx] : -INFINITY);
   }
-  mx = e[0];
-#pragma unroll
-  for (int it = 0; it < IT; ++it) mx = mx > e[it] ? mx : e[it];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float b = __shfl_xor(mx, off, 64);
-    mx = mx < b ? b : mx;
-  }
-  sum = 0.0f;
-#pragma unroll
-  for (int it = 0; it < IT; ++it) sum += expf(e[it] - mx);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum = sum + __shfl_xor(sum, off, 64);
+  exp_stats<IT>(e, mx, sum);
 }
 
 // Where a tail's scores come from: the mask row of S row r (problem r / cols, its row r % cols reading query
@@ -219,9 +232,62 @@ __global__ void __launch_bounds__(NT) k_softmax_pt(const float* __restrict__ S, 
   }
 }
 
+// Few rows (decoding: a query a head): k_softmax_pt gives 128 rows to a workgroup, so that R rows run on R / 128
+// CUs, and one lane walks a whole row of exponentials.  Here a workgroup takes one row: each of its waves takes the
+// row's statistics (the same lane holding the same elements, so the same bits), then keeps the exponentials of
+// every W-th run of 64 keys in its registers for pass 2, where a half wave is a 32-key block.  The codes leave as
+// 4-byte stores R apart, which is what bounds it over many rows.  2048 keys: 32 rows 87 us in
+// k_softmax_pt and at most 14 here (a call's host time), 512 rows 195 -> 18 us, 4096: 202 -> 64 us.
+template <int ELEM, int MODE, int IT>
+__global__ void __launch_bounds__(256) k_softmax_row(const float* __restrict__ S, int64_t R, int T,
+                                                     float* __restrict__ PT_P, float* __restrict__ PT_X,
+                                                     mxq_block_spec s) {
+  constexpr int W = 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // workgroups go to the 8 XCDs in turn: 32 rows, a line of P^T, to one XCD, whose L2 puts their stores together
+  const uint32_t g = blockIdx.x, i = g / 8;
+  const int64_t r = g < R / 256 * 256 ? i / 32 * 256 + g % 8 * 32 + i % 32 : g;
+  const float* row = S + r * T;
+  float e[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int idx = lane + 64 * it;
+    e[it] = idx < T ? row[idx] : -INFINITY;
+  }
+  float mx, sm;
+  exp_stats<IT>(e, mx, sm);
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    if (it % W != w) continue;
+    const int k = lane + 64 * it;
+    const float pr = k < T ? (sm == 0.0f ? NAN : e[it] / sm) : 0.0f;   // past T: padding
+    uint32_t am = f2u(pr) & 0x7FFFFFFFu;               // a NaN pattern lies above +Inf: NaN wins, as torch.amax
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) am = max(am, (uint32_t)__shfl_xor((int)am, off, 64));
+    const float xs = block_scale(u2f(am), s);
+    const Div d = make_div(xs);
+    if (k < T) {
+      PT_P[(int64_t)k * R + r] = elem_qm<ELEM, MODE>(s.scale_rule ? apply_div(pr, d) : pr, s);
+      if ((lane & 31) == 0) PT_X[(int64_t)(k >> 5) * R + r] = xs;
+    }
+  }
+}
+
 template <int ELEM, int MODE>
 void launch_it(int it, dim3 grid, hipStream_t st, const float* S, int64_t R, int T, float* PT_P, float* PT_X,
                const mxq_block_spec& s, uint8_t* live, int64_t cols, const mxq_softmax_tail& tl, int has_tail) {
+  if (!live && R <= kRowKernelRows) {
+    const dim3 rows((unsigned)R);
+    switch (it) {
+      case 1: k_softmax_row<ELEM, MODE, 1><<<rows, 256, 0, st>>>(S, R, T, PT_P, PT_X, s); break;
+      case 2: k_softmax_row<ELEM, MODE, 2><<<rows, 256, 0, st>>>(S, R, T, PT_P, PT_X, s); break;
+      case 4: k_softmax_row<ELEM, MODE, 4><<<rows, 256, 0, st>>>(S, R, T, PT_P, PT_X, s); break;
+      case 8: k_softmax_row<ELEM, MODE, 8><<<rows, 256, 0, st>>>(S, R, T, PT_P, PT_X, s); break;
+      case 16: k_softmax_row<ELEM, MODE, 16><<<rows, 256, 0, st>>>(S, R, T, PT_P, PT_X, s); break;
+      default: k_softmax_row<ELEM, MODE, 32><<<rows, 256, 0, st>>>(S, R, T, PT_P, PT_X, s); break;
+    }
+    return;
+  }
   switch (it) {
     case 1: k_softmax_pt<ELEM, MODE, 1><<<grid, NT, 0, st>>>(S, R, T, PT_P, PT_X, s, live, cols, tl, has_tail); break;
     case 2: k_softmax_pt<ELEM, MODE, 2><<<grid, NT, 0, st>>>(S, R, T, PT_P, PT_X, s, live, cols, tl, has_tail); break;

@@ -479,6 +479,27 @@ def test_softmax_quantize_t_against_torch(cuda, T):
     assert np.array_equal(live.cpu().numpy(), (nz | bad).transpose(1, 0, 2).astype(np.uint8))
 
 
+@pytest.mark.parametrize("T", [33, 200, 2048])
+@pytest.mark.parametrize("R", [1, 255, 257, 8192, 8193])
+def test_softmax_quantize_t_row_counts(cuda, R, T):
+    """Either side of the row kernel's range (8192 rows) and of its 256-row XCD pieces, against torch.softmax and
+    the quantizer of the transpose, bit for bit; a fully masked row and one with a NaN among them."""
+    from functools import partial
+
+    from mxq import block
+    from mxq.nn import _attention
+    g = torch.Generator(device="cuda").manual_seed(R + T)
+    S = torch.randn(R, T, device="cuda", generator=g) * 4
+    if R > 2:
+        S[R // 2], S[R - 1, T - 1] = float("-inf"), float("nan")
+    q = partial(block.mxgemmini.quantize, fmt="MXFP8_E4M3", axis=0, rounding_mode="rne")
+    got = _attention._softmax_pt(S, q, 32, None)
+    want = q(torch.softmax(S, dim=-1).contiguous().t().contiguous())
+    for name, x, y in zip(("codes", "scales"), got, want):
+        assert torch.equal(torch.isnan(x), torch.isnan(y)), f"{name}: NaN places"
+        assert torch.equal(torch.nan_to_num(x).view(torch.int32), torch.nan_to_num(y).view(torch.int32)), name
+
+
 def test_exp_underflows_past_minus_128(cuda):
     """The softmax kernel's tail rule rests on exp(x) = +0 on the device for every float32 x <= -128 (e^-103.98 is
     already below half the smallest subnormal): every float32 in [-512, -128] and a strided sample of the rest down
