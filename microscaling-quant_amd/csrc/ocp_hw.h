@@ -29,10 +29,18 @@ __host__ __device__ inline bool has_hw(int e, int m) {
 }
 
 // The formats whose conversion of N values a lane takes here: the FP6 forms convert 32 values at a time, whose
-// register vectors are not worth it for fewer than 16 (a kernel converting fewer leaves FP6 to the grid).
+// register vectors are not worth it for fewer than 16.  (four_codes and four_values take FP6 otherwise.)
 template <int N>
 __host__ __device__ inline bool has_hw_n(int e, int m) {
   return has_hw(e, m) && (N >= 16 || !((e == 2 && m == 3) || (e == 3 && m == 2)));
+}
+
+// FP6 of four values goes through the FP8 conversions: E2M3 is E4M3's grid on z * 2^-6 and E3M2 is E5M2's on z * 2^-12, the same mantissa
+// widths, the exponent offsets mapping one format's subnormal step and binades onto the other's.
+// z clamped to the format's largest value, where its grid saturates, -0 made +0, and scaled.
+__device__ __forceinline__ float fp6_as_fp8(float z, bool e2m3) {
+  const float top = e2m3 ? 7.5f : 28.0f, scale = e2m3 ? 0.015625f : 0.000244140625f;
+  return __builtin_fmaf(__builtin_amdgcn_fmed3f(z, -top, top), scale, 0.0f);
 }
 
 // The format's largest finite value, where the conversions saturate (E4M3 448, E5M2 57344, E2M3 7.5, E3M2 28,
@@ -86,9 +94,13 @@ __device__ __forceinline__ uint32_t field6(const u6v& p, int k) {
   return v & 63u;
 }
 
+template <bool SIGNED0>
+__device__ __forceinline__ float plus0(float z) { return SIGNED0 ? z : z + 0.0f; }
+
 // The element codes of N values (N % 4 == 0, N <= 32), code j in byte j % 4 of w[j / 4]; FP6 for N >= 16 only
-// (has_hw_n).
-template <int N>
+// (has_hw_n).  SIGNED0: a
+// -0 keeps its sign (the caller has made the grid's own +0, so that a -0 left is a value that underflowed).
+template <int N, bool SIGNED0 = false>
 __device__ __forceinline__ void codes(const float (&z)[N], int e, int m, uint32_t (&w)[N / 4]) {
   static_assert(N % 4 == 0 && N <= 32, "N values in whole words");
   if (e == 4 || e == 5) {
@@ -96,11 +108,11 @@ __device__ __forceinline__ void codes(const float (&z)[N], int e, int m, uint32_
     for (int q = 0; q < N / 4; ++q) {
       s2v r = {0, 0};
       if (e == 4) {
-        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, z[4 * q] + 0.0f, z[4 * q + 1] + 0.0f, 1.0f, false);
-        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, z[4 * q + 2] + 0.0f, z[4 * q + 3] + 0.0f, 1.0f, true);
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, plus0<SIGNED0>(z[4 * q]), plus0<SIGNED0>(z[4 * q + 1]), 1.0f, false);
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, plus0<SIGNED0>(z[4 * q + 2]), plus0<SIGNED0>(z[4 * q + 3]), 1.0f, true);
       } else {
-        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, z[4 * q] + 0.0f, z[4 * q + 1] + 0.0f, 1.0f, false);
-        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, z[4 * q + 2] + 0.0f, z[4 * q + 3] + 0.0f, 1.0f, true);
+        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, plus0<SIGNED0>(z[4 * q]), plus0<SIGNED0>(z[4 * q + 1]), 1.0f, false);
+        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, plus0<SIGNED0>(z[4 * q + 2]), plus0<SIGNED0>(z[4 * q + 3]), 1.0f, true);
       }
       w[q] = __builtin_bit_cast(uint32_t, r);
     }
@@ -108,8 +120,8 @@ __device__ __forceinline__ void codes(const float (&z)[N], int e, int m, uint32_
 #pragma unroll
     for (int q = 0; q < N / 4; ++q) {
       const uint32_t r =
-          __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, z[4 * q] + 0.0f, z[4 * q + 1] + 0.0f, 1.0f, 0) |
-          (__builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, z[4 * q + 2] + 0.0f, z[4 * q + 3] + 0.0f, 1.0f, 0) << 8);
+          __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, plus0<SIGNED0>(z[4 * q]), plus0<SIGNED0>(z[4 * q + 1]), 1.0f, 0) |
+          (__builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, plus0<SIGNED0>(z[4 * q + 2]), plus0<SIGNED0>(z[4 * q + 3]), 1.0f, 0) << 8);
       // nibbles n0 n1 | n2 n3 in the low two bytes -> one code a byte
       w[q] = (r & 0xFu) | ((r & 0xF0u) << 4) | ((r & 0xF00u) << 8) | ((r & 0xF000u) << 12);
     }
@@ -125,7 +137,7 @@ __device__ __forceinline__ void codes(const float (&z)[N], int e, int m, uint32_
 
 // The grid values of N values (N even, N <= 32), in place: converted and converted back; FP6 for N >= 16 only
 // (has_hw_n).
-template <int N>
+template <int N, bool SIGNED0 = false>
 __device__ __forceinline__ void values(float (&z)[N], int e, int m) {
   static_assert(N % 2 == 0 && N <= 32, "N values in pairs");
   if (e == 4 || e == 5 || m == 1) {
@@ -133,13 +145,13 @@ __device__ __forceinline__ void values(float (&z)[N], int e, int m) {
     for (int q = 0; q < N / 2; ++q) {
       f2v r;
       if (e == 4) {
-        const s2v c = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(s2v{0, 0}, z[2 * q] + 0.0f, z[2 * q + 1] + 0.0f, 1.0f, false);
+        const s2v c = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(s2v{0, 0}, plus0<SIGNED0>(z[2 * q]), plus0<SIGNED0>(z[2 * q + 1]), 1.0f, false);
         r = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(__builtin_bit_cast(uint32_t, c), 1.0f, false);
       } else if (e == 5) {
-        const s2v c = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(s2v{0, 0}, z[2 * q] + 0.0f, z[2 * q + 1] + 0.0f, 1.0f, false);
+        const s2v c = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(s2v{0, 0}, plus0<SIGNED0>(z[2 * q]), plus0<SIGNED0>(z[2 * q + 1]), 1.0f, false);
         r = __builtin_amdgcn_cvt_scalef32_pk_f32_bf8(__builtin_bit_cast(uint32_t, c), 1.0f, false);
       } else {
-        const uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, z[2 * q] + 0.0f, z[2 * q + 1] + 0.0f, 1.0f, 0);
+        const uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, plus0<SIGNED0>(z[2 * q]), plus0<SIGNED0>(z[2 * q + 1]), 1.0f, 0);
         r = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c, 1.0f, 0);
       }
       z[2 * q] = r.x;
@@ -151,6 +163,32 @@ __device__ __forceinline__ void values(float (&z)[N], int e, int m) {
     const f32v r = unpack32(pack16x2(even, odd, e == 2), e == 2);
 #pragma unroll
     for (int k = 0; k < N; ++k) z[k] = r[k];
+  }
+}
+
+// codes and values of four values of any of the formats.
+__device__ __forceinline__ void four_codes(const float (&z)[4], int e, int m, uint32_t (&w)[1]) {
+  if (e + m == 5) {
+    const bool e2m3 = e == 2;
+    float y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y[k] = fp6_as_fp8(z[k], e2m3);
+    codes<4, true>(y, e2m3 ? 4 : 5, e2m3 ? 3 : 2, w);
+    w[0] = (w[0] & 0x1F1F1F1Fu) | ((w[0] >> 2) & 0x20202020u);       // sign: bit 7 -> bit 5
+  } else {
+    codes<4>(z, e, m, w);
+  }
+}
+__device__ __forceinline__ void four_values(float (&z)[4], int e, int m) {
+  if (e + m == 5) {
+    const bool e2m3 = e == 2;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) z[k] = fp6_as_fp8(z[k], e2m3);
+    values<4, true>(z, e2m3 ? 4 : 5, e2m3 ? 3 : 2);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) z[k] = z[k] * (e2m3 ? 64.0f : 4096.0f);
+  } else {
+    values<4>(z, e, m);
   }
 }
 

@@ -3,8 +3,7 @@
 // A tensor is viewed as (outer, n, inner) with the block axis n in the middle.  Three layouts:
 //   split    (block 32): eight lanes of a wavefront share one block column of VEC adjacent columns, four rows
 //            each; their maxima meet through cross-lane exchanges; the block stays in registers.
-//   contig32 (inner == 1, block 32, n % 32 == 0): eight lanes own one contiguous 128-byte block, four
-//            elements each.
+//   row      (inner == 1, block 32): eight lanes own one contiguous block, four elements each.
 //   strided  (any other block size): one thread per block column, the block read twice.
 // Kernels are specialised on the element rule and, for the OCP grid and the microxcaling step, on the
 // rounding mode.
@@ -29,8 +28,9 @@ __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(bf16_t x) { return u2f((uint32_t)x.v << 16); }
 __device__ __forceinline__ float to_f32(f16_t x) { return (float)__builtin_bit_cast(_Float16, x.v); }
 
+// VEC adjacent elements at any element's address: gfx950's vector memory takes them there as one access.
 template <typename T, int VEC>
-struct alignas(sizeof(T) * VEC) VecT { T v[VEC]; };
+struct __attribute__((packed, aligned(sizeof(T)))) VecT { T v[VEC]; };
 
 template <typename T, int VEC>
 __device__ __forceinline__ void load_vec(const T* p, float (&out)[VEC]) {
@@ -49,11 +49,12 @@ __device__ __forceinline__ void store_vec(float* p, const float (&in)[VEC]) {
 
 // Codes are written once and not read back by this kernel: streaming (non-temporal) stores.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // at any element's address
 template <int VEC>
 __device__ __forceinline__ void store_vec_nt(float* p, const float (&in)[VEC]) {
   if constexpr (VEC == 4) {
     f32x4 r = {in[0], in[1], in[2], in[3]};
-    __builtin_nontemporal_store(r, reinterpret_cast<f32x4*>(p));
+    __builtin_nontemporal_store(r, reinterpret_cast<f32x4_any*>(p));
   } else {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) __builtin_nontemporal_store(in[j], p + j);
@@ -64,7 +65,7 @@ __device__ __forceinline__ void store_vec_nt(float* p, const float (&in)[VEC]) {
 //   FloatSink  float32 P and X, the reference's outputs (codes written with streaming stores).
 //   ByteSink   one element-code byte per element and one E8M0 byte per scale (mx_encode, e8m0_encode); a value
 //              neither format holds sets *err (a zero block's scale is free, its value being 0 under any).
-// `at` is an element index of P (or X); VEC consecutive elements, VEC-aligned.
+// `at` is an element index of P (or X); VEC consecutive elements, at any of them.
 struct FloatSink {
   float* P;
   float* X;
@@ -101,35 +102,34 @@ struct FloatSink {
       }
     }
   }
+  // The first `live` of four scaled values, converted as hw_rows does.
+  __device__ __forceinline__ void hw_four(int64_t at, const float (&v)[4], int live, const mxq_block_spec& s) const {
+    float z[4] = {v[0], v[1], v[2], v[3]};
+    mxq_ocp_hw::four_values(z, s.e, s.m);
+    if (live == 4) {
+      store_vec_nt<4>(P + at, z);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (j < live) P[at + j] = z[j];
+    }
+  }
   __device__ __forceinline__ bool hw_format(const mxq_block_spec&) const { return true; }
-  __device__ __forceinline__ uintptr_t p_addr() const { return reinterpret_cast<uintptr_t>(P); }
-  __device__ __forceinline__ uintptr_t x_addr() const { return reinterpret_cast<uintptr_t>(X); }
 };
 
 template <int VEC>
 __device__ __forceinline__ void store_bytes(uint8_t* p, uint32_t w) {
-  if constexpr (VEC == 4) *reinterpret_cast<uint32_t*>(p) = w;
-  else if constexpr (VEC == 2) *reinterpret_cast<uint16_t*>(p) = (uint16_t)w;
-  else *p = (uint8_t)w;
+  __builtin_memcpy(p, &w, VEC);
 }
 
-// W words of code bytes (1, 2 or 4: 4, 8 or 16 bytes, aligned), one store.
+// W words of code bytes (1, 2 or 4: 4, 8 or 16 bytes, at any address), one store.
 // The byte sink's stores: plain, not streaming.  A wave writes 64 bytes of a code row and the next wave the rest of
 // its 128-byte line; streaming stores of those halves wrote 1.28x the code and scale bytes (bf16 8192 x 8192: 88.4 MB for 69.2),
 // plain ones exactly them, in the same time.  (The float sink's rows are whole lines; its streaming stores keep
 // 268 MB of codes out of L2 and run faster than plain ones.)
 template <int W>
 __device__ __forceinline__ void store_words(uint8_t* p, const uint32_t (&w)[W]) {
-  if constexpr (W == 1) {
-    *reinterpret_cast<uint32_t*>(p) = w[0];
-  } else if constexpr (W == 4) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<u32x4*>(p) = u32x4{w[0], w[1], w[2], w[3]};
-  } else {
-    static_assert(W == 2, "4, 8 or 16 bytes");
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
-  }
+  __builtin_memcpy(p, w, 4 * W);
 }
 
 // The element format's constants for the byte sink's short encoder.
@@ -263,6 +263,17 @@ struct ByteSink {
       store_words<VEC / 4>(P + at + (int64_t)i * stride, row);
     }
   }
+  __device__ __forceinline__ void hw_four(int64_t at, const float (&v)[4], int live, const mxq_block_spec& s) const {
+    uint32_t w[1];
+    mxq_ocp_hw::four_codes(v, s.e, s.m, w);
+    if (live == 4) {
+      store_words<1>(P + at, w);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (j < live) P[at + j] = (uint8_t)(w[0] >> (8 * j));
+    }
+  }
   // the codes the conversions give are the byte format's when it is the grid's
   __device__ __forceinline__ bool hw_format(const mxq_block_spec& s) const { return e == s.e && m == s.m; }
   template <int VEC>
@@ -275,8 +286,6 @@ struct ByteSink {
     else store_bytes<VEC>(X + at, w[0]);
     if (!ok) atomicOr(err, 2);
   }
-  __device__ __forceinline__ uintptr_t p_addr() const { return reinterpret_cast<uintptr_t>(P); }
-  __device__ __forceinline__ uintptr_t x_addr() const { return reinterpret_cast<uintptr_t>(X); }
 };
 
 // (o, b, column group) of a flat thread index over outer * nb * groups.
@@ -306,20 +315,66 @@ __device__ __forceinline__ bool wave_needs_div(const Div (&d)[VEC]) {
   return __any(need);
 }
 
+// Whether a wave's scaled values may take the hardware conversions (ocp_hw.h), and `hs`, the spec that names them
+// their element format.  Every scaled value has to be finite and within their range (a column's largest |z| is its
+// maximum scaled, the division being monotone) and the grid has to saturate where they do (max_norm the format's
+// own).  microxcaling's "even" (mxq/microxcaling/elemwise.py:29-60) is the OCP grid at nearest even, saturating at
+// max_norm, with one exception: the float32 just below half the smallest subnormal step, which its float32
+// floor(|A| + 0.5) rounds up to that step.  So with every value and scaled value finite and none of that magnitude,
+// the values, clamped here to +-max_norm, go to the conversions.
+// N: the values a lane converts at once.  am, d: the block columns' maxima (as bit patterns) and divisors; v: the lane's scaled values.
+template <int ELEM, int N, typename SINK, int COLS, int ROWS, int VEC>
+__device__ __forceinline__ bool hw_gate(const SINK& out, const mxq_block_spec& s, mxq_block_spec& hs,
+                                        const uint32_t (&am)[COLS], const Div (&d)[COLS], bool div,
+                                        float (&v)[ROWS][VEC]) {
+  constexpr bool MS = ELEM == MXQ_ELEM_MICROSOFT;
+  if constexpr (MS) hs.m = s.m - 2;                  // microxcaling's mbits count the sign and hidden bits
+  if (!(s.via_e == 0 && mxq_ocp_hw::has_hw_n<N>(hs.e, hs.m) && out.hw_format(hs) &&
+        s.max_norm == mxq_ocp_hw::fmt_max(hs.e, hs.m)))
+    return false;
+  const float lim = MS ? INFINITY : mxq_ocp_hw::hw_limit(hs.e, hs.m);
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < COLS; ++j) {                   // finite inputs and scaled values (a NaN scale fails)
+    const float a = u2f(am[j]);
+    const float zm = !s.scale_rule ? a : (div ? apply_div(a, d[j]) : a * d[j].inv);
+    ok = ok && am[j] < 0x7F800000u && zm < lim;
+  }
+  if constexpr (MS) {
+    const int emin = 2 - (1 << (hs.e - 1));
+    const uint32_t odd = (uint32_t)(127 + emin - hs.m - 1) << 23;  // 2^(emin - m - 1), then one float below
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) ok = ok && (f2u(v[i][j]) & 0x7FFFFFFFu) != odd - 1u;
+  }
+  const bool hw = __all(ok);
+  if constexpr (MS) {
+    if (hw) {
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[i][j] = fminf(fmaxf(v[i][j], -s.max_norm), s.max_norm);
+    }
+  }
+  return hw;
+}
+
 // Any block size (read twice: once for the amax, once for the elements), one thread per block column of
 // VEC adjacent columns.
 template <typename T, int ELEM, int MODE, int VEC, typename SINK>
 __global__ void __launch_bounds__(256) k_quant_strided(const T* __restrict__ V, const SINK out, int64_t outer,
                                                        int64_t n, int64_t inner, int64_t bs, int64_t nb,
                                                        mxq_block_spec s) {
-  const int64_t groups = inner / VEC;
+  const int64_t groups = (inner + VEC - 1) / VEC;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= outer * nb * groups) return;
   int64_t o, b, g;
   split_index(t, groups, nb, o, b, g);
   const int64_t k0 = b * bs;
   const int64_t rows = (n - k0 < bs) ? n - k0 : bs;
-  const int64_t off = (o * n + k0) * inner + g * VEC;
+  const int64_t col = g * VEC < inner - VEC ? g * VEC : inner - VEC;   // the last group ends on the last column
+  const int64_t off = (o * n + k0) * inner + col;
   float amax[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) amax[j] = 0.0f;
@@ -346,7 +401,7 @@ __global__ void __launch_bounds__(256) k_quant_strided(const T* __restrict__ V, 
   bool zero[VEC];
 #pragma unroll
   for (int j = 0; j < VEC; ++j) zero[j] = amax[j] == 0.0f;
-  out.template scales<VEC>((o * nb + b) * inner + g * VEC, xs, zero);
+  out.template scales<VEC>((o * nb + b) * inner + col, xs, zero);
 }
 
 // Block size 32 with R lanes of one wavefront sharing a block column: lane l of a wave takes row part
@@ -356,7 +411,9 @@ __global__ void __launch_bounds__(256) k_quant_strided(const T* __restrict__ V, 
 // bf16 and on 4096 x 512 float32).
 //   * The wave's index is uniform, so the (outer, block, column-group) split of it runs in scalar registers.
 //   * A whole block (all but a tail) loads without per-row conditions; lanes past the last column group read
-//     column group 0 (valid memory) and store nothing.
+//     the last one's columns and store nothing.
+//   * Rows of any length and address: a group of VEC columns is one access wherever it begins (rows that
+//     were not whole fours had a column a lane: a call on 5632 x 333 float32 20.9 -> 10.7 us, 4096 x 2049 27.9 -> 19.9).
 //   * The block maximum is the largest |v| bit pattern (non-negative floats order like their patterns, and
 //     every NaN pattern lies above +Inf, so a NaN wins as torch.amax's does).
 //   * The R lanes of a column group hold the same maxima after the exchanges; lane r computes the scales of
@@ -369,7 +426,7 @@ __global__ void __launch_bounds__(256) k_quant_split(const T* __restrict__ V, co
   constexpr int CPW = 64 / R;          // column groups per wave
   constexpr int ROWS = 32 / R;         // rows per lane
   constexpr int PER = (VEC + R - 1) / R;  // scales each lane evaluates
-  const int64_t groups = inner / VEC;
+  const int64_t groups = (inner + VEC - 1) / VEC;
   const int lane = threadIdx.x & 63;
   const int64_t nb = nb_div.d, waves_per_row = wpr_div.d;
   // the launch keeps the wave count below 2^31
@@ -383,7 +440,9 @@ __global__ void __launch_bounds__(256) k_quant_split(const T* __restrict__ V, co
   const int c = lane % CPW, r = lane / CPW;
   const int64_t cg = (int64_t)(wave - wr * wpr_div.d) * CPW + c;
   const bool live = cg < groups;
-  const T* src = V + (o * n + k0 + r * ROWS) * inner + (live ? cg : 0) * VEC;
+  // the last group ends on the last column, sharing some with the group before it (the same values stored twice)
+  const int64_t col = cg * VEC < inner - VEC ? cg * VEC : inner - VEC;
+  const T* src = V + (o * n + k0 + r * ROWS) * inner + col;
 
   float v[ROWS][VEC];
   uint32_t am[VEC];
@@ -441,60 +500,13 @@ __global__ void __launch_bounds__(256) k_quant_split(const T* __restrict__ V, co
 #pragma unroll
       for (int j = 0; j < VEC; ++j) v[i][j] = v[i][j] * d[j].inv;
   }
-  // the OCP grid at nearest even by the hardware conversions when every scaled value of the wave is finite
-  // and within their range (a column's largest |z| is its maximum scaled, the division being monotone) and the
-  // grid saturates where they do (max_norm the format's own)
-  constexpr bool HW_OCP = ELEM == MXQ_ELEM_OCP && MODE == MXQ_RNE && VEC >= 4;
-  constexpr bool HW_MS = ELEM == MXQ_ELEM_MICROSOFT && MODE == MXQ_RNE && VEC >= 4;
+  constexpr bool HW = VEC >= 4 && MODE == MXQ_RNE && (ELEM == MXQ_ELEM_OCP || ELEM == MXQ_ELEM_MICROSOFT);
+  mxq_block_spec hs = s;
   bool hw = false;
-  if constexpr (HW_OCP) {
-    if (s.via_e == 0 && mxq_ocp_hw::has_hw_n<ROWS * VEC>(s.e, s.m) && out.hw_format(s) &&
-        s.max_norm == mxq_ocp_hw::fmt_max(s.e, s.m)) {
-      const float lim = mxq_ocp_hw::hw_limit(s.e, s.m);
-      bool ok = true;
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        const float a = u2f(am[j]);
-        const float zm = !s.scale_rule ? a : (div ? apply_div(a, d[j]) : a * d[j].inv);
-        ok = ok && am[j] < 0x7F800000u && zm < lim;
-      }
-      hw = __all(ok);
-    }
-  }
-  // microxcaling's "even" (mxq/microxcaling/elemwise.py:29-60) is the OCP grid at nearest even, saturating at
-  // max_norm, with one exception: the float32 just below half the smallest subnormal step, which its float32
-  // floor(|A| + 0.5) rounds up to that step.  So with every value and scaled value finite and none of that
-  // magnitude, the values clamped to +-max_norm go to the hardware conversions.
-  mxq_block_spec hs = s;                             // the element format as the conversions name it
-  if constexpr (HW_MS) {
-    hs.m = s.m - 2;                                   // microxcaling's mbits count the sign and hidden bits
-    if (s.via_e == 0 && mxq_ocp_hw::has_hw_n<ROWS * VEC>(hs.e, hs.m) && out.hw_format(hs) &&
-        s.max_norm == mxq_ocp_hw::fmt_max(hs.e, hs.m)) {
-      const int emin = 2 - (1 << (hs.e - 1));
-      const uint32_t odd = (uint32_t)(127 + emin - hs.m - 1) << 23;  // 2^(emin - m - 1), then one float below
-      bool ok = true;
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {               // finite inputs and finite scaled values (a NaN scale fails)
-        const float a = u2f(am[j]);
-        const float zm = !s.scale_rule ? a : (div ? apply_div(a, d[j]) : a * d[j].inv);
-        ok = ok && am[j] < 0x7F800000u && zm < INFINITY;
-      }
-#pragma unroll
-      for (int i = 0; i < ROWS; ++i)
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) ok = ok && (f2u(v[i][j]) & 0x7FFFFFFFu) != odd - 1u;
-      hw = __all(ok);
-      if (hw) {
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i)
-#pragma unroll
-          for (int j = 0; j < VEC; ++j) v[i][j] = fminf(fmaxf(v[i][j], -s.max_norm), s.max_norm);
-      }
-    }
-  }
+  if constexpr (HW) hw = hw_gate<ELEM, ROWS * VEC>(out, s, hs, am, d, div, v);
   if (!live) return;
-  const int64_t dst = (o * n + k0 + r * ROWS) * inner + cg * VEC;
-  if constexpr (HW_OCP || HW_MS) {
+  const int64_t dst = (o * n + k0 + r * ROWS) * inner + col;
+  if constexpr (HW) {
     if (hw) out.template hw_rows<ROWS, VEC>(dst, inner, v, rows == 32 ? ROWS : rows - r * ROWS, hs);
   }
   if (!hw) {
@@ -521,39 +533,143 @@ __global__ void __launch_bounds__(256) k_quant_split(const T* __restrict__ V, co
     bool zero[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) zero[j] = am[j] == 0u;
-    out.template scales<VEC>((o * nb + b) * inner + cg * VEC, xs, zero);
+    out.template scales<VEC>((o * nb + b) * inner + col, xs, zero);
   }
 }
 
-// inner == 1, blocks of 32 contiguous elements, n % 32 == 0: eight lanes per block, four elements per lane.
-template <typename T, int ELEM, int MODE, typename SINK>
-__global__ void __launch_bounds__(256) k_quant_contig32(const T* __restrict__ V, const SINK out, int64_t nblocks,
-                                                        mxq_block_spec s) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t blk = t >> 3;
-  const bool live = blk < nblocks;
-  const int64_t off = t * 4;
-  float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (live) load_vec<T, 4>(V + off, v);
-  float a = 0.0f;
+// inner == 1, blocks of 32 contiguous elements of rows of any length n: eight lanes per block, four elements a
+// lane (those past the row's end are 0 and are not stored), one access wherever they begin.  A wave takes Q runs
+// of eight blocks, and lane l of a block's eight evaluates the scale of its l % Q-th run for the others: the scale
+// rule, some hundred instructions, is what Q = 1 spends most of its time on.
+// Half-precision rows of 2001 values to E2M3, 2331 of them: 71 -> 12.6 us, 16,384: 451 -> 35 us (their blocks went
+// one a wave through k_quant_split, an element a lane); of 2048, 16,384: 44 -> 33 us, through microxcaling's grid
+// 72 -> 33 us (no conversions were used for contiguous blocks).  What is left is memory: 33 us is 6.1 TB/s.
+template <typename T, int ELEM, int MODE, int Q, bool WHOLE, typename SINK>
+__global__ void __launch_bounds__(256) k_quant_row(const T* __restrict__ V, const SINK out, int64_t nblocks,
+                                                   int64_t outer, int64_t n, mxq::DivU31 nb_div, mxq_block_spec s) {
+  static_assert(Q >= 1 && Q <= 8, "a lane evaluates one scale");
+  const int lane = threadIdx.x & 63, l8 = lane & 7;
+  const int64_t total = outer * n;
+  const int64_t first = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (8 * Q) + (lane >> 3);
+  // this lane's four elements of run q: their place, and how many of them there are
+  auto place = [&](int q, int64_t& blk, int64_t& off) {
+    blk = first + 8 * q;
+    if constexpr (WHOLE) {                              // rows are whole blocks: no row to find, no part of one
+      off = blk * 32 + l8 * 4;
+      return blk < nblocks ? 4 : 0;
+    }
+    const int64_t o = mxq::divu31((uint32_t)blk, nb_div);
+    const int64_t k = (blk - o * nb_div.d) * 32 + l8 * 4;
+    off = o * n + k;
+    return blk < nblocks ? (int)(n - k < 4 ? n - k : 4) : 0;
+  };
+  // every run's load is issued before any is waited for: four elements from each lane's place whatever the row
+  // holds there, moved back where that would leave the tensor (of at least four elements)
+  VecT<T, 4> w[Q];
+  int64_t blk[Q], off[Q];
+  int left[Q];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) a = amax_combine(a, fabsf(v[j]));
-  // all 64 lanes take part in the exchanges; lanes past the end hold 0 and belong to no live block
-  a = amax_combine(a, __shfl_xor(a, 1, 8));
-  a = amax_combine(a, __shfl_xor(a, 2, 8));
-  a = amax_combine(a, __shfl_xor(a, 4, 8));
-  if (!live) return;
-  const float xs = block_scale(a, s);
-  const Div d = make_div(xs);
-  float z[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) z[j] = s.scale_rule ? apply_div(v[j], d) : v[j];
-  out.template elems<ELEM, MODE, 4>(off, z, s);
-  if ((t & 7) == 0) {
-    const float x1[1] = {xs};
-    const bool z1[1] = {a == 0.0f};
-    out.template scales<1>(blk, x1, z1);
+  for (int q = 0; q < Q; ++q) {
+    left[q] = place(q, blk[q], off[q]);
+    w[q] = *reinterpret_cast<const VecT<T, 4>*>(V + (off[q] < total - 4 ? off[q] : total - 4));
   }
+  float v[Q][4];
+  uint32_t am[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (!WHOLE && off[q] > total - 4) {              // the tensor's last elements
+      const int64_t back = off[q] - (total - 4);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) w[q].v[j] = back == 1 ? w[q].v[j + 1] : back == 2 ? w[q].v[j < 2 ? j + 2 : 3] : w[q].v[3];
+    }
+    am[q] = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[q][j] = WHOLE || j < left[q] ? to_f32(w[q].v[j]) : 0.0f;
+      am[q] = max(am[q], f2u(v[q][j]) & 0x7FFFFFFFu);
+    }
+  }
+  // all 64 lanes take part in the exchanges; lanes past the end belong to no live block
+#pragma unroll
+  for (int step = 1; step < 8; step <<= 1)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) am[q] = max(am[q], (uint32_t)__shfl_xor((int)am[q], step, 8));
+  uint32_t mine = am[0];
+#pragma unroll
+  for (int q = 1; q < Q; ++q) mine = l8 % Q == q ? am[q] : mine;
+  const float own = block_scale(u2f(mine), s);
+  Div d[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) d[q] = make_div(Q == 1 ? own : __shfl(own, q, 8));
+  const bool div = s.scale_rule && wave_needs_div<Q>(d);
+  constexpr bool HW = MODE == MXQ_RNE && (ELEM == MXQ_ELEM_OCP || ELEM == MXQ_ELEM_MICROSOFT);
+  mxq_block_spec hs = s;
+  bool hw = false;
+  if constexpr (HW) {
+    if (div) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[q][j] = apply_div(v[q][j], d[q]);
+    } else if (s.scale_rule) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[q][j] = v[q][j] * d[q].inv;
+    }
+    hw = hw_gate<ELEM, 32>(out, s, hs, am, d, div, v);   // four_values takes every format
+    if (hw) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        if (left[q] > 0) out.hw_four(off[q], v[q], left[q], hs);
+    }
+  }
+  if constexpr (!HW) {                                 // software grids: from the registers
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[q][j] = !s.scale_rule ? v[q][j] : (div ? apply_div(v[q][j], d[q]) : v[q][j] * d[q].inv);
+      if (left[q] == 4) {
+        out.template elems<ELEM, MODE, 4>(off[q], v[q], s);
+      } else {
+#pragma unroll 1
+        for (int j = 0; j < left[q]; ++j) {
+          const float z[1] = {j == 0 ? v[q][0] : j == 1 ? v[q][1] : v[q][2]};
+          out.template elems<ELEM, MODE, 1>(off[q] + j, z, s);
+        }
+      }
+    }
+  } else if (!hw) {
+    // the element grid in software, a run at a time from a second read of its elements, so that its registers are
+    // one run's
+#pragma unroll 1
+    for (int q = 0; q < Q; ++q) {
+      int64_t b, at;
+      const int count = place(q, b, at);
+      const Div dq = make_div(__shfl(own, q, 8));
+      auto scaled = [&](float x) { return !s.scale_rule ? x : (div ? apply_div(x, dq) : x * dq.inv); };
+      if (count == 4) {
+        float z[4];
+        load_vec<T, 4>(V + at, z);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) z[j] = scaled(z[j]);
+        out.template elems<ELEM, MODE, 4>(at, z, s);
+      } else {
+#pragma unroll 1
+        for (int j = 0; j < count; ++j) {
+          const float z[1] = {scaled(to_f32(V[at + j]))};
+          out.template elems<ELEM, MODE, 1>(at + j, z, s);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (l8 == q && blk[q] < nblocks) {
+      const float x1[1] = {own};
+      const bool z1[1] = {mine == 0u};
+      out.template scales<1>(blk[q], x1, z1);
+    }
 }
 
 // ------------------------------------------------------ code bytes of the OCP grid at nearest even, one pass
@@ -584,8 +700,8 @@ struct In<float> {
   static constexpr int NW = 8, NA = 8;                // words per row, words of column maxima
   static constexpr uint32_t kFin = 0x7F800000u;       // |x| patterns below this are finite
   __device__ static void load(const float* p, uint32_t (&w)[NW]) {
-    const uint4 a = *reinterpret_cast<const uint4*>(p), b = *reinterpret_cast<const uint4*>(p + 4);
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w; w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
+    __builtin_memcpy(w, p, 16);
+    __builtin_memcpy(w + 4, p + 4, 16);
   }
   __device__ static void amax(uint32_t (&am)[NA], const uint32_t (&w)[NW]) {
 #pragma unroll
@@ -604,8 +720,7 @@ struct In16 {
   static constexpr int NW = 4, NA = 4;
   template <typename T>
   __device__ static void load(const T* p, uint32_t (&w)[NW]) {
-    const uint4 a = *reinterpret_cast<const uint4*>(p);
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w;
+    __builtin_memcpy(w, p, 16);
   }
   __device__ static void amax(uint32_t (&am)[NA], const uint32_t (&w)[NW]) {
 #pragma unroll
@@ -669,7 +784,7 @@ __global__ void __launch_bounds__(256) k_pack_rne(const T* __restrict__ V, const
   using Cd = pkr::Code<E, M>;
   constexpr int VEC = 8, CPW = 64 / R, ROWS = 32 / R, PER = VEC / R;
   static_assert(R == 4 || R == 8, "4 or 8 lanes per block column");
-  const int64_t groups = inner / VEC;
+  const int64_t groups = (inner + VEC - 1) / VEC;
   const int lane = threadIdx.x & 63;
   const int64_t nb = nb_div.d;
   const uint32_t wave = blockIdx.x * (256 / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -682,7 +797,9 @@ __global__ void __launch_bounds__(256) k_pack_rne(const T* __restrict__ V, const
   const int c = lane % CPW, r = lane / CPW;
   const int64_t cg = (int64_t)(wave - wr * wpr_div.d) * CPW + c;
   const bool live = cg < groups;
-  const T* src = V + (o * n + k0 + r * ROWS) * inner + (live ? cg : 0) * VEC;
+  // the last group ends on the last column, sharing some with the group before it (the same values stored twice)
+  const int64_t col = cg * VEC < inner - VEC ? cg * VEC : inner - VEC;
+  const T* src = V + (o * n + k0 + r * ROWS) * inner + col;
 
   uint32_t w[ROWS][In::NW];
   uint32_t am[In::NA];
@@ -726,8 +843,8 @@ __global__ void __launch_bounds__(256) k_pack_rne(const T* __restrict__ V, const
     eb[j] = (uint32_t)__shfl((int)own_b[j / R], c + (j % R) * CPW, 64);
     fast = fast && eb[j] != 0u;
   }
-  const int64_t dst = (o * n + k0 + r * ROWS) * inner + cg * VEC;
-  const int64_t xat = (o * nb + b) * inner + cg * VEC;
+  const int64_t dst = (o * n + k0 + r * ROWS) * inner + col;
+  const int64_t xat = (o * nb + b) * inner + col;
   if (__all(fast)) {
     if (!live) return;
     float inv[VEC];
@@ -899,13 +1016,12 @@ inline int validate(const mxq_block_spec& s) {
   return MXQ_OK;
 }
 
-// k_pack_rne for blocks of 32 along the axis, inner % 8 == 0, V 16-byte aligned, codes and scales 8-byte
-// aligned: four lanes per block column (eight rows each) while that gives the chip at least 2048 waves,
+// k_pack_rne for blocks of 32 along the axis, inner >= 8: four lanes per block column (eight rows each) while that gives the chip at least 2048 waves,
 // else eight (four rows each).
 template <typename T>
 int launch_pack_rne(const T* V, const ByteSink& out, int64_t outer, int64_t n, int64_t inner, int64_t nb,
                     const mxq_block_spec& q, hipStream_t st) {
-  const int64_t groups = inner / 8;
+  const int64_t groups = mxq::ceil_div(inner, 8);
   if (outer * nb * mxq::ceil_div(groups, 8) >= (int64_t(1) << 31))
     return mxq::invalid("block quantize: tensor too large (2^31 waves of 2048 elements)");
   auto go = [&](auto r_const) {
@@ -936,36 +1052,49 @@ int launch_quant(const T* V, const SINK& out, int64_t outer, int64_t n, int64_t 
   }
   mxq::KernelTimer timer("block_quantize", st);
   const int64_t nb = mxq::ceil_div(n, bs);
-  const uintptr_t av = reinterpret_cast<uintptr_t>(V), ap = reinterpret_cast<uintptr_t>(out.P),
-                  ax = reinterpret_cast<uintptr_t>(out.X);
-  constexpr int OB = SINK::kBytes;
-  if (inner == 1 && bs == 32 && n % 32 == 0 && av % (4 * sizeof(T)) == 0 && ap % (4 * OB) == 0) {
+  // contiguous blocks: rows of whole blocks in any number (no row to find); others count their blocks in 31 bits
+  if (inner == 1 && bs == 32 && outer * n >= 4 &&
+      (n % 32 == 0 || (outer * nb < (int64_t(1) << 31) && n < (int64_t(1) << 31)))) {
     const int64_t nblocks = outer * nb;
-    k_quant_contig32<T, ELEM, MODE, SINK><<<mxq::grid_for(nblocks * 8, 256), 256, 0, st>>>(V, out, nblocks, q);
+    auto go = [&](auto q_const) {
+      constexpr int Q = decltype(q_const)::value;
+      const dim3 grid = mxq::grid_for(mxq::ceil_div(nblocks, Q) * 8, 256);
+      if (n % 32 == 0) k_quant_row<T, ELEM, MODE, Q, true><<<grid, 256, 0, st>>>(V, out, nblocks, outer, n, {}, q);
+      else k_quant_row<T, ELEM, MODE, Q, false><<<grid, 256, 0, st>>>(V, out, nblocks, outer, n,
+                                                                       mxq::make_divu31((uint32_t)nb), q);
+    };
+    // Q = 4 for the grids the conversions take, while it leaves the chip two waves a SIMD (16,384 rows of 2001
+    // half-precision values: 35 us); a software grid is VALU work enough to hide the rest (16,384 x 2048
+    // float32 through mxquant's: 53 us at Q = 4, 48 at Q = 1)
+    if constexpr (MODE == MXQ_RNE && (ELEM == MXQ_ELEM_OCP || ELEM == MXQ_ELEM_MICROSOFT)) {
+      if (nblocks >= 2048 * 8 * 4) {
+        go(std::integral_constant<int, 4>{});
+        return mxq::check_launch("mxq_block_quantize");
+      }
+    }
+    go(std::integral_constant<int, 1>{});
     return mxq::check_launch("mxq_block_quantize");
   }
-  auto aligned = [&](int vec) {
-    return inner % vec == 0 && av % (vec * sizeof(T)) == 0 && ap % (vec * OB) == 0 && ax % (vec * OB) == 0;
-  };
-  const int vec = aligned(4) ? 4 : (aligned(2) ? 2 : 1);
+  const int vec = inner >= 4 ? 4 : (inner % 2 == 0 ? 2 : 1);
   if constexpr (SINK::kBytes == 1 && ELEM == MXQ_ELEM_OCP && MODE == MXQ_RNE) {
     if (bs == 32 && q.via_e == 0 && out.e == q.e && out.m == q.m && mxq_ocp_hw::has_hw(q.e, q.m) &&
-        q.max_norm == mxq_ocp_hw::fmt_max(q.e, q.m) && aligned(8) && av % 16 == 0)
+        q.max_norm == mxq_ocp_hw::fmt_max(q.e, q.m) && inner >= 8)
       return launch_pack_rne(V, out, outer, n, inner, nb, q, st);
   }
   if (bs == 32) {
-    // code bytes: eight columns a lane when they align (8-byte stores: a wave's eight lanes write 64 contiguous
+    // code bytes: eight columns a lane when there are as many (8-byte stores: a wave's eight lanes write 64 contiguous
     // bytes of a row, the next wave the other half of the line; sixteen would keep 64 values a lane, which
     // this layout's registers do not hold)
-    const int bvec = SINK::kBytes == 1 && aligned(8) ? 8 : 0;
+    const int bvec = SINK::kBytes == 1 && inner >= 8 ? 8 : 0;
     const int kvec = bvec ? bvec : vec;
     // R = 8 lanes per block column (4 rows each) while that gives the chip at least 8 waves per SIMD; smaller
     // tensors take R = 32 (one row per lane, four times the waves), which keeps more loads in flight (MI355X,
     // block.ocp on 4096 x 512 float32: 12.2 us at R = 8, 9.7 us at R = 32; bf16 8192 x 8192: R = 8 fastest)
-    const int64_t waves8 = outer * nb * mxq::ceil_div(inner / kvec, 64 / 8);
+    const int64_t groups = mxq::ceil_div(inner, kvec);
+    const int64_t waves8 = outer * nb * mxq::ceil_div(groups, 64 / 8);
     auto go = [&](auto r_const) {
       constexpr int R = decltype(r_const)::value;
-      const int64_t wpr = mxq::ceil_div(inner / kvec, 64 / R);
+      const int64_t wpr = mxq::ceil_div(groups, 64 / R);
       const dim3 grid = mxq::grid_for(outer * nb * wpr * 64, 256);
       const mxq::DivU31 dnb = mxq::make_divu31((uint32_t)nb), dwpr = mxq::make_divu31((uint32_t)wpr);
       if constexpr (SINK::kBytes == 1) {
@@ -979,13 +1108,13 @@ int launch_quant(const T* V, const SINK& out, int64_t outer, int64_t n, int64_t 
       else k_quant_split<T, ELEM, MODE, 1, R, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, dnb, dwpr, q);
     };
     // the kernel indexes waves in 32 bits
-    if (outer * nb * mxq::ceil_div(inner / kvec, 64 / 32) >= (int64_t(1) << 31))
+    if (outer * nb * mxq::ceil_div(groups, 64 / 32) >= (int64_t(1) << 31))
       return mxq::invalid("block quantize: tensor too large (2^31 waves of 2048 elements)");
     if (waves8 >= 8 * 1024) go(std::integral_constant<int, 8>{});
     else go(std::integral_constant<int, 32>{});
     return mxq::check_launch("mxq_block_quantize");
   }
-  const int64_t threads = outer * nb * (inner / vec);
+  const int64_t threads = outer * nb * mxq::ceil_div(inner, vec);
   const dim3 grid = mxq::grid_for(threads, 256);
   if (vec == 4) k_quant_strided<T, ELEM, MODE, 4, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, bs, nb, q);
   else if (vec == 2) k_quant_strided<T, ELEM, MODE, 2, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, bs, nb, q);

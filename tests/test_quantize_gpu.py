@@ -177,6 +177,42 @@ def test_dequantize(cuda):
         assert_bits_equal(got3, ob.dequantize(P3.cpu().numpy(), X3.cpu().numpy(), axis, bs), f"dequantize {shape}")
 
 
+def _at_odd_address(V):
+    """V's values in a contiguous tensor that begins one element past an allocation's start."""
+    out = torch.empty(V.numel() + 1, dtype=V.dtype, device="cuda")[1:].view(V.shape)
+    return out.copy_(V)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("method", ["mxgemmini", "ocp", "mxquant"])
+def test_ragged_rows_at_any_address(cuda, method, dtype, fmt):
+    """Rows of every length around a lane's four columns and a block's 32 elements, at an odd address, blocks along
+    the contiguous axis and along the outer one (block sizes 32, 16 and 6), quantized and read back, against the
+    oracle: edges, subnormals, Inf and NaN in some of them, plain values (the conversions' path) in the others."""
+    from mxq import block
+    rng = np.random.default_rng(13)
+    kw = {"rounding_mode": "rne"} if method == "mxgemmini" else {}
+    for shape, axis, bs in [((7, n), 1, 32) for n in (1, 2, 3, 4, 5, 31, 32, 33, 63, 96, 131)] + \
+            [((70, n), 0, 32) for n in (2, 3, 4, 5, 7, 9, 33, 257)] + \
+            [((3, 41, 5), 1, 16), ((3, 41, 13), 1, 6), ((9, 29), 1, 6), ((2, 40, 517), 1, 32), ((70, 100), 1, 3)]:
+        for plain in (True, False):
+            V = (rng.standard_normal(shape) * 3).astype(np.float32) if plain else \
+                _edge_matrix(rng, shape[0], int(np.prod(shape[1:]))).reshape(shape)
+            Vt = _at_odd_address(torch.from_numpy(V).to(dtype))
+            V = Vt.float().cpu().numpy()
+            q = getattr(block, method)
+            P, X = q.quantize(Vt, fmt, axis=axis, block_size=bs, **kw)
+            want = {"mxgemmini": lambda: ob.mxgemmini_quantize(V, fmt, axis, bs, "rne"),
+                    "ocp": lambda: ob.ocp_quantize(V, fmt, axis, bs),
+                    "mxquant": lambda: ob.mxquant_quantize(V, fmt, axis, bs)}[method]()
+            at = f"{method} {fmt} {dtype} {shape} axis {axis} blocks of {bs}"
+            assert_bits_equal(P.cpu().numpy(), want[0], "P " + at)
+            assert_bits_equal(X.cpu().numpy(), want[1], "X " + at)
+            back = block.dequantize(_at_odd_address(P), _at_odd_address(X), axis=axis, block_size=bs)
+            assert_bits_equal(back.cpu().numpy(), ob.dequantize(*want, axis, bs), "read back " + at)
+
+
 # ------------------------------------------------------------------------------------------ elementwise
 @pytest.fixture(scope="module")
 def corpus():
