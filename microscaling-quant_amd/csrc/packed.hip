@@ -5,7 +5,9 @@
 //   k_pack             float32 P and X -> bytes; one thread per block column (it needs the whole block to
 //                      know whether a scale E8M0 lacks belongs to an all-zero block)
 //   k_unpack_codes     bytes -> float32 P, and k_unpack_scales -> float32 X
-//   k_dequant_packed   bytes -> the dequantized float32 values P * X, without materialising either
+// The dequantized float32 values P * X (the float32 multiply mxq/block/_driver.py:66-72 makes of the float32 codes
+// and scales) come straight from the bytes, without materialising either (dequant_impl.h).
+#include "dequant_impl.h"
 #include "mxq_common.h"
 #include "mxq_numerics.h"
 
@@ -65,22 +67,6 @@ __global__ void __launch_bounds__(256) k_unpack_scales(const uint8_t* __restrict
     X[i] = e8m0_decode(scales[i]);
 }
 
-// One thread per block column: decode, scale, store (the float32 multiply mxq/block/_driver.py:66-72 makes of
-// the float32 codes and scales).
-__global__ void __launch_bounds__(256) k_dequant_packed(const uint8_t* __restrict__ codes,
-                                                        const uint8_t* __restrict__ scales, float* __restrict__ out,
-                                                        int64_t outer, int64_t n, int64_t inner, int64_t bs,
-                                                        int64_t nb, int e, int m) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= outer * nb * inner) return;
-  int64_t o, b, c;
-  block_col(t, inner, nb, o, b, c);
-  const int64_t k0 = b * bs, rows = (n - k0 < bs) ? n - k0 : bs;
-  const int64_t off = (o * n + k0) * inner + c;
-  const float x = e8m0_decode(scales[t]);
-  for (int64_t r = 0; r < rows; ++r) out[off + r * inner] = mx_decode(codes[off + r * inner], e, m) * x;
-}
-
 int check_shape(int64_t outer, int64_t n, int64_t inner, int64_t bs, int e, int m, const char* who) {
   if (outer < 0 || n < 0 || inner < 0 || bs < 1) return mxq::invalid(std::string(who) + ": bad shape");
   if (!code_format_ok(e, m)) return mxq::invalid(std::string(who) + ": not an OCP MX element format");
@@ -123,8 +109,13 @@ extern "C" int mxq_dequantize_packed(const uint8_t* codes, const uint8_t* scales
   if (int rc = check_shape(outer, n, inner, block_size, e, m, "mxq_dequantize_packed")) return rc;
   if (outer == 0 || n == 0 || inner == 0) return MXQ_OK;
   if (!codes || !scales || !out) return mxq::invalid("mxq_dequantize_packed: NULL pointer");
-  const int64_t nb = mxq::ceil_div(n, block_size), threads = outer * nb * inner;
-  k_dequant_packed<<<mxq::grid_for(threads, 256), 256, 0, mxq::as_stream(stream)>>>(codes, scales, out, outer, n, inner,
-                                                                                     block_size, nb, e, m);
+  auto go = [&](auto src) {
+    mxq_quant::launch_dequant(src, out, outer, n, inner, block_size, mxq::as_stream(stream));
+  };
+  if (e == 4) go(mxq_quant::ByteSource<4, 3>{codes, scales});
+  else if (e == 5) go(mxq_quant::ByteSource<5, 2>{codes, scales});
+  else if (e == 3) go(mxq_quant::ByteSource<3, 2>{codes, scales});
+  else if (m == 3) go(mxq_quant::ByteSource<2, 3>{codes, scales});
+  else go(mxq_quant::ByteSource<2, 1>{codes, scales});
   return mxq::check_launch("mxq_dequantize_packed");
 }

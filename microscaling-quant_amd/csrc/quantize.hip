@@ -1,5 +1,6 @@
 // C entry points of block quantization and dequantization; the kernels live in quantize_impl.h and are
 // instantiated per input type in quantize_{f32,bf16,f16}.hip.
+#include "dequant_impl.h"
 #include "quantize_impl.h"
 
 int mxq_quantize_f32(const void*, float*, float*, int64_t, int64_t, int64_t, int64_t, const mxq_block_spec&, hipStream_t);
@@ -54,23 +55,7 @@ extern "C" int mxq_block_dequantize(const float* P, const float* X, float* out, 
   if (outer < 0 || n < 0 || inner < 0 || block_size < 1) return mxq::invalid("mxq_block_dequantize: bad shape");
   if (outer == 0 || n == 0 || inner == 0) return MXQ_OK;
   if (!P || !X || !out) return mxq::invalid("mxq_block_dequantize: NULL pointer");
-  const int64_t nb = mxq::ceil_div(n, block_size);
-  const uintptr_t ap = reinterpret_cast<uintptr_t>(P), ax = reinterpret_cast<uintptr_t>(X),
-                  ao = reinterpret_cast<uintptr_t>(out);
-  auto aligned = [&](int vec) { return inner % vec == 0 && (ap | ax | ao) % (vec * 4) == 0; };
-  const int vec = aligned(4) ? 4 : (aligned(2) ? 2 : 1);
-  const int64_t count = outer * n * (inner / vec), xcount = outer * nb * inner;
-  hipStream_t st = mxq::as_stream(stream);
-  auto go = [&](auto vec_const, auto idx) {
-    constexpr int VEC = decltype(vec_const)::value;
-    using I = decltype(idx);
-    mxq_quant::k_dequant_flat<VEC, I><<<mxq::grid_for(count, 256), 256, 0, st>>>(
-        P, X, out, (I)count, (I)(inner / VEC), (I)n, (I)block_size, (I)nb);
-  };
-  const bool narrow = count * vec < ((int64_t)1 << 31) && xcount < ((int64_t)1 << 31);   // no wrap near the end
-  if (vec == 4) narrow ? go(std::integral_constant<int, 4>{}, uint32_t{}) : go(std::integral_constant<int, 4>{}, int64_t{});
-  else if (vec == 2) narrow ? go(std::integral_constant<int, 2>{}, uint32_t{}) : go(std::integral_constant<int, 2>{}, int64_t{});
-  else narrow ? go(std::integral_constant<int, 1>{}, uint32_t{}) : go(std::integral_constant<int, 1>{}, int64_t{});
+  mxq_quant::launch_dequant(mxq_quant::FloatSource{P, X}, out, outer, n, inner, block_size, mxq::as_stream(stream));
   return mxq::check_launch("mxq_block_dequantize");
 }
 

@@ -1,4 +1,4 @@
-// Fused MX block quantization and dequantization for gfx950.
+// Fused MX block quantization for gfx950.
 //
 // A tensor is viewed as (outer, n, inner) with the block axis n in the middle.  Three layouts:
 //   split    (block 32): eight lanes of a wavefront share one block column of VEC adjacent columns, four rows
@@ -971,25 +971,6 @@ int launch_quant_t(const T* M, float* P, float* X, int64_t n, int64_t inner, con
   const int vec_out = inner % 4 == 0 && reinterpret_cast<uintptr_t>(P) % 16 == 0;
   k_quant_t<T, ELEM, MODE><<<dim3((unsigned)tiles), 256, 0, st>>>(M, P, X, n, inner, tiles_k, vec_in, vec_out, q);
   return mxq::check_launch("mxq_block_quantize_t");
-}
-
-// out = P * expand(X) as one flat pass over the (outer, n, inner) view: a thread takes VEC adjacent elements of a
-// row (one block, so one VEC-wide load of X), and every thread has work, whatever the block size and shape.
-// I is uint32_t while the element count fits it (cheap index arithmetic), else int64_t.
-template <int VEC, typename I>
-__global__ void __launch_bounds__(256) k_dequant_flat(const float* __restrict__ P, const float* __restrict__ X,
-                                                      float* __restrict__ out, I count, I inner_v, I n, I bs, I nb) {
-  const I t = (I)blockIdx.x * 256u + (I)threadIdx.x;
-  if (t >= count) return;
-  const I row = t / inner_v;                      // (o, k) flattened
-  const I iv = t - row * inner_v;
-  const I o = row / n, k = row - o * n;
-  float v[VEC], xs[VEC];
-  load_vec<float, VEC>(P + (int64_t)t * VEC, v);
-  load_vec<float, VEC>(X + ((int64_t)(o * nb + k / bs) * inner_v + iv) * VEC, xs);
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) v[j] = v[j] * xs[j];
-  store_vec_nt<VEC>(out + (int64_t)t * VEC, v);
 }
 
 // ------------------------------------------------------------------------------------------ host side

@@ -84,6 +84,47 @@ def test_pack_unpack_dequantize(cuda, fmt):
     assert_bits_equal(d.cpu().numpy(), mxq.block.mxgemmini.dequantize(P, X).cpu().numpy(), "dequantize")
 
 
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("shape,axis,bs", [((40, 256), 0, 32), ((70, 9), 0, 32), ((33, 5), 0, 16), ((70, 3), 0, 32),
+                                           ((9, 259), 1, 32), ((11, 37), 1, 6), ((11, 2), 1, 32), ((1100, 2049), 0, 32),
+                                           ((2, 50, 7), 1, 6)])
+def test_dequantize_every_code_at_any_address(cuda, fmt, shape, axis, bs):
+    """All 256 code bytes under all 256 scale bytes (subnormal scales, NaN, bits past the code's among them), rows
+    of every length around the four codes a thread takes, at odd addresses, against the oracle."""
+    import mxq
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(n)
+    C = (rng.permutation(n) % 256).astype(np.uint8).reshape(shape)
+    xs = list(shape)
+    xs[axis] = -(-shape[axis] // bs)
+    S = (rng.permutation(int(np.prod(xs))) * 7 % 256).astype(np.uint8).reshape(xs)
+    odd = [torch.empty(a.size + 1, dtype=torch.uint8, device="cuda")[1:].view(a.shape).copy_(torch.from_numpy(a))
+           for a in (C, S)]
+    got = mxq.packed.dequantize(*odd, fmt, axis, bs).cpu().numpy()
+    e, m = op.FORMATS[fmt]
+    with np.errstate(all="ignore"):                         # a code is its byte's low 1 + e + m bits
+        want = ob.dequantize(op.decode(C & ((2 << (e + m)) - 1), e, m), op.e8m0_decode(S), axis, bs)
+    assert_bits_equal(got, want, f"{fmt} {shape} axis {axis} blocks of {bs}")
+
+
+@pytest.mark.parametrize("method,opts", [("mxgemmini", {"rounding_mode": "rne"}), ("ocp", {}), ("mxquant", {})])
+@pytest.mark.parametrize("fmt", FMTS)
+def test_quantize_packed_ragged_rows(cuda, method, opts, fmt):
+    """One-pass bytes of rows of any length, at an odd address, against pack() of the float32 quantizer's outputs."""
+    import mxq
+    g = torch.Generator(device="cuda").manual_seed(5)
+    for dtype in (torch.float32, torch.bfloat16, torch.float16):
+        for shape, axis in [((7, n), 1) for n in (1, 3, 4, 31, 33, 131)] + \
+                [((70, n), 0) for n in (2, 3, 5, 7, 8, 9, 15, 33, 67)] + [((2, 4100, 1029), 1)]:
+            V = torch.empty(int(np.prod(shape)) + 1, dtype=dtype, device="cuda")[1:].view(shape)
+            V.copy_(torch.randn(shape, generator=g, device="cuda") * 3)
+            kw = dict(opts)
+            P, X = getattr(mxq.block, method).quantize(V, fmt, axis=axis, **kw)
+            want = mxq.packed.pack(P, X, fmt, axis, check=False)
+            got = mxq.packed.quantize(V, fmt, method, axis, check=False, **kw)
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), f"{method} {fmt} {dtype} {shape} {axis}"
+
+
 def test_packed_specials_and_errors(cuda):
     """NaN codes: E4M3 and E5M2 have them, FP6 and FP4 raise; a non-power-of-two scale of a nonzero block
     raises; mxquant's smallest E4M3 qtorch values are no OCP E4M3 codes; check=False returns the bytes."""
