@@ -500,6 +500,25 @@ def test_softmax_quantize_t_row_counts(cuda, R, T):
         assert torch.equal(torch.nan_to_num(x).view(torch.int32), torch.nan_to_num(y).view(torch.int32)), name
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("tokens", [0, 1, 2, 31, 65, 333])
+def test_mxlinear_reads_tokens_as_they_lie(cuda, dtype, tokens):
+    """A library quantizer on x^T as it lies against the same quantizer behind a callable, which is given the
+    contiguous float32 copy: the same bits, for token views with strides and an odd offset too, whole and in chunks."""
+    import mxq
+    from mxq import Scheme
+    from mxq.nn import MXLinear
+    hw = _hw(mxq)
+    copied = Scheme("copied", a=lambda V: hw.a(V), b=hw.b, reduce=hw.reduce)
+    lin = torch.nn.Linear(131, 48, device="cuda", dtype=dtype)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x = torch.randn(tokens * 140 + 1, generator=g, device="cuda").to(dtype)[1:].view(tokens, 140)
+    for view in (x[:, :131], x[:, 5:136].contiguous(), x[:, :131].reshape(1, tokens, 131)):
+        want = MXLinear(lin, copied)(view)
+        for chunk in (None, 7):
+            assert torch.equal(MXLinear(lin, hw, chunk=chunk)(view), want)
+
+
 def test_exp_underflows_past_minus_128(cuda):
     """The softmax kernel's tail rule rests on exp(x) = +0 on the device for every float32 x <= -128 (e^-103.98 is
     already below half the smallest subnormal): every float32 in [-512, -128] and a strided sample of the rest down
