@@ -44,8 +44,8 @@ VALU_LANE_OPS = 157.3e12 / 2
 # rounds it to the lane grid (adding and subtracting a constant, two full-rate operations, or v_rndne_f32 at half
 # rate: 2 slots either way), adds exactly and rounds to nearest even at m bits (three full-rate operations) = 8.
 # The roof prices every MAC at that step.
-SLOTS_PER_MAC_MODEL = 8
-VALU_ROOF_TOPS = VALU_LANE_OPS / SLOTS_PER_MAC_MODEL * 2 / 1e12   # 19.66 TOP/s emulated
+SLOTS_PER_MAC_MODEL = 7
+VALU_ROOF_TOPS = VALU_LANE_OPS / SLOTS_PER_MAC_MODEL * 2 / 1e12   # 22.47 TOP/s emulated
 # The algorithmic model of the reference's MAC (roofline.frac_survey_model): 10 lane-operations per emulated MAC
 # (multiply, truncate, flush, saturate, the two lane roundings, the +0 fix-up, the exact add, its rounding, the
 # zero short-circuit), priced at the same 78.6 T lane-operations per second; the fast kernel does the step in
@@ -792,10 +792,10 @@ def main():
                          "source": "SQ_INSTS_VALU x 64 / emulated MACs, profiles/systolic_fast_c2_valu.txt"},
                      "note": "VALU-bound emulation (neither HBM nor MFMA): achieved = 2 x 8,589,934,592 emulated "
                              "MACs / the fast kernel's average duration; peak = MI355X vector FP32 157.3 TFLOP/s = "
-                             "78.6 T full-rate lane-slots/s, / 8 slots per emulated MAC (an e4 lane step on gfx950: "
+                             "78.6 T full-rate lane-slots/s, / 7 slots per emulated MAC (an e4 lane step on gfx950: "
                              "multiply, mask, the add and subtract that round to the lane's step, the exact add and "
-                             "a 3-op nearest-even split, one slot each) x 2 ops per MAC; frac_survey_model prices every "
-                             "MAC at 10 lane-operations (15.73 TOP/s), a model the kernel's 8-operation step beats; "
+                             "a 2-op nearest even, one slot each) x 2 ops per MAC; frac_survey_model prices every "
+                             "MAC at 10 lane-operations (15.73 TOP/s), a model the kernel's 7-operation step beats; "
                              "`executed.frac` holds the counted instructions (full- and half-rate alike) against "
                              "the 78.6 T lane rate"},
     }
