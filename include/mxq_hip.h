@@ -34,8 +34,9 @@ typedef void* mxq_stream_t;
  *      mask values; mxq_systolic_fast_lanes; the dither entry points.
  *   3  mxq_mx_pack_bytes; the MXQ_EBUSY status of mxq_systolic_noalloc.
  *   4  mxq_attend_windows writes one flag word per call and 64 query rows, each whole (was one per call, zeroed
- *      by the caller). */
-#define MXQ_ABI_VERSION 4
+ *      by the caller).
+ *   5  mxq_systolic_plan_of. */
+#define MXQ_ABI_VERSION 5
 
 enum { MXQ_OK = 0, MXQ_EINVAL = 1, MXQ_EHIP = 2, MXQ_EBUSY = 3 };
 
@@ -202,6 +203,20 @@ typedef struct mxq_systolic_hints {
  * other case runs the general kernel alone, which reads every row of A and computes every tile), else 0.  No
  * counterpart in the reference: a caller that leaves rows of A unwritten under k_end asks this first. */
 int mxq_systolic_fast_lanes(const int32_t* lane_e, const int32_t* lane_m, int32_t size, const mxq_arith_spec* arith);
+
+/* Which kernel a systolic call of this shape runs, and on what tile of outputs a workgroup; no counterpart in the
+ * reference (tests state with it which kernel they reach).  Answered on the host from the rule the calls themselves
+ * use: no device is touched, of the hints only which are NULL matters, a NULL layout means contiguous operands, and
+ * force_general is taken as 0.  A kernel other than MXQ_SYS_GENERAL hands operands outside its datapath's range to the
+ * general rule, tile by tile. */
+enum { MXQ_SYS_GENERAL = 0, MXQ_SYS_SMALL = 1, MXQ_SYS_TILE = 2, MXQ_SYS_FAST = 3 };
+typedef struct mxq_systolic_plan {
+  int32_t kernel;              /* MXQ_SYS_* */
+  int32_t rows, cols, waves;   /* outputs and waves of a workgroup */
+} mxq_systolic_plan;
+int mxq_systolic_plan_of(const mxq_systolic_layout* layout, int64_t count, int64_t K, int64_t M, int64_t N,
+                         const int32_t* lane_e, const int32_t* lane_m, int32_t size, int32_t block_size,
+                         const mxq_arith_spec* arith, const mxq_systolic_hints* hints, mxq_systolic_plan* plan);
 
 /* An elementwise step mxq_systolic_batched applies to every output as it is stored (no counterpart in the
  * reference as a fused step: it is attention's score step, mxq/nn/_attention.py:128-135, done where the scores

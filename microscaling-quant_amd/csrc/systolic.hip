@@ -982,7 +982,7 @@ void launch_fast(int size, bool bf16_last, bool hwf, dim3 grid, hipStream_t st, 
 
 // Which kernel computes a call, and its tile.
 struct Plan {
-  enum Kernel { kGeneral, kSmall, kTile, kFast } kernel;
+  enum Kernel { kGeneral = MXQ_SYS_GENERAL, kSmall = MXQ_SYS_SMALL, kTile = MXQ_SYS_TILE, kFast = MXQ_SYS_FAST } kernel;
   SmallTile small;
   int bm, bn;              // the tile kernels' tile
 };
@@ -1013,12 +1013,16 @@ constexpr double kMacCost[] = {1.0, 1.29, 1.36, 2.27, 2.3, 2.02};
 
 Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
   // hints that leave rows of A unread (a_live) or outputs unstored (c_end) need a tile kernel, whose own limits are
-  // blocks of 32 and a lane's offset in 32 bits; k_systolic_small's are its 32-bit rows and lane offsets
+  // blocks of 32 and a lane's offset in 32 bits; k_systolic_small's are its 32-bit rows and lane offsets: of B, and of
+  // the 64 * waves / rows rows of A its threads reach from one address (small_fits)
   const bool small_ok = !a.c_end && !a.a_live && a.K < (int64_t(1) << 30) && a.B.ld < (int64_t(1) << 18);
   const bool tile_ok = a.block_size == KT && a.A.ld < (int64_t(1) << 28) && a.B.ld < (int64_t(1) << 28);
   const bool every_small = kind == kE4Final || kind == kMxqFinal;
+  auto small_fits = [&](int rows, int waves) {
+    return small_ok && a.A.ld < (int64_t(1) << 32) / (64 * waves / rows) && mxq::ceil_div(a.M, rows) <= 65535;
+  };
   Plan p{};
-  if (a.M == 1 && every_small && small_ok) {
+  if (a.M == 1 && every_small && small_fits(1, 16)) {
     // one row: 32 columns a workgroup while that leaves half the CUs one (K = 2048, 5632 columns: 23 us, 35 with 16,
     // 25 with 64), 64 when that makes one for every CU (32000 columns: 65, 85 with 32)
     auto wgs = [&](int log_cw) { return mxq::ceil_div(a.N, int64_t(1) << log_cw) * count; };
@@ -1029,9 +1033,8 @@ Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
   double best = 0.0;
   for (const Shape& sh : kShapes) {
     const bool tile = sh.kernel == Plan::kTile;
-    if (tile ? !tile_ok : !small_ok) continue;
+    if (tile ? !tile_ok : !small_fits(sh.rows, sh.waves)) continue;
     if (!tile && !every_small && !(sh.rows == 4 || (sh.rows == 8 && sh.waves == 8))) continue;
-    if (!tile && mxq::ceil_div(a.M, sh.rows) > 65535) continue;
     const int64_t n = mxq::ceil_div(a.M, sh.rows) * mxq::ceil_div(a.N, int64_t(1) << sh.log_cols) * count;
     double t = std::max(sh.alone, sh.fill + sh.round * (double)mxq::ceil_div(n, 256));
     t *= (sh.fixed + (1.0 - sh.fixed) * kMacCost[kind]) * (double)a.K / 2048.0;
@@ -1047,7 +1050,7 @@ Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
   }
   // e4 lanes with other blocks than 32 (or wider rows): k_systolic_fast while it has a workgroup for every CU
   if (!tile_ok && kind <= kE4 &&
-      (!small_ok || (a.M > 16 && mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= 256))) {
+      (p.kernel == Plan::kGeneral || (a.M > 16 && mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= 256))) {
     // its tiles: 64 x 64, 32 x 64 or 32 x 32 outputs, the largest that gives every CU four workgroups
     const int64_t want = 4 * 256;
     p.kernel = Plan::kFast;
@@ -1055,6 +1058,22 @@ Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
     p.bn = p.bm == 64 || mxq::ceil_div(a.M, 32) * mxq::ceil_div(a.N, 64) * count >= want ? 64 : 32;
   }
   return p;
+}
+
+// The fast datapath of these lanes (-1: none), its constants and its bound on max|a| * max|b|.
+int datapath_of(const int32_t* e, const int32_t* m, int size, const mxq_arith_spec& ar, int64_t K, FastLanes* fl,
+                float* prod_max) {
+  const bool hwf = is_hw_final(e, m, size);
+  bool high = false;
+  if (K <= 0) return -1;
+  if (lanes_fast(e, m, size, ar)) {
+    *fl = make_fast_lanes(e, m, size, ar);
+    *prod_max = fast_prod_bound(e, m, size);
+    return hwf ? kE4Final : kE4;
+  }
+  if (lanes_wide(e, m, size, ar, fl, prod_max)) return kWide;
+  if (lanes_mxquant(e, m, size, ar, K, fl, prod_max, &high)) return high ? kMxqHigh : hwf ? kMxqFinal : kMxq;
+  return -1;
 }
 
 bool lanes_valid(const int32_t* e, const int32_t* m, int size) {
@@ -1070,22 +1089,9 @@ int run_systolic(const SysArgs& base, const int32_t* lane_e, const int32_t* lane
   const mxq_arith_spec& ar = base.ar;
   SysArgs a = base;
   for (int i = 0; i < a.size; ++i) { a.lane_e[i] = (int8_t)lane_e[i]; a.lane_m[i] = (int8_t)lane_m[i]; }
-  // the datapath: its constants and its bound on max|a| * max|b|
-  int kind = -1;
   FastLanes fl;
+  const int kind = force_general ? -1 : datapath_of(lane_e, lane_m, a.size, ar, a.K, &fl, &a.fast_prod_max);
   const bool bf16_last = lane_e[a.size - 1] == 8, hwf = is_hw_final(lane_e, lane_m, a.size);
-  if (!force_general && a.K > 0) {
-    bool high = false;
-    if (lanes_fast(lane_e, lane_m, a.size, ar)) {
-      kind = hwf ? kE4Final : kE4;
-      fl = make_fast_lanes(lane_e, lane_m, a.size, ar);
-      a.fast_prod_max = fast_prod_bound(lane_e, lane_m, a.size);
-    } else if (lanes_wide(lane_e, lane_m, a.size, ar, &fl, &a.fast_prod_max)) {
-      kind = kWide;
-    } else if (lanes_mxquant(lane_e, lane_m, a.size, ar, a.K, &fl, &a.fast_prod_max, &high)) {
-      kind = high ? kMxqHigh : hwf ? kMxqFinal : kMxq;
-    }
-  }
   const Plan plan = kind < 0 ? Plan{} : plan_launch(a, count, kind);
   if (plan.kernel == Plan::kSmall) {
     mxq::KernelTimer timer("systolic_small", st);
@@ -1148,6 +1154,17 @@ int run_systolic(const SysArgs& base, const int32_t* lane_e, const int32_t* lane
   return mxq::check_launch("mxq_systolic");
 }
 
+void take_hints(SysArgs& a, const mxq_systolic_hints* hints) {
+  if (!hints) return;
+  a.skip = hints->skip;
+  a.skip_rows = mxq::ceil_div(a.M, 32);
+  a.skip_cols = mxq::ceil_div(a.N, 32);
+  a.k_end = hints->k_end;
+  a.kend_groups = mxq::ceil_div(a.M, 64);
+  a.a_live = hints->k_end ? hints->a_live : nullptr;
+  a.c_end = hints->skip ? hints->c_end : nullptr;
+}
+
 int check_common(int64_t K, int64_t M, int64_t N, int64_t count, const int32_t* lane_e, const int32_t* lane_m,
                  int32_t size, int32_t block_size, const mxq_arith_spec* arith) {
   if (!arith || !lane_e || !lane_m) return mxq::invalid("mxq_systolic: NULL spec or lanes");
@@ -1168,6 +1185,27 @@ extern "C" int mxq_systolic_fast_lanes(const int32_t* lane_e, const int32_t* lan
                                        const mxq_arith_spec* arith) {
   if (!arith || !lane_e || !lane_m || size < 1 || size > kMaxLanes || !lanes_valid(lane_e, lane_m, size)) return 0;
   return lanes_fast(lane_e, lane_m, size, *arith) ? 1 : 0;
+}
+
+extern "C" int mxq_systolic_plan_of(const mxq_systolic_layout* layout, int64_t count, int64_t K, int64_t M, int64_t N,
+                                    const int32_t* lane_e, const int32_t* lane_m, int32_t size, int32_t block_size,
+                                    const mxq_arith_spec* arith, const mxq_systolic_hints* hints,
+                                    mxq_systolic_plan* plan) {
+  if (int rc = check_common(K, M, N, count, lane_e, lane_m, size, block_size, arith)) return rc;
+  if (!plan) return mxq::invalid("mxq_systolic_plan_of: NULL plan");
+  SysArgs a{};
+  a.A.ld = layout ? layout->ld_a : M;
+  a.B.ld = layout ? layout->ld_b : N;
+  a.K = K; a.M = M; a.N = N; a.size = size; a.block_size = block_size;
+  take_hints(a, hints);
+  FastLanes fl;
+  const int kind = datapath_of(lane_e, lane_m, size, *arith, K, &fl, &a.fast_prod_max);
+  const Plan p = kind < 0 ? Plan{} : plan_launch(a, count, kind);
+  *plan = mxq_systolic_plan{p.kernel, 32, 32, 4};                 // k_systolic_gen's tile
+  if (p.kernel == Plan::kSmall) *plan = {p.kernel, p.small.rows, 1 << p.small.log_cw, p.small.waves};
+  if (p.kernel == Plan::kTile) *plan = {p.kernel, p.bm, p.bn, p.bm / 8};
+  if (p.kernel == Plan::kFast) *plan = {p.kernel, p.bm, p.bn, 4};
+  return MXQ_OK;
 }
 
 extern "C" int mxq_systolic(const float* P_A, const float* X_A, const float* P_B, const float* X_B, float* C,
@@ -1213,15 +1251,7 @@ extern "C" int mxq_systolic_batched(const float* P_A, const float* X_A, const fl
   a.B = {P_B, L.ld_b, L.batch_b}; a.XB = {X_B, L.ld_xb, L.batch_xb};
   a.C = C; a.ldc = L.ld_c; a.batch_c = L.batch_c; a.flags = workspace;
   a.K = K; a.M = M; a.N = N; a.size = size; a.block_size = block_size; a.ar = *arith;
-  if (hints) {
-    a.skip = hints->skip;
-    a.skip_rows = mxq::ceil_div(M, 32);
-    a.skip_cols = mxq::ceil_div(N, 32);
-    a.k_end = hints->k_end;
-    a.kend_groups = mxq::ceil_div(M, 64);
-    a.a_live = hints->k_end ? hints->a_live : nullptr;
-    a.c_end = hints->skip ? hints->c_end : nullptr;
-  }
+  take_hints(a, hints);
   if (epilogue) {
     a.epi_on = 1;
     a.epi = *epilogue;

@@ -26,7 +26,7 @@ _lib: Optional[ctypes.CDLL] = None
 _FN = {}            # entry point name -> its ctypes function, filled by load()
 
 #: the MXQ_ABI_VERSION of include/mxq_hip.h these signatures follow; a library reporting another is refused
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 c_i32, c_i64, c_f32, c_f64, c_ptr = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_double, ctypes.c_void_p
 
@@ -69,6 +69,11 @@ class SystolicLayout(ctypes.Structure):
                                      "ld_c", "batch_c")]
 
 
+class SystolicPlan(ctypes.Structure):
+    """mxq_systolic_plan (include/mxq_hip.h): the kernel (SYS_*), and the outputs and waves of a workgroup."""
+    _fields_ = [("kernel", c_i32), ("rows", c_i32), ("cols", c_i32), ("waves", c_i32)]
+
+
 class AnchorSpec(ctypes.Structure):
     """mxq_anchor_spec (include/mxq_hip.h)."""
     _fields_ = [(n, c_i32) for n in ("width", "drop", "headroom", "has_emin", "emin", "nbits")]
@@ -98,6 +103,8 @@ SIGNATURES = {
     "mxq_systolic_batched": (c_i32, [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, ctypes.POINTER(SystolicLayout), c_i64,
                                      c_i64, c_i64, c_i64, c_ptr, c_ptr, c_i32, c_i32, ctypes.POINTER(ArithSpec),
                                      c_ptr, c_ptr, c_ptr, c_i32, c_ptr]),
+    "mxq_systolic_plan_of": (c_i32, [ctypes.POINTER(SystolicLayout), c_i64, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_i32,
+                                     c_i32, ctypes.POINTER(ArithSpec), c_ptr, ctypes.POINTER(SystolicPlan)]),
     "mxq_systolic_noalloc": (c_i32, [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_ptr, c_ptr, c_i32,
                                      c_i32, ctypes.POINTER(ArithSpec), c_i32, c_ptr]),
     "mxq_systolic_workspace": (c_i64, [c_i64, c_i64, c_i64, c_i64]),
@@ -150,6 +157,7 @@ MODE_CODE = {"ties_away": 0, "rne": 1, "truncate": 2}
 MS_MODE_CODE = {"nearest": 0, "even": 1, "floor": 2, "dither": 3}
 GRID_CODE = {"qtorch": 0, "ieee": 1, "ocp": 2}
 ARITH_MXGEMMINI, ARITH_MXQUANT = 0, 1
+SYS_GENERAL, SYS_SMALL, SYS_TILE, SYS_FAST = 0, 1, 2, 3
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:

@@ -153,3 +153,17 @@ class HostNumerics:
 
     def e8m0_decode(self, b):
         return self._un("h_e8m0_decode", b, in_dtype=np.uint8)
+
+
+def systolic_plan(K, M, N, arith, schedule, size=16, block_size=32, count=1, ld_a=None, ld_b=None, **hints):
+    """(kernel, rows, cols, waves) of a systolic call (mxq_systolic_plan_of; no GPU needed): kernel "general",
+    "small", "tile" or "fast".  hints: any of skip, k_end, a_live, c_end set to True stands for that hint given."""
+    from mxq import _lib
+    le, lm = ((ctypes.c_int32 * size)(*[int(f[i]) for f in schedule]) for i in (0, 1))
+    lay = _lib.SystolicLayout(ld_a=ld_a or M, ld_b=ld_b or N)
+    h = _lib.SystolicHints(**{k: 1 for k, v in hints.items() if v})
+    p = _lib.SystolicPlan()
+    _lib.load()
+    _lib.run("mxq_systolic_plan_of", ctypes.byref(lay), count, K, M, N, le, lm, size, block_size, arith.kernel.ctype(),
+             ctypes.byref(h), ctypes.byref(p))
+    return ("general", "small", "tile", "fast")[p.kernel], p.rows, p.cols, p.waves

@@ -49,7 +49,7 @@ def test_structs_match_header():
     from mxq import _lib
     text = open(HEADER).read()
     for struct, py in (("mxq_block_spec", _lib.BlockSpec), ("mxq_arith_spec", _lib.ArithSpec),
-                       ("mxq_systolic_layout", _lib.SystolicLayout)):
+                       ("mxq_systolic_layout", _lib.SystolicLayout), ("mxq_systolic_plan", _lib.SystolicPlan)):
         body = re.search(r"typedef struct " + struct + r"\s*\{(.*?)\}\s*" + struct + ";", text, flags=re.S).group(1)
         body = re.sub(r"/\*.*?\*/|//[^\n]*", "", body, flags=re.S)
         fields = [(t, n.strip()) for t, names in re.findall(r"\b(int32_t|float|double|int64_t)\s+([a-z_0-9, ]+);", body)
@@ -67,7 +67,7 @@ def test_struct_offsets_match_header(tmp_path):
     from mxq import _lib
     structs = {"mxq_block_spec": _lib.BlockSpec, "mxq_arith_spec": _lib.ArithSpec,
                "mxq_systolic_layout": _lib.SystolicLayout, "mxq_systolic_hints": _lib.SystolicHints,
-               "mxq_systolic_epilogue": _lib.SystolicEpilogue}
+               "mxq_systolic_epilogue": _lib.SystolicEpilogue, "mxq_systolic_plan": _lib.SystolicPlan}
     lines = ['#include <stddef.h>', '#include <stdio.h>', '#include "mxq_hip.h"', "int main(void) {"]
     for name, py in structs.items():
         lines.append(f'  printf("{name} size %zu\\n", sizeof({name}));')

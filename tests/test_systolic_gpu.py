@@ -653,3 +653,21 @@ def test_tiles_of_any_shape(cuda, name, K, M, N):
     got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
     want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
     assert_bits_equal(got, want, f"{name} {M}x{N}, K={K}")
+
+
+@pytest.mark.parametrize("M,K,ld", [(1, 1100, 4_198_405), (4, 300, (1 << 24) + 1)])
+def test_rows_of_a_far_apart(cuda, M, K, ld):
+    """Rows of A so far apart that a few hundred of them pass 2^32 elements (18 and 20 GB of them), against the same
+    operand side by side."""
+    from mxq import _lib, matmul
+    from mxq.matmul._systolic import systolic_batched
+    N = 160
+    rng = np.random.default_rng(M)
+    P, X = (torch.from_numpy(v).cuda() for v in _codes(rng, K, M))
+    B, XB = (torch.from_numpy(v).cuda() for v in _codes(rng, K, N, scale=0.02))
+    far = torch.empty((K - 1) * ld + M, device="cuda").as_strided((K, M), (ld, 1))
+    far.copy_(P)
+    C = torch.full((M, N), 7.0, device="cuda")
+    lay = _lib.SystolicLayout(ld_a=ld, ld_xa=M, ld_b=N, ld_xb=N, ld_c=N)
+    systolic_batched((far, X, B, XB), lay, 1, K, M, N, C, matmul.MXGEMMINI(), HW_FINAL)
+    assert_bits_equal(C.cpu().numpy(), matmul.systolic(P, X, B, XB, matmul.MXGEMMINI(), HW_FINAL).cpu().numpy())
