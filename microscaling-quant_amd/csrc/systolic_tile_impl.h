@@ -49,12 +49,15 @@ __device__ __forceinline__ void lds_row(const float* src, float (&v)[TM]) {
 }
 
 // WHOLE: every tile lies inside C and the operands' rows are whole fours of columns, 16-byte aligned (HW_FINAL's own
-// instances, which leave the choice a stage out: 512 x 4096 outputs, K = 4096: 0.942 ms, 0.970 without them).
+// instances, which leave the choice a stage out: 512 x 4096 outputs, K = 4096: 0.942 ms, 0.970 without them).  The
+// others take a last block that is alone in its stage of two by itself (2048 x 4096 outputs: K = 32 76 -> 45 us, K = 96
+// 135 -> 102; ladder e4m4, 1024 x 2048, K = 200: 89 -> 81); in WHOLE's instance that code cost 2 % of the time above.
 template <int KIND, int SIZE, bool BF16_LAST, int BM, bool WHOLE>
 __global__ void __launch_bounds__(BM * 8, 4) k_systolic_tile(const SysArgs args, const FastLanes fl) {
   static_assert(BM == 64 || BM == 32, "64 x 64 or 32 x 32 tiles");
   constexpr int BN = BM, TM = BM == 32 ? 2 : 4, TN = 2, KS = BM, NBS = KS / KT;   // a stage has as many rows as a tile
   constexpr int NT = (BM / TM) * (BN / TN), NWV = NT / 64;   // threads, waves
+  constexpr bool HALF = NBS > 1 && !WHOLE;
   const Datapath<KIND, SIZE, BF16_LAST> dp{fl};
   // the two stage buffers are distinct arrays, each named where it is used: the compiler can then tell the
   // direct-to-LDS loads into one from the reads of the other, and does not wait for the loads before them
@@ -121,7 +124,12 @@ __global__ void __launch_bounds__(BM * 8, 4) k_systolic_tile(const SysArgs args,
     if (k + KS <= stop) {
       load_rows<BM, ROWS>(qa + k * args.A.ld, args.A.ld, va, swave * ROWS, da);
       load_rows<BN, ROWS>(qb + k * args.B.ld, args.B.ld, vb, swave * ROWS, db);
-    } else {                                        // the end is inside the stage: through registers, zeros past it
+    } else if (HALF && k + KT == stop) {         // the last block, alone in its stage: the waves of its rows load it
+      if (swave * ROWS < KT) {
+        load_rows<BM, ROWS>(qa + k * args.A.ld, args.A.ld, va, swave * ROWS, da);
+        load_rows<BN, ROWS>(qb + k * args.B.ld, args.B.ld, vb, swave * ROWS, db);
+      }
+    } else {                                        // the end is inside a block: through registers, zeros past it
 #pragma unroll 1
       for (int e = threadIdx.x; e < KS * BM; e += NT) {
         const int r = e / BM, c = e % BM;
@@ -161,11 +169,13 @@ __global__ void __launch_bounds__(BM * 8, 4) k_systolic_tile(const SysArgs args,
     for (int y = 0; y < TN; ++y) C[x][y] = 0.0f;
 
   bool large = false;                               // some scale so far was above xs_hi
-  // one stage: its operand maxima read back from LDS, then its blocks reduced into C
-  auto reduce_stage = [&](const float (&ca)[KS][BM], const float (&cb)[KS][BN], int buf)
+  // a stage of `blocks` blocks: their operand maxima read back from LDS, then the blocks reduced into C
+  static_assert(KT % ROWS == 0 && KT * BN / 4 == NT, "a block is whole waves' rows and a float4 a thread");
+  auto reduce_stage = [&](auto blocks, const float (&ca)[KS][BM], const float (&cb)[KS][BN], int buf)
                           __attribute__((always_inline)) {
+    constexpr int BLOCKS = decltype(blocks)::value;
 #pragma unroll
-    for (int j = 0; j < KS * BN / 4 / NT; ++j) {
+    for (int j = 0; j < BLOCKS; ++j) {
       const float4 qa = reinterpret_cast<const float4*>(&ca[0][0])[threadIdx.x + NT * j];
       const float4 qb = reinterpret_cast<const float4*>(&cb[0][0])[threadIdx.x + NT * j];
       max_a = umax(max_a, umax(umax(f2u(qa.x) & 0x7FFFFFFFu, f2u(qa.y) & 0x7FFFFFFFu),
@@ -173,9 +183,9 @@ __global__ void __launch_bounds__(BM * 8, 4) k_systolic_tile(const SysArgs args,
       max_b = umax(max_b, umax(umax(f2u(qb.x) & 0x7FFFFFFFu, f2u(qb.y) & 0x7FFFFFFFu),
                                umax(f2u(qb.z) & 0x7FFFFFFFu, f2u(qb.w) & 0x7FFFFFFFu)));
     }
-    constexpr int BLOCKS_AT_ONCE = KIND == kE4Final || KIND == kE4 ? NBS : 1;   // the others' code is long
+    constexpr int BLOCKS_AT_ONCE = KIND == kE4Final || KIND == kE4 ? BLOCKS : 1;   // the others' code is long
 #pragma unroll BLOCKS_AT_ONCE
-    for (int q = 0; q < NBS; ++q) {
+    for (int q = 0; q < BLOCKS; ++q) {
       uint32_t denies = 0u;
 #pragma unroll
       for (int v = 0; v < NWV; ++v) denies |= denies_w[buf][q][v];
@@ -237,22 +247,31 @@ __global__ void __launch_bounds__(BM * 8, 4) k_systolic_tile(const SysArgs args,
       write_tile<TM, TN>(args, z, m0 + tm * TM, n0 + tn * TN, C);
     return;
   }
-  const int64_t kst = (stop + KS - 1) / KS * KS;    // whole stages, the last one's rows past `stop` zeros
+  // stages of NBS blocks up to `whole`, rows past `stop` zeros in the last of them; with HALF one block may be left
+  const int64_t kst = (nb + NBS - 1) / NBS * KS, whole = HALF ? nb / NBS * KS : kst;
+  constexpr std::integral_constant<int, NBS> kWholeStage{};
   if (kst > 0) {
     load_stage(0, sa0, sb0);
     finish_stage(0);
   }
-  for (int64_t k0 = 0; k0 < kst; k0 += 2 * KS) {
-    // even stage: buffer 0 reduced while stage k0 + 64 lands in buffer 1; odd stage: the other way round
+  for (int64_t k0 = 0; k0 < whole; k0 += 2 * KS) {
+    // even stage: buffer 0 reduced while stage k0 + KS lands in buffer 1; odd stage: the other way round
     const bool more1 = k0 + KS < kst;
     if (more1) load_stage(k0 + KS, sa1, sb1);
-    reduce_stage(sa0, sb0, 0);
+    reduce_stage(kWholeStage, sa0, sb0, 0);
     if (!more1) break;
     finish_stage(1);
+    if (HALF && k0 + KS >= whole) break;         // the block left over
     const bool more2 = k0 + 2 * KS < kst;
     if (more2) load_stage(k0 + 2 * KS, sa0, sb0);
-    reduce_stage(sa1, sb1, 1);
+    reduce_stage(kWholeStage, sa1, sb1, 1);
     if (more2) finish_stage(0);
+  }
+  if (HALF && whole < kst) {
+    const bool odd = (nb / NBS & 1) != 0;
+    const float (&ha)[KS][BM] = odd ? sa1 : sa0;
+    const float (&hb)[KS][BN] = odd ? sb1 : sb0;
+    reduce_stage(std::integral_constant<int, 1>{}, ha, hb, odd ? 1 : 0);
   }
 
   // rows from `stop` on: exact only if A holds +-0 there and B and every remaining block scale are finite
@@ -318,7 +337,9 @@ void launch_tile_ladder(dim3 grid, const SysArgs& a, const FastLanes& fl, hipStr
     auto aligned = [](const Operand& o) {
       return o.ld % 4 == 0 && o.batch % 4 == 0 && reinterpret_cast<uintptr_t>(o.p) % 16 == 0;
     };
-    if (a.M % a.fbm == 0 && a.N % a.fbm == 0 && aligned(a.A) && aligned(a.B))
+    // a half-full last stage of 64 rows is more than the instance saves (3 %) below 1024 rows
+    const bool half = a.fbm == 64 && a.K % 64 > 0 && a.K % 64 <= 32 && a.K < 1024;
+    if (a.M % a.fbm == 0 && a.N % a.fbm == 0 && !half && aligned(a.A) && aligned(a.B))
       return launch_tile_shape<KIND, SIZE, BF16_LAST, true>(grid, a, fl, st);
   }
   launch_tile_shape<KIND, SIZE, BF16_LAST, false>(grid, a, fl, st);

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import assert_bits_equal, special_f32
+from _util import assert_bits_equal, special_f32, systolic_plan
 from oracle import block as ob
 from oracle import numerics as nx
 from oracle import systolic as osys
@@ -671,3 +671,22 @@ def test_rows_of_a_far_apart(cuda, M, K, ld):
     lay = _lib.SystolicLayout(ld_a=ld, ld_xa=M, ld_b=N, ld_xb=N, ld_c=N)
     systolic_batched((far, X, B, XB), lay, 1, K, M, N, C, matmul.MXGEMMINI(), HW_FINAL)
     assert_bits_equal(C.cpu().numpy(), matmul.systolic(P, X, B, XB, matmul.MXGEMMINI(), HW_FINAL).cpu().numpy())
+
+
+@pytest.mark.parametrize("M,N", [(4096, 4096), (4033, 4001)])
+@pytest.mark.parametrize("K", [32, 96, 100, 224, 230, 1056])
+@pytest.mark.parametrize("name", ["hw_final", "e4m4", "e5m6", "mxquant_hw"])
+def test_tiles64_whose_last_stage_is_part_full(cuda, name, K, M, N):
+    """64 x 64 tiles over K that ends in the first block of a 64-row stage, in the second, or inside one, with an
+    outlier in the last row, against the general kernel."""
+    from mxq import matmul
+    ar_args, ladder, size = SMALL_LADDERS[name]
+    ar = getattr(matmul, ar_args[0])(*ar_args[1:])
+    assert systolic_plan(K, M, N, ar, ladder, size)[:3] == ("tile", 64, 64)
+    rng = np.random.default_rng(K + M)
+    ops = [torch.from_numpy(np.ascontiguousarray(x)).cuda()
+           for x in (*_codes(rng, K, M, mode="rne"), *_codes(rng, K, N, scale=0.02))]
+    ops[0][K - 1, 70] = 300.0
+    got = matmul.systolic(*ops, ar, ladder, size)
+    want = matmul.systolic(*ops, ar, ladder, size, force_general=True)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
