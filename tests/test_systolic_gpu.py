@@ -690,3 +690,36 @@ def test_tiles64_whose_last_stage_is_part_full(cuda, name, K, M, N):
     got = matmul.systolic(*ops, ar, ladder, size)
     want = matmul.systolic(*ops, ar, ladder, size, force_general=True)
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+FAST_TILES = {"64x64": (2050, 2047), "32x64": (1020, 2049), "32x32": (500, 2050)}
+
+
+@pytest.mark.parametrize("tile", FAST_TILES)
+@pytest.mark.parametrize("name,block", [(n, b) for n in ("hw_final", "e4m4", "e4m5_bf16_8", "e4m9_4") for b in (16, 48, 64, 96)]
+                         + [("e4m6_32", 64), ("e4m6_32", 96)])
+def test_other_blocks_on_the_register_staged_kernel(cuda, name, block, tile):
+    """Blocks of other sizes than 32 on k_systolic_fast's three tiles, whose operands end inside a tile, a stage and a
+    block: scales that leave the short tile add's range (one of them large, ahead of blocks inside it), a tile of zeros
+    and codes past the fast bound, against the general kernel."""
+    from mxq import matmul
+    _, ladder, size = {**SMALL_LADDERS, "e4m6_32": (None, [(4, 6)] * 32, 32)}[name]
+    (M, N), K = FAST_TILES[tile], 330
+    assert systolic_plan(K, M, N, matmul.MXGEMMINI(), ladder, size, block)[:3] == ("fast", *map(int, tile.split("x")))
+    g = torch.Generator(device="cuda").manual_seed(M + block)
+    P = [torch.randn(K, n, generator=g, device="cuda").mul_(s).to(torch.float8_e4m3fn).float() for n, s in ((M, 1.0), (N, 0.5))]
+    X = [torch.exp2(torch.randint(-3, 3, (-(-K // block), n), generator=g, device="cuda").float()) for n in (M, N)]
+    for x in X:
+        n = x.shape[1]
+        x[1, : n // 2] = 2.0 ** 46
+        x[1, n // 2] = 2.0 ** 63
+        x[2, 1::5] = 1e-38
+        x[3, ::7] = 0.0
+        x[3, 1::7] = 2.0 ** -60
+    P[0][:, 64:192] = 0.0
+    P[0][K // 2, M - 3] = 300.0
+    ops = (P[0], X[0], P[1], X[1])
+    got = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder, size, block)
+    want = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder, size, block, force_general=True)
+    same = (got.view(torch.int32) == want.view(torch.int32)) | (got.isnan() & want.isnan())
+    assert bool(same.all())
