@@ -989,29 +989,36 @@ struct Plan {
   int bm, bn;              // the tile kernels' tile
 };
 
-// What a launch takes: `fill` and a `round` for every 256 workgroups (one a CU) begun, at least `alone`, which that many
-// of one wave a SIMD take; `start` whatever K is.  Microseconds, measured under HW_FINAL at K = 2048 over 8 x 256 to
-// 1024 x 4096 outputs, and at K = 128 to 704 for `start`; all but `start` are proportional to K.  `fixed` is the part of
-// a workgroup's time that does not grow with the datapath's instructions (from the same on MXQUANT).
+// What a launch takes, in microseconds: `start`, `each` for every 256 workgroups (one a CU) begun, and for every 2048
+// rows of K `fill` and a `round` for every 256 workgroups, at least `alone`, which that many of one wave a SIMD take; the
+// last three times `cost`, a datapath's (by LaneKind; 0: no such instance).  K counts rounded up to what a workgroup
+// takes at once: a block of a tile kernel, or a small kernel's round of one reduction for every wave and group of columns
+// (up to 1024 rows: 128 x 2048 outputs of K = 64 take 4-row tiles of 16 columns 117 us, tiles of 32 x 32 12).
+// Fitted to every kernel's time on 12 shapes of 16 x 4096 to 2048 x 4096 outputs at K = 32 to 2048, under HW_FINAL
+// (within 3 to 5 % each), `cost` under the other datapaths.  On average the shape chosen takes 0.1 to 3 % longer than the
+// fastest, 17 % at the worst of 455.
 struct Shape {
   Plan::Kernel kernel;
   int rows, log_cols, waves;
-  double fill, round, alone, start, fixed;
+  double start, each, fill, round, alone;
+  double cost[6];
 };
 constexpr Shape kShapes[] = {
-    {Plan::kTile, 64, 6, 8, 35, 237, 275, 14, 0.0},    // 256 x 4096: 280, 512 x 4096: 508, 333 x 5632: 733
-    {Plan::kTile, 32, 5, 4, 24, 66, 172, 12, 0.1},     // 64 x 4096: 170, 256 x 2048: 180, 333 x 5632: 519
-    {Plan::kSmall, 16, 6, 8, 28, 74, 103, 20, 0.23},   // 128 x 4096: 174, 192 x 4096: 252, 512 x 2048: 324
-    {Plan::kSmall, 8, 6, 8, 14, 45, 66, 12, 0.38},     // 64 x 4096: 104, 320 x 2048: 241
-    {Plan::kSmall, 8, 6, 16, 0, 54, 53, 20, 0.38},     // 32 x 4096: 59, 64 x 4096: 111
-    {Plan::kSmall, 8, 5, 16, 1, 33, 33, 8, 0.48},      // 16 x 4096: 36
-    {Plan::kSmall, 8, 5, 8, 8, 29, 40, 8, 0.48},       // (the ladders without the sixteen-wave tiles)
-    {Plan::kSmall, 4, 6, 16, 2, 36, 37, 8, 0.57},      // 16 x 4096: 39
-    {Plan::kSmall, 4, 5, 16, 1, 22, 23, 8, 0.57},      // 32 x 1024: 24
-    {Plan::kSmall, 4, 4, 16, 5, 15, 18, 8, 0.57},      // 32 x 1024: 31
+    // (HW_FINAL: 512 x 2048 outputs at K = 32 and 2048, then 200 x 2048)
+    {Plan::kTile, 64, 6, 8, 5.1, 2.3, 71, 206, 279, {1, 1.35, 1.40, 2.39, 2.10, 2.10}},     // 13, 282; 12, 293
+    {Plan::kTile, 32, 5, 4, 6.0, 0.7, 76, 52, 164, {1, 1.32, 1.36, 2.24, 1.96, 1.96}},      // 14, 286; 10, 181
+    {Plan::kSmall, 16, 6, 8, 2.2, 1.3, 27, 71, 109, {1, 0, 0, 2.00, 0, 0}},                 // 28, 322; 15, 160
+    {Plan::kSmall, 8, 6, 8, 2.4, 1.1, 16, 42, 66, {1, 1.28, 1.28, 1.83, 1.70, 1.70}},       // 34, 369; 19, 183
+    {Plan::kSmall, 8, 6, 16, 1.7, 2.7, 4, 50, 0, {1, 0, 0, 1.86, 0, 0}},                    // 74, 422; 38, 205
+    {Plan::kSmall, 8, 5, 16, 1.8, 1.4, 1, 31, 33, {1, 0, 0, 1.70, 0, 0}},                   // 147, 514; 66, 214
+    {Plan::kSmall, 8, 5, 8, 2.2, 0.8, 7, 24, 40, {1, 1.30, 1.29, 1.73, 1.69, 1.69}},        // 64, 419; 30, 176
+    {Plan::kSmall, 4, 6, 16, 1.8, 2.7, 1, 32, 35, {1, 1.18, 1.22, 1.63, 1.58, 1.58}},       // 114, 561; 50, 241
+    {Plan::kSmall, 4, 5, 16, 2.0, 2.1, 0, 19, 40, {1, 1.16, 1.21, 1.53, 1.51, 1.51}},       // 225, 651; 92, 266
+    {Plan::kSmall, 4, 4, 16, 0.0, 0.0, 5, 15, 64, {1, 1.08, 1.13, 1.33, 1.30, 1.30}},       // 465, 987; 183, 384
+    {Plan::kFast, 64, 6, 4, 5.1, 2.0, 179, 198, 528, {1, 1.23, 0, 0, 0, 0}},                // 16, 567; 16, 548
+    {Plan::kFast, 32, 6, 4, 5.7, 1.2, 119, 101, 301, {1, 1.26, 0, 0, 0, 0}},                // 13, 326; 12, 320
+    {Plan::kFast, 32, 5, 4, 6.0, 0.8, 101, 51, 185, {1, 1.34, 0, 0, 0, 0}},                 // 14, 299; 11, 200
 };
-// A MAC's cost on the tile kernels by datapath (512 x 4096 outputs), HW_FINAL's being 1.
-constexpr double kMacCost[] = {1.0, 1.29, 1.36, 2.27, 2.3, 2.02};
 
 Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
   // hints that leave rows of A unread (a_live) or outputs unstored (c_end) need a tile kernel, whose own limits are
@@ -1034,30 +1041,36 @@ Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
   }
   double best = 0.0;
   for (const Shape& sh : kShapes) {
-    const bool tile = sh.kernel == Plan::kTile;
-    if (tile ? !tile_ok : !small_fits(sh.rows, sh.waves)) continue;
-    if (!tile && !every_small && !(sh.rows == 4 || (sh.rows == 8 && sh.waves == 8))) continue;
-    const int64_t n = mxq::ceil_div(a.M, sh.rows) * mxq::ceil_div(a.N, int64_t(1) << sh.log_cols) * count;
-    double t = std::max(sh.alone, sh.fill + sh.round * (double)mxq::ceil_div(n, 256));
-    t *= (sh.fixed + (1.0 - sh.fixed) * kMacCost[kind]) * (double)a.K / 2048.0;
-    if (tile && a.k_end) t *= 0.6;                    // a causal mask's half, and the uneven rest of it
-    t += sh.start;
-    if (tile && (a.skip || a.k_end)) t += 20.0;       // the dispatch order's and the suffix check's launches
+    const bool small = sh.kernel == Plan::kSmall;
+    if (sh.cost[kind] == 0.0 || (small && !small_fits(sh.rows, sh.waves))) continue;
+    if (sh.kernel == Plan::kTile && !tile_ok) continue;
+    // k_systolic_fast takes what k_systolic_tile does not, and the ladders whose constants are no literals, some of
+    // which it runs faster (e4m4 lanes, 2048 x 4096 outputs of K = 200: 245 us on 64 x 64 tiles, 282)
+    if (sh.kernel == Plan::kFast && tile_ok && kind != kE4) continue;
+    // Per ladder: shorter reductions pay a small kernel's LDS round trip and tile add more often, 32 lanes' constants
+    // spill; and k_systolic_fast's ragged rows go a float at a time.
+    double cost = sh.cost[kind];
+    if (small) cost *= a.size == 4 ? (sh.rows == 4 ? 1.7 : 1.25) : a.size == 8 ? (sh.rows == 4 ? 1.2 : 1.05) : a.size == 32 ? 1.08 : 1.0;
+    else if (a.size == 32) cost *= sh.kernel == Plan::kTile && sh.rows == 32 ? 1.13 : 1.07;
+    else if (sh.kernel == Plan::kTile) cost *= a.size < 16 ? 0.97 : 1.0;
+    else cost *= a.size == 4 ? 1.1 : a.size == 8 ? 0.93 : 1.0;
+    if (sh.kernel == Plan::kFast && (a.M % 4 != 0 || a.N % 4 != 0)) cost *= 1.1;
+    // (one wave a SIMD waits as long as it issues: a datapath's longer code costs it less)
+    const double alone = sh.alone * (small ? cost : 1.0 + 0.45 * (cost - 1.0));
+    const int64_t wgs = mxq::ceil_div(a.M, sh.rows) * mxq::ceil_div(a.N, int64_t(1) << sh.log_cols) * count;
+    const double n = (double)mxq::ceil_div(wgs, 256);
+    const int64_t at_once = small ? (int64_t)sh.waves * (64 >> sh.log_cols) * a.size : KT;
+    double t = std::max(alone, cost * (sh.fill + sh.round * n)) * (double)(mxq::ceil_div(a.K, at_once) * at_once) / 2048.0;
+    if (!small && a.k_end) t *= 0.6;                  // a causal mask's half, and the uneven rest of it
+    t += sh.start + sh.each * n;
+    if (!small && (a.skip || a.k_end)) t += 20.0;     // the dispatch order's and the suffix check's launches
     if (p.kernel == Plan::kGeneral || t < best) {
       best = t;
       p.kernel = sh.kernel;
       p.small = {sh.rows, sh.log_cols, sh.waves};
-      p.bm = p.bn = sh.rows;
+      p.bm = sh.rows;
+      p.bn = 1 << sh.log_cols;
     }
-  }
-  // e4 lanes with other blocks than 32 (or wider rows): k_systolic_fast while it has a workgroup for every CU
-  if (!tile_ok && kind <= kE4 &&
-      (p.kernel == Plan::kGeneral || (a.M > 16 && mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= 256))) {
-    // its tiles: 64 x 64, 32 x 64 or 32 x 32 outputs, the largest that gives every CU four workgroups
-    const int64_t want = 4 * 256;
-    p.kernel = Plan::kFast;
-    p.bm = mxq::ceil_div(a.M, 64) * mxq::ceil_div(a.N, 64) * count >= want ? 64 : 32;
-    p.bn = p.bm == 64 || mxq::ceil_div(a.M, 32) * mxq::ceil_div(a.N, 64) * count >= want ? 64 : 32;
   }
   return p;
 }

@@ -28,3 +28,22 @@ def test_small_kernel_refuses_strides_its_offsets_cannot_hold(name, M, block):
             if kernel == "tile":
                 assert ld < 1 << 28 and block == 32
     assert _plan(name, 4096, M, 256, block_size=block)[0] == "small"     # (the shapes are the small kernel's)
+
+
+@pytest.mark.parametrize("name", LADDERS)
+@pytest.mark.parametrize("block", [32, 64])
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 256, 1024, 4096])
+def test_a_short_product_is_not_computed_for_padding(name, K, block):
+    """A small kernel's workgroup computes a whole round of reductions, one for every wave and group of columns, however
+    few K holds.  Where the outputs make more than a round of workgroups for the chip (256 CUs), the padded rows of K times
+    the rounds of workgroups stay under twice what the tiles would compute (of 64 x 64, rounded up the same way)."""
+    for M in (8, 16, 33, 64, 128, 200, 333, 512, 1024, 2048):
+        for N in (64, 512, 1000, 2048, 4096):
+            kernel, rows, cols, waves = _plan(name, K, M, N, block_size=block)
+            wgs = -(-M // rows) * -(-N // cols)
+            if kernel != "small" or wgs <= 256:
+                continue
+            at_once = waves * (64 // cols) * 16
+            work = -(-K // at_once) * at_once * wgs * rows * cols
+            assert work <= 2 * max(-(-K // 32) * 32, 128) * -(-M // 64) * -(-N // 64) * 4096, \
+                f"{M} x {N}, K = {K}: {wgs} workgroups of {rows} x {cols}, {waves} waves"
