@@ -994,9 +994,9 @@ struct Plan {
 // last three times `cost`, a datapath's (by LaneKind; 0: no such instance).  K counts rounded up to what a workgroup
 // takes at once: a block of a tile kernel, or a small kernel's round of one reduction for every wave and group of columns
 // (up to 1024 rows: 128 x 2048 outputs of K = 64 take 4-row tiles of 16 columns 117 us, tiles of 32 x 32 12).
-// Fitted to every kernel's time on 12 shapes of 16 x 4096 to 2048 x 4096 outputs at K = 32 to 2048, under HW_FINAL
-// (within 3 to 5 % each), `cost` under the other datapaths.  On average the shape chosen takes 0.1 to 3 % longer than the
-// fastest, 17 % at the worst of 455.
+// Fitted to every kernel's time on 39 shapes of 1 x 1000 to 2048 x 4096 outputs at K = 32 to 2048, under HW_FINAL
+// (within 3 to 8 % each), `cost` under the other datapaths.  On average the shape chosen takes 0.5 % longer than the
+// fastest, 18 % at the worst of 950.
 struct Shape {
   Plan::Kernel kernel;
   int rows, log_cols, waves;
@@ -1005,19 +1005,19 @@ struct Shape {
 };
 constexpr Shape kShapes[] = {
     // (HW_FINAL: 512 x 2048 outputs at K = 32 and 2048, then 200 x 2048)
-    {Plan::kTile, 64, 6, 8, 5.1, 2.3, 71, 206, 279, {1, 1.35, 1.40, 2.39, 2.10, 2.10}},     // 13, 282; 12, 293
-    {Plan::kTile, 32, 5, 4, 6.0, 0.7, 76, 52, 164, {1, 1.32, 1.36, 2.24, 1.96, 1.96}},      // 14, 286; 10, 181
-    {Plan::kSmall, 16, 6, 8, 2.2, 1.3, 27, 71, 109, {1, 0, 0, 2.00, 0, 0}},                 // 28, 322; 15, 160
-    {Plan::kSmall, 8, 6, 8, 2.4, 1.1, 16, 42, 66, {1, 1.28, 1.28, 1.83, 1.70, 1.70}},       // 34, 369; 19, 183
-    {Plan::kSmall, 8, 6, 16, 1.7, 2.7, 4, 50, 0, {1, 0, 0, 1.86, 0, 0}},                    // 74, 422; 38, 205
-    {Plan::kSmall, 8, 5, 16, 1.8, 1.4, 1, 31, 33, {1, 0, 0, 1.70, 0, 0}},                   // 147, 514; 66, 214
-    {Plan::kSmall, 8, 5, 8, 2.2, 0.8, 7, 24, 40, {1, 1.30, 1.29, 1.73, 1.69, 1.69}},        // 64, 419; 30, 176
-    {Plan::kSmall, 4, 6, 16, 1.8, 2.7, 1, 32, 35, {1, 1.18, 1.22, 1.63, 1.58, 1.58}},       // 114, 561; 50, 241
-    {Plan::kSmall, 4, 5, 16, 2.0, 2.1, 0, 19, 40, {1, 1.16, 1.21, 1.53, 1.51, 1.51}},       // 225, 651; 92, 266
-    {Plan::kSmall, 4, 4, 16, 0.0, 0.0, 5, 15, 64, {1, 1.08, 1.13, 1.33, 1.30, 1.30}},       // 465, 987; 183, 384
-    {Plan::kFast, 64, 6, 4, 5.1, 2.0, 179, 198, 528, {1, 1.23, 0, 0, 0, 0}},                // 16, 567; 16, 548
-    {Plan::kFast, 32, 6, 4, 5.7, 1.2, 119, 101, 301, {1, 1.26, 0, 0, 0, 0}},                // 13, 326; 12, 320
-    {Plan::kFast, 32, 5, 4, 6.0, 0.8, 101, 51, 185, {1, 1.34, 0, 0, 0, 0}},                 // 14, 299; 11, 200
+    {Plan::kTile, 64, 6, 8, 5.1, 2.2, 61, 215, 278, {1, 1.35, 1.40, 2.39, 2.10, 2.10}},    // 13, 282; 12, 293
+    {Plan::kTile, 32, 5, 4, 5.9, 0.6, 60, 55, 164, {1, 1.32, 1.36, 2.24, 1.96, 1.96}},     // 14, 286; 10, 181
+    {Plan::kSmall, 16, 6, 8, 2.4, 1.1, 22, 74, 105, {1, 0, 0, 2.00, 0, 0}},                // 28, 322; 15, 160
+    {Plan::kSmall, 8, 6, 8, 2.5, 1.1, 14, 43, 64, {1, 1.28, 1.28, 1.83, 1.70, 1.70}},      // 34, 369; 19, 183
+    {Plan::kSmall, 8, 6, 16, 1.9, 2.5, 0, 51, 0, {1, 0, 0, 1.86, 0, 0}},                   // 74, 422; 38, 205
+    {Plan::kSmall, 8, 5, 16, 2.1, 1.5, 0, 31, 0, {1, 0, 0, 1.70, 0, 0}},                   // 147, 514; 66, 214
+    {Plan::kSmall, 8, 5, 8, 2.5, 0.7, 5, 25, 37, {1, 1.30, 1.29, 1.73, 1.69, 1.69}},       // 64, 419; 30, 176
+    {Plan::kSmall, 4, 6, 16, 1.9, 2.6, 0, 33, 33, {1, 1.18, 1.22, 1.63, 1.58, 1.58}},      // 114, 561; 50, 241
+    {Plan::kSmall, 4, 5, 16, 1.9, 2.1, 0, 19, 0, {1, 1.16, 1.21, 1.53, 1.51, 1.51}},       // 225, 651; 92, 266
+    {Plan::kSmall, 4, 4, 16, 1.8, 0.0, 0, 15, 0, {1, 1.08, 1.13, 1.33, 1.30, 1.30}},       // 465, 987; 183, 384
+    {Plan::kFast, 64, 6, 4, 5.1, 1.9, 174, 203, 533, {1, 1.23, 0, 0, 0, 0}},               // 16, 567; 16, 548
+    {Plan::kFast, 32, 6, 4, 5.7, 1.1, 110, 106, 305, {1, 1.26, 0, 0, 0, 0}},               // 13, 326; 12, 320
+    {Plan::kFast, 32, 5, 4, 5.9, 0.8, 99, 52, 190, {1, 1.34, 0, 0, 0, 0}},                 // 14, 299; 11, 200
 };
 
 Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
@@ -1047,13 +1047,20 @@ Plan plan_launch(const SysArgs& a, int64_t count, int kind) {
     // k_systolic_fast takes what k_systolic_tile does not, and the ladders whose constants are no literals, some of
     // which it runs faster (e4m4 lanes, 2048 x 4096 outputs of K = 200: 245 us on 64 x 64 tiles, 282)
     if (sh.kernel == Plan::kFast && tile_ok && kind != kE4) continue;
-    // Per ladder: shorter reductions pay a small kernel's LDS round trip and tile add more often, 32 lanes' constants
-    // spill; and k_systolic_fast's ragged rows go a float at a time.
+    // A small kernel's last columns, where they are not a whole group, go by checked loads, and its workgroups there end
+    // last.  Per ladder: shorter reductions pay its LDS round trip and tile add more often, 32 lanes' constants spill; and
+    // k_systolic_fast's ragged rows go a float at a time.
     double cost = sh.cost[kind];
-    if (small) cost *= a.size == 4 ? (sh.rows == 4 ? 1.7 : 1.25) : a.size == 8 ? (sh.rows == 4 ? 1.2 : 1.05) : a.size == 32 ? 1.08 : 1.0;
-    else if (a.size == 32) cost *= sh.kernel == Plan::kTile && sh.rows == 32 ? 1.13 : 1.07;
-    else if (sh.kernel == Plan::kTile) cost *= a.size < 16 ? 0.97 : 1.0;
-    else cost *= a.size == 4 ? 1.1 : a.size == 8 ? 0.93 : 1.0;
+    if (small) {
+      cost *= a.size == 4 ? (sh.rows == 4 ? 1.7 : 1.25) : a.size == 8 ? (sh.rows == 4 ? 1.2 : 1.05) : a.size == 32 ? 1.08 : 1.0;
+      const bool whole = a.N % (int64_t(1) << sh.log_cols) == 0;
+      cost *= whole ? 0.97 : sh.log_cols == 6 ? 1.10 : sh.log_cols == 5 ? 1.05 : 1.02;
+      if (!whole && a.size == 32) cost *= 1.12;
+    } else if (a.size == 32) {
+      cost *= sh.kernel == Plan::kTile && sh.rows == 32 ? 1.13 : 1.07;
+    } else {
+      cost *= sh.kernel == Plan::kTile ? (a.size < 16 ? 0.97 : 1.0) : a.size == 4 ? 1.1 : a.size == 8 ? 0.93 : 1.0;
+    }
     if (sh.kernel == Plan::kFast && (a.M % 4 != 0 || a.N % 4 != 0)) cost *= 1.1;
     // (one wave a SIMD waits as long as it issues: a datapath's longer code costs it less)
     const double alone = sh.alone * (small ? cost : 1.0 + 0.45 * (cost - 1.0));

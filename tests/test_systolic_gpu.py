@@ -675,8 +675,9 @@ def test_rows_of_a_far_apart(cuda, M, K, ld):
 
 @pytest.mark.parametrize("M,N", [(512, 2048), (509, 2041)])
 @pytest.mark.parametrize("name,K", [(n, K) for n in ("hw_final", "e4m4", "e4m9_4", "e5m6", "e5m5_e7m10_32")
-                                    for K in (32, 96, 100, 224, 230, 1056)]
-                         + [(n, K) for n in ("mxquant_hw", "mxquant_e6m9") for K in (32, 96)])
+                                    for K in (32, 96, 100, 224, 230)]
+                         + [("hw_final", 1056), ("hw_final", 1130), ("e5m5_e7m10_32", 1056), ("mxquant_hw", 32),
+                            ("mxquant_e6m9", 32)])
 def test_tiles64_whose_last_stage_is_part_full(cuda, name, K, M, N):
     """64 x 64 tiles over K that ends in the first block of a 64-row stage, in the second, or inside one, with an
     outlier in the last row, against the general kernel."""
@@ -693,7 +694,7 @@ def test_tiles64_whose_last_stage_is_part_full(cuda, name, K, M, N):
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
 
 
-FAST_TILES = {"64x64": (8202, 4093), "32x64": (1018, 4091), "32x32": (500, 2050)}
+FAST_TILES = {"64x64": (330, 8202, 4093), "32x64": (298, 1386, 4091), "32x32": (330, 500, 2050)}   # K, M, N
 
 
 @pytest.mark.parametrize("tile", FAST_TILES)
@@ -705,7 +706,7 @@ def test_other_blocks_on_the_register_staged_kernel(cuda, name, block, tile):
     and codes past the fast bound, against the general kernel."""
     from mxq import matmul
     _, ladder, size = {**SMALL_LADDERS, "e4m6_32": (None, [(4, 6)] * 32, 32)}[name]
-    (M, N), K = FAST_TILES[tile], 330
+    K, M, N = FAST_TILES[tile]
     assert systolic_plan(K, M, N, matmul.MXGEMMINI(), ladder, size, block)[:3] == ("fast", *map(int, tile.split("x")))
     g = torch.Generator(device="cuda").manual_seed(M + block)
     P = [torch.randn(K, n, generator=g, device="cuda").mul_(s).to(torch.float8_e4m3fn).float() for n, s in ((M, 1.0), (N, 0.5))]

@@ -47,3 +47,18 @@ def test_a_short_product_is_not_computed_for_padding(name, K, block):
             work = -(-K // at_once) * at_once * wgs * rows * cols
             assert work <= 2 * max(-(-K // 32) * 32, 128) * -(-M // 64) * -(-N // 64) * 4096, \
                 f"{M} x {N}, K = {K}: {wgs} workgroups of {rows} x {cols}, {waves} waves"
+
+
+# HW_FINAL on MI355X: K, M, N -> the tiles (rows, columns) within a tenth of the fastest's time
+MEASURED = {(64, 4, 4096): [(8, 64), (8, 32)], (64, 333, 2048): [(32, 32)], (64, 512, 2048): [(64, 64), (32, 32)],
+            (512, 16, 1024): [(4, 32)], (512, 256, 512): [(8, 64), (8, 32)], (2048, 4, 512): [(4, 16)],
+            (2048, 4, 4096): [(4, 16), (4, 32)], (2048, 8, 4096): [(4, 32)], (2048, 16, 256): [(4, 16)],
+            (2048, 16, 1024): [(4, 16)], (2048, 16, 4096): [(8, 32), (4, 64)], (2048, 24, 2048): [(8, 32)],
+            (2048, 32, 4096): [(8, 64), (4, 64)], (2048, 128, 512): [(8, 32)], (2048, 64, 4096): [(8, 64), (8, 32)],
+            (2048, 128, 4096): [(16, 64), (32, 32)], (2048, 200, 2048): [(16, 64)], (2048, 512, 1000): [(32, 32)],
+            (2048, 333, 5632): [(32, 32)], (2048, 1024, 2048): [(64, 64)], (4096, 512, 4096): [(64, 64)]}
+
+
+@pytest.mark.parametrize("K,M,N", MEASURED, ids=str)
+def test_measured_choices(K, M, N):
+    assert _plan("hw_final", K, M, N)[1:3] in MEASURED[K, M, N]
