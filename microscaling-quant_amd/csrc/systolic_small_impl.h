@@ -10,7 +10,11 @@
 // while this one is computed.
 //
 // The arithmetic is the tile kernels' fast datapath (Datapath), under the same check of the operands read.  Where it
-// fails, the workgroup computes its outputs by the general rule itself: a call is one launch, without flags.
+// fails (after the first round of a long K, or at the end), the workgroup computes its outputs by the general rule itself:
+// a call is one launch, without flags.  Operands all past the check (E4M3 codes to 448 under HW_FINAL), a whole call
+// against the tile kernel's and the general kernel's after it: 1 x 4096 outputs, K = 4096: 0.22 ms against 7.9; 8 x 4096:
+// 1.0 against 10.0; 64 x 4096, K = 2048: 2.0 against 5.1; MXGEMMINI e5m6 lanes 512 x 2048, K = 2048: 13.0 against the
+// general kernel's 12.8, MXQUANT(4, 3): 3.2 against 3.0 (36 and 3.7 with each output's K in one thread).
 //
 // Bound by VALU issue (8.0 to 8.6 instructions a MAC, the datapath's 7 among them) and, for one row, by reading B.
 // HW_FINAL, a whole call against the tile kernel's: 1 x 5632 outputs, K = 2048: 23 us against 207 (45 MB of codes);
@@ -130,6 +134,29 @@ __global__ void __launch_bounds__(64 * NW, 4) k_systolic_small(const SysArgs arg
         x[u] = in ? t : 0.0f;
       }
     };
+    // the workgroup's verdict on what it has read, as the tile kernels'
+    auto verdict = [&]() __attribute__((always_inline)) {
+      for (int off = 32; off > 0; off >>= 1) {
+        max_a = umax(max_a, (uint32_t)__shfl_xor((int)max_a, off, 64));
+        max_b = umax(max_b, (uint32_t)__shfl_xor((int)max_b, off, 64));
+        max_x = umax(max_x, (uint32_t)__shfl_xor((int)max_x, off, 64));
+      }
+      if (lane == 0) {
+        red[0][wave] = max_a;
+        red[1][wave] = max_b;
+        red[2][wave] = max_x;
+      }
+      __syncthreads();
+      uint32_t wa = 0u, wb = 0u, wx = 0u;
+#pragma unroll
+      for (int v = 0; v < NW; ++v) {
+        wa = umax(wa, red[0][v]);
+        wb = umax(wb, red[1][v]);
+        wx = umax(wx, red[2][v]);
+      }
+      return wa < kFastAMaxBits && wb < 0x7F800000u && wx < 0x7F800000u && u2f(wa) * u2f(wb) <= args.fast_prod_max;
+    };
+    bool ok = true;
     load_a(0);
     load_b(0, b, xb);
     __syncthreads();                                // large_w cleared
@@ -215,6 +242,9 @@ __global__ void __launch_bounds__(64 * NW, 4) k_systolic_small(const SysArgs arg
           }
         }
       }
+      // operands past the datapath are so in their first rows as a rule: the rest of a long K is left to the general rule
+      // (not by the four-row tiles, whose loop takes 2 to 4 % longer with it; the others' does not)
+      if (TM != 4 && r0 == 0 && nred > 4 * round && !(ok = verdict())) break;
       if (more) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -225,44 +255,65 @@ __global__ void __launch_bounds__(64 * NW, 4) k_systolic_small(const SysArgs arg
       }
       buf ^= 1;                                     // the next round's tiles are written two barriers from here
     }
-    // the workgroup's verdict, as the tile kernels'
-    for (int off = 32; off > 0; off >>= 1) {
-      max_a = umax(max_a, (uint32_t)__shfl_xor((int)max_a, off, 64));
-      max_b = umax(max_b, (uint32_t)__shfl_xor((int)max_b, off, 64));
-      max_x = umax(max_x, (uint32_t)__shfl_xor((int)max_x, off, 64));
-    }
-    if (lane == 0) {
-      red[0][wave] = max_a;
-      red[1][wave] = max_b;
-      red[2][wave] = max_x;
-    }
-    __syncthreads();
-    uint32_t wa = 0u, wb = 0u, wx = 0u;
+    if (ok) ok = verdict();
+    if (!ok) {
+      // Any codes and scales: the general rule, the reductions shared among the waves as above.  B is read again (the
+      // next row's value while a row is computed), A through LDS.  Its loads are its own and its rows are taken one after
+      // another: with the loads above and the rows interleaved it is 5 to 15 % faster, and the registers that takes cost
+      // the datapath above 1 to 5 % (as it is, from -3 to 3 % by ladder, none on average).
 #pragma unroll
-    for (int v = 0; v < NW; ++v) {
-      wa = umax(wa, red[0][v]);
-      wb = umax(wb, red[1][v]);
-      wx = umax(wx, red[2][v]);
-    }
-    const bool ok = wa < kFastAMaxBits && wb < 0x7F800000u && wx < 0x7F800000u && u2f(wa) * u2f(wb) <= args.fast_prod_max;
-    if (!ok && owner) {
-      // any codes and scales: the general rule, step by step
-#pragma unroll
-      for (int j = 0; j < PER; ++j) {
-        const int mm = om + j * (NT >> log_cw);
-        if (mm >= rows_in || n0 + oc >= N) continue;
-        float c = 0.0f;
-        for (int r = 0; r < nred; ++r) {
-          float S = 0.0f;
-          for (int i = 0; i < SIZE && r * SIZE + i < K; ++i) {
-            const int64_t k = r * SIZE + i;
-            S = gen_acc(S, gen_product(A[k * args.A.ld + mm], B[k * args.B.ld + oc], args.ar), args.lane_e[i],
-                        args.lane_m[i], args.ar);
-          }
-          const int64_t g = mxq::divu31(r, per_block);
-          c = gen_tile(c, S * (XA[g * args.XA.ld + mm] * XB[g * args.XB.ld + oc]), args.ar);
+      for (int j = 0; j < PER; ++j) C[j] = 0.0f;
+#pragma unroll 1
+      for (int r0 = 0; r0 < nred; r0 += round) {
+        __syncthreads();                            // the tiles before are added, A's rows before used
+#pragma unroll 1
+        for (int e = threadIdx.x; e < round * SIZE * TM; e += NT) {
+          const int row = e / TM, x = e % TM;
+          const bool in = x < rows_in && r0 * SIZE + row < K;
+          const float v = A[in ? (int64_t)(r0 * SIZE + row) * args.A.ld + x : 0];
+          sa[row / SIZE * APAD + row % SIZE * TM + x] = in ? v : 0.0f;
         }
-        C[j] = c;
+#pragma unroll 1
+        for (int e = threadIdx.x; e < round * TM; e += NT) {
+          const int r = r0 + e / TM, x = e % TM;
+          const bool in = x < rows_in && r < nred;
+          const float v = XA[(in ? mxq::divu31(r, per_block) : 0u) * args.XA.ld + (in ? x : 0)];
+          xs[e] = in ? v : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int u = 0; u < U; ++u) {
+          const int slot = (wave * U + u) * subs + sub, r = r0 + slot, k0 = r * SIZE;
+          const float* as = &sa[slot * APAD];
+          auto b_at = [&](int k) { return B[(k < K && col_in ? (int64_t)k * args.B.ld + col : 0)]; };
+          float S[TM];
+#pragma unroll
+          for (int x = 0; x < TM; ++x) S[x] = 0.0f;
+          float next = b_at(k0);
+#pragma unroll 1
+          for (int i = 0; i < SIZE; ++i) {
+            const float v = next;
+            next = b_at(k0 + i + 1);
+            if (k0 + i >= K) break;                 // a reduction cut short by K's end ends as it stands
+#pragma unroll
+            for (int x = 0; x < TM; ++x) {
+              asm volatile("" : "+v"(S[x]));        // this row after the one before
+              S[x] = gen_acc(S[x], gen_product(as[i * TM + x], v, args.ar), args.lane_e[i], args.lane_m[i], args.ar);
+            }
+          }
+          const bool in = r < nred && col_in;
+          const float x_b = XB[(in ? mxq::divu31(r, per_block) : 0u) * args.XB.ld + (in ? col : 0)];
+#pragma unroll
+          for (int x = 0; x < TM; ++x) tiles[0][slot * TM * cw + col + x * cw] = S[x] * (xs[slot * TM + x] * x_b);
+        }
+        __syncthreads();
+        const int cnt = nred - r0 < round ? nred - r0 : round;
+        if (owner) {
+#pragma unroll
+          for (int j = 0; j < PER; ++j)
+#pragma unroll 1
+            for (int s = 0; s < cnt; ++s) C[j] = gen_tile(C[j], tiles[0][threadIdx.x + j * NT + s * TM * cw], args.ar);
+        }
       }
     }
   }

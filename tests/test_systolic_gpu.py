@@ -725,3 +725,46 @@ def test_other_blocks_on_the_register_staged_kernel(cuda, name, block, tile):
     want = matmul.systolic(*ops, matmul.MXGEMMINI(), ladder, size, block, force_general=True)
     same = (got.view(torch.int32) == want.view(torch.int32)) | (got.isnan() & want.isnan())
     assert bool(same.all())
+
+
+# every tile of k_systolic_small (rows, columns, waves); the first shape below that the launch rule gives it
+SMALL_TILES = {"hw_final": [(1, 16, 16), (1, 32, 16), (1, 64, 16), (4, 16, 16), (4, 32, 16), (4, 64, 16), (8, 32, 8),
+                            (8, 32, 16), (8, 64, 8), (8, 64, 16), (16, 64, 8)],
+               "mxquant_hw": [(1, 16, 16), (1, 64, 16), (4, 32, 16), (8, 32, 16), (8, 64, 8), (16, 64, 8)]}
+OTHER_TILES = [(4, 16, 16), (4, 32, 16), (4, 64, 16), (8, 32, 8), (8, 64, 8)]
+SMALL_SHAPES = [(316, 1, 17), (700, 1, 5001), (500, 1, 20001), (1100, 3, 515), (2070, 8, 130), (515, 2, 17),
+                (1030, 13, 1030), (300, 33, 515), (400, 70, 515), (537, 9, 2895), (300, 17, 2771), (323, 552, 33),
+                (333, 520, 102), (545, 589, 97), (309, 36, 3326), (365, 336, 1164), (130, 70, 1030), (250, 100, 2060),
+                (450, 100, 515), (200, 260, 700), (1500, 40, 1300), (330, 11, 4099), (2500, 40, 1300), (90, 130, 515),
+                (1200, 90, 2060), (100, 33, 1100), (90, 60, 4099), (600, 60, 2571), (2100, 12, 2060)]
+
+
+@pytest.mark.parametrize("name,tile", [(n, t) for n in SMALL_LADDERS for t in SMALL_TILES.get(n, OTHER_TILES)], ids=str)
+def test_every_tile_of_few_outputs(cuda, name, tile):
+    """Each tile of the kernel for few outputs, at shapes whose rows, columns, rounds and reductions are cut short, with
+    operands inside its datapath, all of them outside (refused after the first round or at the end), and a few outside
+    (an outlier in the last row, an Inf, a NaN, large and tiny scales), against the general kernel (checked against the
+    oracle above)."""
+    from mxq import matmul
+    ar_args, ladder, size = SMALL_LADDERS[name]
+    ar = getattr(matmul, ar_args[0])(*ar_args[1:])
+    cut = size if name == "mxquant_falling_8" else 1      # (the lanes of a cut reduction are the general kernel's)
+    shapes = [(K // cut * cut, M, N) for K, M, N in SMALL_SHAPES]
+    shapes = [s for s in shapes if systolic_plan(*s, ar, ladder, size) == ("small", *tile)]
+    assert shapes, f"no shape reaches the tile {tile}"
+    K, M, N = min(shapes, key=lambda s: s[0] * s[1] * s[2])
+    rng = np.random.default_rng(K + M + N)
+    inside = [*_codes(rng, K, M, mode="rne"), *_codes(rng, K, N, scale=0.02)]
+    outside = [*ob.ocp_quantize(rng.standard_normal((K, M)).astype(np.float32), "MXFP8_E4M3", 0),
+               *ob.ocp_quantize(rng.standard_normal((K, N)).astype(np.float32), "MXFP8_E4M3", 0)]
+    some = [x.copy() for x in inside]
+    some[0][K - 1, M - 1] = 30000.0
+    some[2][K // 3, N // 2] = np.inf
+    some[2][K // 2, N // 4] = np.nan
+    some[3][1, : N // 5] = np.float32(2.0 ** 70)
+    some[3][2, N // 3:] = np.float32(3e-39)
+    for what, ops in (("inside", inside), ("outside", outside), ("some outside", some)):
+        ops = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in ops]
+        got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
+        want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
+        assert_bits_equal(got, want, f"{what}: {M}x{N}, K={K}")
