@@ -765,19 +765,24 @@ __global__ void __launch_bounds__((BM / TM) * (BN / TN), 4) k_systolic_gen(const
   gen_tile_at<BM, BN, TM, TN>(args, blockIdx.z, (int64_t)blockIdx.y * BM, (int64_t)blockIdx.x * BN, args.K, sm);
 }
 
-// After a fast kernel, the tiles it flagged: workgroup g reads the flags of tiles [g * per, (g + 1) * per) of
-// the `total` (in the flags' order), 256 at a time, lists the set ones in LDS and recomputes each in BM x BN
-// pieces.  At most 1024 workgroups, so a launch whose tiles are all exact (the usual case) costs the loads of
-// the flags, not a workgroup per tile that exits at once (9 us for the 32768 tiles of one attention product).
+// After a fast kernel, the tiles it flagged, recomputed in BM x BN pieces, `pieces` a tile: workgroup g takes piece
+// g % pieces of the set tiles among [g / pieces * per, ...) of the `total` (in the flags' order), 256 flags read at a
+// time and the set ones listed in LDS.  At most 1024 workgroups, so a launch whose tiles are all exact (the usual case)
+// costs the loads of the flags, not a workgroup per tile that exits at once (9 us for the 32768 tiles of one attention
+// product).  A workgroup a piece and not a tile: with 64 x 64 tiles all refused, 512 x 2048 outputs of e4m4 lanes, K =
+// 2048, took 20.6 ms on 256 workgroups (7.5 on 1024), 512 x 4096 of HW_FINAL, K =
+// 4096, 43 (29).
 template <int BM, int BN, int TM, int TN>
 __global__ void __launch_bounds__((BM / TM) * (BN / TN), 4) k_systolic_gen_flagged(const SysArgs args, int64_t total,
-                                                                                  int64_t per) {
+                                                                                  int64_t per, uint32_t pieces) {
   static_assert(32 % BM == 0 && 32 % BN == 0, "a general tile lies inside one fast tile");
   static_assert((BM / TM) * (BN / TN) == 256, "a flag per thread");
   __shared__ Smem<BM, BN> sm;
   __shared__ uint32_t list[256];
   __shared__ uint32_t nl;
-  const int64_t t0 = (int64_t)blockIdx.x * per, t1 = t0 + per < total ? t0 + per : total;
+  const uint32_t share = blockIdx.x / pieces, piece = blockIdx.x - share * pieces;
+  const uint32_t across = (uint32_t)args.fbn / BN, pm = piece / across * BM, pn = piece % across * BN;
+  const int64_t t0 = (int64_t)share * per, t1 = t0 + per < total ? t0 + per : total;
   for (int64_t c0 = t0; c0 < t1; c0 += 256) {
     if (threadIdx.x == 0) nl = 0u;
     __syncthreads();
@@ -791,11 +796,11 @@ __global__ void __launch_bounds__((BM / TM) * (BN / TN), 4) k_systolic_gen_flagg
       const int64_t zy = tt / args.tiles_x, tx = tt - zy * args.tiles_x;
       const int64_t z = zy / args.tiles_y, ty = zy - z * args.tiles_y;
       const int64_t tm0 = ty * args.fbm, tn0 = tx * args.fbn;
-      for (int64_t m0 = tm0; m0 < tm0 + args.fbm && m0 < args.M; m0 += BM)
-        for (int64_t n0 = tn0; n0 < tn0 + args.fbn && n0 < args.N; n0 += BN) {
-          gen_tile_at<BM, BN, TM, TN>(args, z, m0, n0, piece_kstop(args, flag, z, m0, n0, tm0, tn0), sm);
-          __syncthreads();   // the next piece restages sm
-        }
+      const int64_t m0 = tm0 + pm, n0 = tn0 + pn;
+      if (m0 < args.M && n0 < args.N) {
+        gen_tile_at<BM, BN, TM, TN>(args, z, m0, n0, piece_kstop(args, flag, z, m0, n0, tm0, tn0), sm);
+        __syncthreads();   // the next piece restages sm
+      }
     }
     __syncthreads();         // list and nl are rewritten for the next 256 flags
   }
@@ -1166,9 +1171,11 @@ int run_systolic(const SysArgs& base, const int32_t* lane_e, const int32_t* lane
     if (int rc = mxq::check_launch("mxq_systolic fast")) return rc;
     mxq::KernelTimer timer("systolic_general", st);
     const int64_t tiles = a.tiles_x * a.tiles_y * count;
-    const int64_t wgs = tiles < 1024 ? tiles : 1024;
-    if (wgs > 0)
-      k_systolic_gen_flagged<32, 32, 2, 2><<<(unsigned)wgs, 256, 0, st>>>(a, tiles, mxq::ceil_div(tiles, wgs));
+    const uint32_t pieces = (uint32_t)(a.fbm / 32 * (a.fbn / 32));
+    const int64_t shares = std::min(tiles, (int64_t)(1024 / pieces));
+    if (shares > 0)
+      k_systolic_gen_flagged<32, 32, 2, 2><<<(unsigned)(shares * pieces), 256, 0, st>>>(a, tiles, mxq::ceil_div(tiles, shares),
+                                                                                       pieces);
   } else {
     mxq::KernelTimer timer("systolic_general", st);
     k_systolic_gen<32, 32, 2, 2><<<grid_g, 256, 0, st>>>(a);
