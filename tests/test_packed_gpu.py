@@ -247,3 +247,24 @@ def test_quantize_packed_full_size_c3(c3_input, fmt):
         assert err == 0
         assert np.array_equal(codes[:, cols].cpu().numpy(), wc), f"{fmt} codes {cols}"
         assert np.array_equal(scales[:, cols].cpu().numpy(), ws), f"{fmt} scales {cols}"
+
+
+@pytest.mark.parametrize("shape,axis,bs", [((70, 2), 0, 32), ((3, 50, 2), 1, 6), ((64, 3), 1, 2), ((5, 2), 1, 3),
+                                           ((4097, 3), 0, 16), ((9, 31), 1, 3), ((1 << 30, 2), 0, 32)], ids=str)
+def test_dequantize_narrow_rows(cuda, shape, axis, bs):
+    """Rows of two and three columns and blocks under four elements, from bytes and from float32, and 2^31 elements (the
+    kernel of 64-bit indexes): against torch's repeat_interleave, the last piece of the large one."""
+    import mxq
+    g = torch.Generator(device="cuda").manual_seed(shape[0])
+    xs = list(shape)
+    xs[axis] = -(-shape[axis] // bs)
+    C = torch.randint(0, 120, shape, generator=g, device="cuda", dtype=torch.uint8)
+    S = torch.randint(100, 150, xs, generator=g, device="cuda", dtype=torch.uint8)
+    got = mxq.packed.dequantize(C, S, "MXFP8_E4M3", axis, bs)
+    if shape[0] > 1 << 20:
+        n = 1 << 16                                         # whole blocks
+        C, S, got = C[-n:].contiguous(), S[-n // bs:].contiguous(), got[-n:].contiguous()
+    P, X = mxq.packed.unpack(C, S, "MXFP8_E4M3", axis, bs)
+    want = P * X.repeat_interleave(bs, dim=axis).narrow(axis, 0, P.shape[axis])
+    assert torch.equal(got, want)
+    assert torch.equal(mxq.block.dequantize(P, X, axis=axis, block_size=bs), want)
