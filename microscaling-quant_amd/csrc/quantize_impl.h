@@ -420,14 +420,15 @@ __global__ void __launch_bounds__(256) k_quant_strided(const T* __restrict__ V, 
 //   * The R lanes of a column group hold the same maxima after the exchanges; lane r computes the scales of
 //     columns r, r + R, ... alone and the others read them (ceil(VEC / R) scale rule evaluations per lane
 //     instead of VEC).
-template <typename T, int ELEM, int MODE, int VEC, int R, typename SINK>
+// WHOLE: inner % VEC == 0 (the column's clamp, 64-bit work in every lane, costs 8192 x 8192 bfloat16 64 -> 67 us).
+template <typename T, int ELEM, int MODE, int VEC, int R, bool WHOLE, typename SINK>
 __global__ void __launch_bounds__(256) k_quant_split(const T* __restrict__ V, const SINK out, int64_t outer,
                                                      int64_t n, int64_t inner, mxq::DivU31 nb_div,
                                                      mxq::DivU31 wpr_div, mxq_block_spec s) {
   constexpr int CPW = 64 / R;          // column groups per wave
   constexpr int ROWS = 32 / R;         // rows per lane
   constexpr int PER = (VEC + R - 1) / R;  // scales each lane evaluates
-  const int64_t groups = (inner + VEC - 1) / VEC;
+  const int64_t groups = WHOLE ? inner / VEC : (inner + VEC - 1) / VEC;
   const int lane = threadIdx.x & 63;
   const int64_t nb = nb_div.d, waves_per_row = wpr_div.d;
   // the launch keeps the wave count below 2^31
@@ -442,7 +443,7 @@ __global__ void __launch_bounds__(256) k_quant_split(const T* __restrict__ V, co
   const int64_t cg = (int64_t)(wave - wr * wpr_div.d) * CPW + c;
   const bool live = cg < groups;
   // the last group ends on the last column, sharing some with the group before it (the same values stored twice)
-  const int64_t col = cg * VEC < inner - VEC ? cg * VEC : inner - VEC;
+  const int64_t col = WHOLE ? (live ? cg : 0) * VEC : (cg * VEC < inner - VEC ? cg * VEC : inner - VEC);
   const T* src = V + (o * n + k0 + r * ROWS) * inner + col;
 
   float v[ROWS][VEC];
@@ -1057,43 +1058,68 @@ int launch_quant(const T* V, const SINK& out, int64_t outer, int64_t n, int64_t 
     go(std::integral_constant<int, 1>{});
     return mxq::check_launch("mxq_block_quantize");
   }
-  const int vec = inner >= 4 ? 4 : (inner % 2 == 0 ? 2 : 1);
   if constexpr (SINK::kBytes == 1 && ELEM == MXQ_ELEM_OCP && MODE == MXQ_RNE) {
+    // narrow rows that are no whole eights leave k_pack_rne's eight columns a lane partly empty and its last group to
+    // overlapping accesses: 512 x 37 6.1 us, by k_quant_split 5.1; 131,072 x 12 10.6 and 9.9
     if (bs == 32 && q.via_e == 0 && out.e == q.e && out.m == q.m && mxq_ocp_hw::has_hw(q.e, q.m) &&
-        q.max_norm == mxq_ocp_hw::fmt_max(q.e, q.m) && inner >= 8)
+        q.max_norm == mxq_ocp_hw::fmt_max(q.e, q.m) && (inner % 8 == 0 || inner >= 64))
       return launch_pack_rne(V, out, outer, n, inner, nb, q, st);
   }
   if (bs == 32) {
-    // code bytes: eight columns a lane when there are as many (8-byte stores: a wave's eight lanes write 64 contiguous
-    // bytes of a row, the next wave the other half of the line; sixteen would keep 64 values a lane, which
-    // this layout's registers do not hold)
-    const int bvec = SINK::kBytes == 1 && inner >= 8 ? 8 : 0;
-    const int kvec = bvec ? bvec : vec;
-    // R = 8 lanes per block column (4 rows each) while that gives the chip at least 8 waves per SIMD; smaller
-    // tensors take R = 32 (one row per lane, four times the waves), which keeps more loads in flight (MI355X,
-    // block.ocp on 4096 x 512 float32: 12.2 us at R = 8, 9.7 us at R = 32; bf16 8192 x 8192: R = 8 fastest)
-    const int64_t groups = mxq::ceil_div(inner, kvec);
-    const int64_t waves8 = outer * nb * mxq::ceil_div(groups, 64 / 8);
-    auto go = [&](auto r_const) {
-      constexpr int R = decltype(r_const)::value;
-      const int64_t wpr = mxq::ceil_div(groups, 64 / R);
-      const dim3 grid = mxq::grid_for(outer * nb * wpr * 64, 256);
-      const mxq::DivU31 dnb = mxq::make_divu31((uint32_t)nb), dwpr = mxq::make_divu31((uint32_t)wpr);
-      if constexpr (SINK::kBytes == 1) {
-        if (bvec == 8) {
-          k_quant_split<T, ELEM, MODE, 8, R, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, dnb, dwpr, q);
-          return;
-        }
-      }
-      if (vec == 4) k_quant_split<T, ELEM, MODE, 4, R, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, dnb, dwpr, q);
-      else if (vec == 2) k_quant_split<T, ELEM, MODE, 2, R, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, dnb, dwpr, q);
-      else k_quant_split<T, ELEM, MODE, 1, R, SINK><<<grid, 256, 0, st>>>(V, out, outer, n, inner, dnb, dwpr, q);
+    // Columns a lane (VEC) and lanes a block column (R, 32 / R rows each), by the full waves that four columns at R = 8
+    // make.  Measured on inputs and outputs that leave the caches, float32 codes from float32 (bytes from bfloat16), us:
+    //                           VEC 4, R 8    4, 32    2, 32    1, 32
+    //   nearest even, by the conversions (the OCP grid; microxcaling's is alike)
+    //     4096 x 512                  6.3      7.7     11.5     24.9      (bytes 7.9, 10.5, 15.9, 21.9)
+    //     5632 x 333                  7.8     11.4     13.6     21.8      (8.6, 11.3, 14.8, 18.5)
+    //     4096 x 100, 400 waves       4.8      5.1      5.1      6.6      (6.7, 6.5, 7.0, 7.0)
+    //     512 x 37                    3.8      3.9      3.6      3.8      (5.8, 5.3, 5.2, 4.5)
+    //   software grids (mxquant; bytes: the OCP grid, ties away), whose four rows a lane take longer
+    //     4096 x 1536                13.2     21.3     32.3     74.8      (14.2, 24.0, 33.5, 52.5)
+    //     4096 x 512                  7.9      7.8     11.5     25.0      (8.9, 11.3, 14.4, 20.0)
+    //     1000 x 333                  6.7      4.9      4.9      6.0      (8.2, 6.3, 6.1, 6.5)
+    //     512 x 37                    5.5      3.8      3.5      3.8      (6.9, 5.2, 4.7, 4.2)
+    //   rows of eight columns and fewer, whose waves R = 8 leaves three quarters empty
+    //     262,144 x 7                 8.6      6.9      8.6     12.3      (14.4, 10.2, 12.1, 13.9)
+    // So R = 8 from 400 full waves with the conversions, from 2048 (bytes 1024) without, R = 32 for narrow rows, and
+    // single columns or pairs where four make few.  mxquant's bytes, all encoding, keep R = 32 (131,072 x 12: 66 us, 84 at
+    // R = 8).  Code bytes take eight columns (8-byte stores: a wave's eight lanes write 64 contiguous bytes of a row) once
+    // that fills the chip: 8192 x 8192 to bytes, ties away, 66 us, 75 with four.
+    constexpr bool BYTES = SINK::kBytes == 1;
+    constexpr bool HW = MODE == MXQ_RNE && (ELEM == MXQ_ELEM_OCP || ELEM == MXQ_ELEM_MICROSOFT);
+    auto go = [&](auto vec_const, auto r_const, auto whole_const) {
+      constexpr int VEC = decltype(vec_const)::value, R = decltype(r_const)::value;
+      const int64_t wpr = mxq::ceil_div(mxq::ceil_div(inner, VEC), 64 / R);
+      k_quant_split<T, ELEM, MODE, VEC, R, decltype(whole_const)::value, SINK>
+          <<<mxq::grid_for(outer * nb * wpr * 64, 256), 256, 0, st>>>(V, out, outer, n, inner, mxq::make_divu31((uint32_t)nb),
+                                                                      mxq::make_divu31((uint32_t)wpr), q);
     };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    using Four = std::integral_constant<int, 4>;
+    using Eight = std::integral_constant<int, 8>;
+    using Half = std::integral_constant<int, 32>;          // (half a wave to a block column)
     // the kernel indexes waves in 32 bits
-    if (outer * nb * mxq::ceil_div(groups, 64 / 32) >= (int64_t(1) << 31))
+    const int64_t widest = inner >= 4 ? (BYTES && inner >= 8 ? 8 : 4) : (inner % 2 == 0 ? 2 : 1);
+    if (outer * nb * mxq::ceil_div(mxq::ceil_div(inner, widest), 2) >= (int64_t(1) << 31))
       return mxq::invalid("block quantize: tensor too large (2^31 waves of 2048 elements)");
-    if (waves8 >= 8 * 1024) go(std::integral_constant<int, 8>{});
-    else go(std::integral_constant<int, 32>{});
+    const int64_t full = outer * nb * mxq::ceil_div(inner, 4) / 8;
+    constexpr bool ENCODE = BYTES && ELEM == MXQ_ELEM_QTORCH;
+    if (inner < 4) {
+      const bool many = outer * nb >= 8 * 1024;
+      if (inner % 2 == 0) many ? go(Two{}, Eight{}, std::true_type{}) : go(Two{}, Half{}, std::true_type{});
+      else many ? go(One{}, Eight{}, std::true_type{}) : go(One{}, Half{}, std::true_type{});
+    } else if (full < (ENCODE ? 64 : inner <= 8 ? 128 : HW && BYTES ? 400 : 200)) {
+      if constexpr (BYTES || ELEM == MXQ_ELEM_MICROSOFT) go(One{}, Half{}, std::true_type{});
+      else go(Two{}, Half{}, std::false_type{});
+    } else if (ENCODE || inner <= 8 || full < (HW ? 400 : BYTES ? 1024 : 2048)) {
+      go(Four{}, Half{}, std::false_type{});
+    } else if constexpr (!ENCODE) {
+      if (BYTES && inner >= 64 && outer * nb * mxq::ceil_div(inner, 8) / 8 >= 8 * 1024) {
+        if constexpr (BYTES) inner % 8 == 0 ? go(Eight{}, Eight{}, std::true_type{}) : go(Eight{}, Eight{}, std::false_type{});
+      } else if (inner % 4 == 0) go(Four{}, Eight{}, std::true_type{});
+      else go(Four{}, Eight{}, std::false_type{});
+    }
     return mxq::check_launch("mxq_block_quantize");
   }
   const int svec = inner % 4 == 0 ? 4 : (inner % 2 == 0 ? 2 : 1);

@@ -125,6 +125,23 @@ def test_quantize_packed_ragged_rows(cuda, method, opts, fmt):
             assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), f"{method} {fmt} {dtype} {shape} {axis}"
 
 
+@pytest.mark.parametrize("shape", [(64, 37), (1600, 36), (4096, 6), (65536, 7), (65536, 12), (4100, 130), (4130, 517),
+                                   (8200, 2055), (8192, 2056)], ids=str)
+@pytest.mark.parametrize("method,opts", [("mxgemmini", {}), ("mxgemmini", {"rounding_mode": "rne"}), ("ocp", {}),
+                                         ("mxquant", {})])
+def test_quantize_packed_every_split_of_columns(cuda, method, opts, shape):
+    """Blocks down the columns on both sides of each line of the rule that shares a block column's rows and columns among
+    lanes: the bytes against pack() of the float32 quantizer's outputs."""
+    import mxq
+    g = torch.Generator(device="cuda").manual_seed(shape[1])
+    V = (torch.randn(shape, generator=g, device="cuda") * 3).to(torch.bfloat16)
+    for fmt in ("MXFP8_E4M3", "MXFP6_E3M2"):
+        P, X = getattr(mxq.block, method).quantize(V, fmt, axis=0, **opts)
+        want = mxq.packed.pack(P, X, fmt, 0, check=False)
+        got = mxq.packed.quantize(V, fmt, method, 0, check=False, **opts)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), f"{method} {fmt} {shape}"
+
+
 def test_packed_specials_and_errors(cuda):
     """NaN codes: E4M3 and E5M2 have them, FP6 and FP4 raise; a non-power-of-two scale of a nonzero block
     raises; mxquant's smallest E4M3 qtorch values are no OCP E4M3 codes; check=False returns the bytes."""

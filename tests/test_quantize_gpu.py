@@ -213,6 +213,34 @@ def test_ragged_rows_at_any_address(cuda, method, dtype, fmt):
             assert_bits_equal(back.cpu().numpy(), ob.dequantize(*want, axis, bs), "read back " + at)
 
 
+@pytest.mark.parametrize("shape", [(64, 37), (1600, 36), (4096, 6), (65536, 7), (4096, 101), (4100, 130), (4130, 517),
+                                   (8192, 256), (8200, 1031)], ids=str)
+@pytest.mark.parametrize("method", ["mxgemmini", "mxgemmini rne", "ocp", "mxquant"])
+def test_every_split_of_columns(cuda, method, shape):
+    """Blocks down the columns, on both sides of each line of the rule that gives a lane one, two or four columns and a
+    block column 8 or 32 lanes, rows of whole fours and others: the outermost columns against the oracle, all of
+    them against a transposed input's (another kernel)."""
+    from mxq import block
+    rng = np.random.default_rng(shape[1])
+    V = (rng.standard_normal(shape) * np.exp2(rng.integers(-8, 8, (shape[0], 1)))).astype(np.float32)
+    V[5, 0] = V[-1, -1] = np.inf
+    name, _, mode = method.partition(" ")
+    kw = {"rounding_mode": mode} if mode else {}
+    q = getattr(block, name)
+    Vt = torch.from_numpy(V).cuda()
+    P, X = q.quantize(Vt, "MXFP8_E4M3", axis=0, **kw)
+    Pr, Xr = q.quantize(Vt.t().contiguous(), "MXFP8_E4M3", axis=1, **kw)
+    assert torch.equal(P.view(torch.int32), Pr.t().contiguous().view(torch.int32)), f"{method} {shape} P"
+    assert torch.equal(X.view(torch.int32), Xr.t().contiguous().view(torch.int32)), f"{method} {shape} X"
+    ends = np.concatenate([V[:, :5], V[:, -5:]], axis=1) if shape[1] >= 10 else V
+    Pe, Xe = (np.concatenate([a[:, :5], a[:, -5:]], axis=1) if shape[1] >= 10 else a for a in (P.cpu().numpy(), X.cpu().numpy()))
+    want = {"mxgemmini": lambda: ob.mxgemmini_quantize(ends, "MXFP8_E4M3", 0, 32, mode or "ties_away"),
+            "ocp": lambda: ob.ocp_quantize(ends, "MXFP8_E4M3", 0, 32),
+            "mxquant": lambda: ob.mxquant_quantize(ends, "MXFP8_E4M3", 0, 32)}[name]()
+    assert_bits_equal(Pe, want[0], f"{method} {shape} P")
+    assert_bits_equal(Xe, want[1], f"{method} {shape} X")
+
+
 # ------------------------------------------------------------------------------------------ elementwise
 @pytest.fixture(scope="module")
 def corpus():
