@@ -603,8 +603,24 @@ __global__ void __launch_bounds__(256) k_quant_row(const T* __restrict__ V, cons
   Div d[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) d[q] = make_div(Q == 1 ? own : __shfl(own, q, 8));
-  const bool div = s.scale_rule && wave_needs_div<Q>(d);
   constexpr bool HW = MODE == MXQ_RNE && (ELEM == MXQ_ELEM_OCP || ELEM == MXQ_ELEM_MICROSOFT);
+  if constexpr (WHOLE && !HW) {
+    // whole rows through a software grid: straight through, without the code for parts of a lane's four (to bytes, ties
+    // away, 8192 x 8192 half-precision values 84 us, 97 by the general code below)
+    static_assert(Q == 1, "a software grid takes one run a wave");
+    if (left[0] == 0) return;
+    float z[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) z[j] = s.scale_rule ? apply_div(v[0][j], d[0]) : v[0][j];
+    out.template elems<ELEM, MODE, 4>(off[0], z, s);
+    if (l8 == 0) {
+      const float x1[1] = {own};
+      const bool z1[1] = {am[0] == 0u};
+      out.template scales<1>(blk[0], x1, z1);
+    }
+    return;
+  }
+  const bool div = s.scale_rule && wave_needs_div<Q>(d);
   mxq_block_spec hs = s;
   bool hw = false;
   if constexpr (HW) {
