@@ -355,31 +355,25 @@ __device__ __forceinline__ bool fast_verdict(const TreeArgs& a, uint32_t max_a, 
   return ok;
 }
 
-// The block's scales of a thread's TM x TN outputs (zero outside C), with the largest |scale| bit pattern; returns
-// what scale_denies says of them.
+// The block's scales of a thread's TM x TN outputs (zero outside C), with the largest |scale| bit pattern.
 template <int TM, int TN>
-__device__ __forceinline__ uint32_t block_scales(const TreeArgs& a, int64_t g, int64_t mr, int64_t nc,
-                                                 float (&scale)[TM][TN], uint32_t& max_x, uint32_t xs_lo,
-                                                 uint32_t xs_hi) {
+__device__ __forceinline__ void block_scales(const TreeArgs& a, int64_t g, int64_t mr, int64_t nc,
+                                             float (&scale)[TM][TN], uint32_t& max_x) {
   float xa[TM], xb[TN];
-  uint32_t denies = 0u;
 #pragma unroll
   for (int x = 0; x < TM; ++x) {
     xa[x] = mr + x < a.M ? a.XA[g * a.M + mr + x] : 0.0f;
     max_x = umax(max_x, f2u(xa[x]) & 0x7FFFFFFFu);
-    denies |= scale_denies(xa[x], xs_lo, xs_hi);
   }
 #pragma unroll
   for (int y = 0; y < TN; ++y) {
     xb[y] = nc + y < a.N ? a.XB[g * a.N + nc + y] : 0.0f;
     max_x = umax(max_x, f2u(xb[y]) & 0x7FFFFFFFu);
-    denies |= scale_denies(xb[y], xs_lo, xs_hi);
   }
 #pragma unroll
   for (int x = 0; x < TM; ++x)
 #pragma unroll
     for (int y = 0; y < TN; ++y) scale[x][y] = xa[x] * xb[y];
-  return denies;
 }
 
 template <int TM, int TN>
@@ -414,14 +408,13 @@ struct FastLevels {
   uint32_t pmask;     // product truncation to prod_m fraction bits
   float flush_thr;    // bf16 first level: |product| below this becomes +0
   float prod_max;     // bound on max|a| * max|b|: no e4 level overflows, no product saturates
-  uint32_t xs_lo, xs_hi;   // scale magnitudes (bit patterns) that allow the short tile add
 };
 
 // BM = 64: 4 x 4 outputs per thread; BM = 32: 2 x 4, for problems with too few 64 x 64 tiles to fill the chip.
 // Bound by VALU issue: 16 products, 15 level sums and their roundings a reduction.  Each level's nearest even is
-// fma_rne with its power of two held in a VGPR (from an SGPR the fma issues at half rate), and a block whose scales
-// allow it (scale_denies) adds its tile with one fma and one rounding.  512 x 4096 outputs, K = 4096, levels e4m4,
-// e4m5, e4m6, bf16: 1.107 ms a call, 1.195 with the three-operation split and a separate product, sum and roundings.
+// fma_rne with its power of two held in a VGPR (from an SGPR the fma issues at half rate).  Levels e4m4, e4m5, e4m6,
+// bf16, 512 x 4096 outputs, K = 2048: 541 us, 595 with the three-operation split.  Adding a block's tile with one fma
+// and one rounding, where its scales allow that, costs more than it saves (553): the sums wait for the branch.
 template <int SIZE, int BM, bool FIRST_E4>
 __global__ void __launch_bounds__(256, BM == 32 ? 4 : SIZE == 32 ? 2 : 3) k_adder_fast(const TreeArgs args, const FastLevels fl) {
   constexpr int BN = FBN, TM = BM / 16, TN = 4, NT = 256, L = ilog2(SIZE);
@@ -464,8 +457,7 @@ __global__ void __launch_bounds__(256, BM == 32 ? 4 : SIZE == 32 ? 2 : 3) k_adde
   stage(0);
   __syncthreads();
   float scale[TM][TN];
-  bool short_add = false, large = false;            // this block's scales allow the short tile add; one was above
-  int in_block = 0;                                 // xs_hi (scale_denies)
+  int in_block = 0;
   int64_t g = 0;
   for (int64_t k0 = 0; k0 < K; k0 += KT) {
     const bool more = k0 + KT < K;
@@ -476,12 +468,7 @@ __global__ void __launch_bounds__(256, BM == 32 ? 4 : SIZE == 32 ? 2 : 3) k_adde
     const int kend = (int)((K - k0 < KT) ? (K - k0) : KT);
     // rows past K are zero in LDS: zero products, which is what the reference adds past a K tail
     for (int r0 = 0; r0 < kend; r0 += SIZE) {
-      if (in_block == 0) {
-        const uint32_t denies =
-            block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x, fl.xs_lo, fl.xs_hi);
-        large = large || __any((denies & 2u) != 0u) != 0;
-        short_add = __all(denies == 0u) != 0 && !large;
-      }
+      if (in_block == 0) block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x);
       float pend[L][TM][TN];
       float root[TM][TN];
 #pragma unroll
@@ -510,20 +497,13 @@ __global__ void __launch_bounds__(256, BM == 32 ? 4 : SIZE == 32 ? 2 : 3) k_adde
             if (carry) root[x][y] = v;
           }
       }
-      // the roots stand here: sunk into the branches below, the sums keep every operand of the reduction in registers
-      // until there (185 VGPRs instead of 123 at 2 x 4 outputs)
-#pragma unroll
-      for (int x = 0; x < TM; ++x)
-#pragma unroll
-        for (int y = 0; y < TN; ++y) asm volatile("" : "+v"(root[x][y]));
       // tile_add: C (a bf16 value, never -0) plus bf16(root * scale), one rounding to bf16
 #pragma unroll
       for (int x = 0; x < TM; ++x)
 #pragma unroll
         for (int y = 0; y < TN; ++y) {
           const float r = FIRST_E4 ? root[x][y] * fl.out_scale : root[x][y];
-          if (short_add) C[x][y] = fma_rne(__builtin_fmaf(r, scale[x][y], C[x][y]), 65536.0f);
-          else C[x][y] = bf16_rne(C[x][y] + bf16_rne(r * scale[x][y]));
+          C[x][y] = bf16_rne(C[x][y] + bf16_rne(r * scale[x][y]));
         }
       in_block += SIZE;
       if (in_block == bs) {
@@ -630,7 +610,7 @@ __global__ void __launch_bounds__(256) k_anchor_fast(const TreeArgs args, const 
     // rows past K are zero in LDS (zero codes): their products are zeros and never set the anchor, as the
     // reference's missing products
     for (int r0 = 0; r0 < kend; r0 += size) {
-      if (in_block == 0) block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x, 1u, 0u);
+      if (in_block == 0) block_scales<TM, TN>(args, g, m0 + tm * TM, n0 + tn * TN, scale, max_x);
       float c[TM][TN];
 #pragma unroll
       for (int x = 0; x < TM; ++x)
@@ -824,17 +804,6 @@ bool adder_fast_levels(const int32_t* e, const int32_t* m, int levels, const mxq
   fl->pmask = ~((1u << (23 - ar.prod_m)) - 1u);
   fl->flush_thr = first_e4 ? 0.0f : ar.flush_thr;
   fl->prod_max = prod_max;
-  // The short tile add (scale_denies): a root of at most 8 significant bits, a multiple of level 1's step (e4) or of
-  // a kept product's last bit (bf16), below 2^top, times scales of 2^-L .. 2^H is exact in bf16 and normal when
-  // 2L <= 126 + log2 of that step, and leaves C below 2^112 when top + 2H <= 98: as the systolic kernels' lanes.
-  fl->xs_lo = 1u;                                                    // empty range: always the rounded tile add
-  fl->xs_hi = 0u;
-  const int low = first_e4 ? -(6 + m[0]) : (int)std::floor(std::log2((double)ar.flush_thr)) - ar.prod_m;
-  const int top = (int)std::ceil(std::log2((double)prod_max)) + levels + 1;
-  if ((bf16 || prev <= 7) && 126 + low >= 0 && top <= 98) {
-    fl->xs_lo = (uint32_t)(127 - std::min(59, (126 + low) / 2)) << 23;
-    fl->xs_hi = (uint32_t)(127 + std::max(0, std::min(45, (98 - top) / 2))) << 23;
-  }
   return true;
 }
 
