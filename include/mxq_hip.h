@@ -97,7 +97,7 @@ int mxq_valu_probe(int32_t kind, int32_t iters, int64_t workgroups, float* out, 
 
 /* Fused block quantization: per block, amax -> scale X (step 1) -> z = block / X -> P = element rule (step 2).
  * V: (outer, n, inner) of type v_dtype; P: float32, same shape; X: float32 (outer, ceil(n/bs), inner).
- * The last block along n is zero-padded for the amax.
+ * The last block along n is zero-padded for the amax.  P may be V itself (float32); no other overlap.
  * Replaces mxq/block/_driver.py:45-66 `compose` with the pairs of mxq/block/mxquant.py:26-32,
  * mxq/block/mxgemmini.py:37-59 and mxq/block/ocp.py:35-49. */
 int mxq_block_quantize(const void* V, int32_t v_dtype, float* P, float* X, int64_t outer, int64_t n,
@@ -111,7 +111,8 @@ int mxq_block_quantize(const void* V, int32_t v_dtype, float* P, float* X, int64
 int mxq_block_quantize_t(const void* M, int32_t v_dtype, float* P, float* X, int64_t n, int64_t inner,
                          int64_t block_size, const mxq_block_spec* spec, mxq_stream_t stream);
 
-/* out = P * expand(X) along n.  Replaces mxq/block/_driver.py:69-72 `dequantize`. */
+/* out = P * expand(X) along n; out may be P itself, with no other overlap.  Replaces mxq/block/_driver.py:69-72
+ * `dequantize`. */
 int mxq_block_dequantize(const float* P, const float* X, float* out, int64_t outer, int64_t n, int64_t inner,
                          int64_t block_size, mxq_stream_t stream);
 

@@ -171,10 +171,13 @@ __global__ void __launch_bounds__(256) k_dequant_any(const SRC src, float* __res
 // ROWS > 1 (the source's kRows) once its threads are at least kDequantFill, 8 waves a SIMD.
 constexpr int64_t kDequantFill = 8 * 1024 * 64;
 
+// `in_place`: out is where the float32 codes lie, so no thread may read another's (a last group moved back over its
+// neighbour's columns does): rows that are no whole fours go to the kernels whose groups divide them.
 template <typename SRC>
-void launch_dequant(const SRC& src, float* out, int64_t outer, int64_t n, int64_t inner, int64_t bs, hipStream_t st) {
+void launch_dequant(const SRC& src, float* out, int64_t outer, int64_t n, int64_t inner, int64_t bs, hipStream_t st,
+                    bool in_place = false) {
   const int64_t nb = mxq::ceil_div(n, bs), lim = (int64_t)1 << 31, all = outer * n * inner;
-  if (inner >= 4 && outer * n * mxq::ceil_div(inner, 4) < lim && bs < lim) {
+  if (inner >= 4 && (!in_place || inner % 4 == 0) && outer * n * mxq::ceil_div(inner, 4) < lim && bs < lim) {
     const int64_t groups = mxq::ceil_div(inner, 4);
     auto go = [&](auto rows_const) {
       constexpr int ROWS = decltype(rows_const)::value;
@@ -187,7 +190,7 @@ void launch_dequant(const SRC& src, float* out, int64_t outer, int64_t n, int64_
       go(std::integral_constant<int, SRC::kRows>{});
     else
       go(std::integral_constant<int, 1>{});
-  } else if (inner == 1 && n >= 4 && n < lim && bs >= 4 && bs < lim && outer * mxq::ceil_div(n, 4) < lim) {
+  } else if (inner == 1 && n >= 4 && (!in_place || n % 4 == 0) && n < lim && bs >= 4 && bs < lim && outer * mxq::ceil_div(n, 4) < lim) {
     const int64_t groups = mxq::ceil_div(n, 4), count = outer * groups;
     k_dequant_row<<<mxq::grid_for(count, 256), 256, 0, st>>>(src, out, (uint32_t)count, n, nb,
                                                             mxq::make_divu31((uint32_t)groups),

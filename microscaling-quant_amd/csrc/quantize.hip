@@ -55,7 +55,8 @@ extern "C" int mxq_block_dequantize(const float* P, const float* X, float* out, 
   if (outer < 0 || n < 0 || inner < 0 || block_size < 1) return mxq::invalid("mxq_block_dequantize: bad shape");
   if (outer == 0 || n == 0 || inner == 0) return MXQ_OK;
   if (!P || !X || !out) return mxq::invalid("mxq_block_dequantize: NULL pointer");
-  mxq_quant::launch_dequant(mxq_quant::FloatSource{P, X}, out, outer, n, inner, block_size, mxq::as_stream(stream));
+  mxq_quant::launch_dequant(mxq_quant::FloatSource{P, X}, out, outer, n, inner, block_size, mxq::as_stream(stream),
+                            P == out);
   return mxq::check_launch("mxq_block_dequantize");
 }
 

@@ -1051,9 +1051,13 @@ int launch_quant(const T* V, const SINK& out, int64_t outer, int64_t n, int64_t 
   }
   mxq::KernelTimer timer("block_quantize", st);
   const int64_t nb = mxq::ceil_div(n, bs);
+  // Codes that replace their inputs (P is V): no lane may read another's elements, so rows that a lane's columns do not
+  // divide take fewer columns a lane instead of a last group moved back over its neighbour's.
+  bool in_place = false;
+  if constexpr (SINK::kBytes == 4) in_place = static_cast<const void*>(V) == static_cast<const void*>(out.P);
   // contiguous blocks: rows of whole blocks in any number (no row to find); others count their blocks in 31 bits
   if (inner == 1 && bs == 32 && outer * n >= 4 &&
-      (n % 32 == 0 || (outer * nb < (int64_t(1) << 31) && n < (int64_t(1) << 31)))) {
+      (n % 32 == 0 || (!in_place && outer * nb < (int64_t(1) << 31) && n < (int64_t(1) << 31)))) {
     const int64_t nblocks = outer * nb;
     auto go = [&](auto q_const) {
       constexpr int Q = decltype(q_const)::value;
@@ -1116,13 +1120,14 @@ int launch_quant(const T* V, const SINK& out, int64_t outer, int64_t n, int64_t 
     using Eight = std::integral_constant<int, 8>;
     using Half = std::integral_constant<int, 32>;          // (half a wave to a block column)
     // the kernel indexes waves in 32 bits
-    const int64_t widest = inner >= 4 ? (BYTES && inner >= 8 ? 8 : 4) : (inner % 2 == 0 ? 2 : 1);
+    const bool narrow = inner < 4 || (in_place && inner % 4 != 0);
+    const int64_t widest = !narrow ? (BYTES && inner >= 8 ? 8 : 4) : (inner % 2 == 0 ? 2 : 1);
     if (outer * nb * mxq::ceil_div(mxq::ceil_div(inner, widest), 2) >= (int64_t(1) << 31))
       return mxq::invalid("block quantize: tensor too large (2^31 waves of 2048 elements)");
     const int64_t full = outer * nb * mxq::ceil_div(inner, 4) / 8;
     constexpr bool ENCODE = BYTES && ELEM == MXQ_ELEM_QTORCH;
-    if (inner < 4) {
-      const bool many = outer * nb >= 8 * 1024;
+    if (narrow) {
+      const bool many = outer * nb * mxq::ceil_div(inner, 4) >= 8 * 1024;
       if (inner % 2 == 0) many ? go(Two{}, Eight{}, std::true_type{}) : go(Two{}, Half{}, std::true_type{});
       else many ? go(One{}, Eight{}, std::true_type{}) : go(One{}, Half{}, std::true_type{});
     } else if (full < (ENCODE ? 64 : inner <= 8 ? 128 : HW && BYTES ? 400 : 200)) {

@@ -241,6 +241,35 @@ def test_every_split_of_columns(cuda, method, shape):
     assert_bits_equal(Xe, want[1], f"{method} {shape} X")
 
 
+@pytest.mark.parametrize("method", ["mxgemmini", "mxgemmini rne", "ocp", "mxquant"])
+@pytest.mark.parametrize("shape,axis,bs", [((4100, 517), 0, 32), ((4100, 514), 0, 32), ((33, 37), 0, 32), ((300, 6), 0, 32),
+                                           ((70, 133), 1, 32), ((2100, 1027), 1, 32), ((512, 37), 0, 16), ((64, 35), 1, 6)],
+                         ids=str)
+def test_codes_in_place_of_their_inputs(cuda, method, shape, axis, bs):
+    """mxq_block_quantize with P where V lies and mxq_block_dequantize with its output where P lies, rows that are no
+    whole fours among them: as with arrays of their own."""
+    from mxq import _lib, block
+    g = torch.Generator(device="cuda").manual_seed(shape[1])
+    V = torch.randn(shape, generator=g, device="cuda") * 3
+    name, _, mode = method.partition(" ")
+    kw = {"rounding_mode": mode} if mode else {}
+    calls = []
+    with pytest.MonkeyPatch.context() as mp:                  # the native call's arguments, as block.* makes it
+        run = _lib.run
+        mp.setattr(_lib, "run", lambda *a: (calls.append(a), run(*a))[1])
+        P, X = getattr(block, name).quantize(V, "MXFP8_E4M3", axis=axis, block_size=bs, **kw)
+    want = block.dequantize(P, X, axis=axis, block_size=bs)
+    fn, _, dt, _, _, *rest = next(a for a in calls if a[0] == "mxq_block_quantize")
+    X2 = torch.empty_like(X)
+    with _lib.on(V.device):
+        st = _lib.stream(V.device)
+        _lib.run(fn, _lib.ptr(V), dt, _lib.ptr(V), _lib.ptr(X2), *rest[:-1], st)
+        assert torch.equal(V, P) and torch.equal(X2, X), f"{method} {shape} axis {axis} blocks of {bs}"
+        outer, n, inner = rest[:3]
+        _lib.run("mxq_block_dequantize", _lib.ptr(V), _lib.ptr(X2), _lib.ptr(V), outer, n, inner, bs, st)
+    assert torch.equal(V, want), f"read back {method} {shape} axis {axis} blocks of {bs}"
+
+
 # ------------------------------------------------------------------------------------------ elementwise
 @pytest.fixture(scope="module")
 def corpus():
