@@ -289,10 +289,8 @@ def test_batched_side_by_side_outputs(cuda):
 
 
 def test_all_fast_tile_shapes(cuda):
-    """The fast kernel's three tiles: 2048 x 4096 outputs run on 64 x 64 tiles, 1024 x 4096 on 32 x 64 and
-    500 x 4000 on 32 x 32 (too few larger tiles to give every CU 8 workgroups), with HW_FINAL's instance and a
-    generic ladder, two columns of A past the fast kernel's bound (their tiles, one a tail, are computed by the
-    general kernel): every output equal to the general kernel's alone, edge column slices equal to the
+    """Large grids, whole 64 x 64 tiles and others, with HW_FINAL's instance and a generic ladder, two columns of A
+    past the datapath's bound (their tiles, one a tail, are computed by the general kernel): every output equal to the general kernel's alone, edge column slices equal to the
     oracle's (columns are independent chains)."""
     from mxq import matmul
     rng = np.random.default_rng(8)
@@ -318,11 +316,10 @@ def test_all_fast_tile_shapes(cuda):
 
 @pytest.mark.parametrize("case", [0, 1, 3, 4, 5], ids=lambda i: f"l{i}")
 def test_small_grid_fast_kernel(cuda, case):
-    """Grids of 512 to 1023 tiles of 64 x 64 outputs (512 x 4096 and 1024 x 2048 here) run on the fast kernel
-    that stages 64 rows per step straight into LDS and rounds in value units: every ladder with a last bf16
-    lane, K = 128 and K = 192 (an odd count of 64-row stages), two columns of A past the fast bound (their
-    tiles go to the general kernel).  Every output equal to the general kernel's alone, edge column slices
-    equal to the oracle's.  K = 96 (not a multiple of 64) takes the 32-row kernel, checked the same way."""
+    """Grids of 512 tiles of 64 x 64 outputs, whose kernel stages 64 rows a step: every ladder with a last bf16 lane,
+    K = 128, 192 (an odd count of stages) and 96 (a last stage half full), two columns of A past the fast bound
+    (their tiles go to the general kernel).  Every output equal to the general kernel's alone, edge column slices equal
+    to the oracle's."""
     from mxq import matmul
     size, sched, (pe, pm) = FAST_LADDERS[case]
     rng = np.random.default_rng(40 + case)
@@ -345,7 +342,7 @@ def test_small_grid_fast_kernel(cuda, case):
 
 
 def test_zero_stages_skip_exactly(cuda):
-    """Stages (32 K rows) whose A or B tile is all +-0 are skipped by the fast kernel: a zero block for every
+    """Blocks of 32 K rows whose A or B columns are all +-0, which a kernel may leave out: a zero block for every
     tile, zero blocks for some row or column tiles only, -0 codes, a zero stage whose block scale is not a power
     of two, and a would-be-zero stage holding one NaN (which must not be skipped): every output equal to the
     general kernel's and the oracle's."""
@@ -370,14 +367,13 @@ def test_zero_stages_skip_exactly(cuda):
 
 
 @pytest.mark.parametrize("count,M,N,K", [(32, 512, 512, 160), (32, 512, 512, 192), (3, 200, 300, 160)],
-                         ids=["tiles64", "stages64", "tiles32"])
+                         ids=["tiles64_odd_stage", "tiles64", "small"])
 def test_batched_hints(cuda, count, M, N, K):
     """mxq_systolic_batched's hints change no needed bit.  Skip maps (a causal triangle, random 32 x 32 groups,
     random whole 64 x 64 tiles, everything): each group the map leaves is bit-equal to the hint-free result, each
     it marks is that result or +0, and a fully marked map gives +0 everywhere.  k_end: the true bound of A's
     nonzero rows, and a bound too small for some groups (those tiles fall back to the general kernel), both
-    equal to the hint-free result.  K = 192 runs the 64-row-stage kernel (2048 tiles of 64 x 64), whose
-    stop under k_end rounds up to a whole stage."""
+    equal to the hint-free result.  512 x 512 runs 64 x 64 tiles, whose stop under k_end rounds up to a stage of 64 rows."""
     from mxq import _lib, matmul
     from mxq.matmul._systolic import systolic_batched
     rng = np.random.default_rng(M + K)
@@ -465,11 +461,11 @@ def test_batched_hints_large_orders(cuda, count):
     assert torch.equal(got, want), "k_end changed a result"
 
 
-@pytest.mark.parametrize("count,K,M,N", [(3, 200, 96, 70), (8, 256, 512, 256)], ids=["stages32", "stages64"])
+@pytest.mark.parametrize("count,K,M,N", [(3, 200, 96, 70), (8, 256, 512, 256)], ids=["small", "small_16_rows"])
 def test_k_end_nonfinite_past_the_end(cuda, count, K, M, N):
     """Rows past k_end where A is +-0 but B holds an Inf, or a scale of A's is NaN, or one of B's is Inf: 0 * Inf
     makes NaN there, so those tiles must not stop early.  Every output equals the hint-free run (NaN included).
-    The second shape runs the 64-row-stage kernel, whose stop rounds k_end = 40 up to 64 rows."""
+    (The tiles of 64 and 32 rows: test_hints_and_epilogue_on_every_kernel.)"""
     from mxq import _lib, matmul
     from mxq.matmul._systolic import systolic_batched
     rng = np.random.default_rng(5)
@@ -562,17 +558,19 @@ def test_batched_hint_and_epilogue_errors(cuda):
 
 @pytest.mark.parametrize("ladder", [HW_FINAL, [(4, 5)] * 15 + [(8, 7)], [(4, 4)] * 16, [(4, 9)] * 16],
                          ids=["hw_final", "e4m5_bf16", "e4m4", "e4m9"])
-@pytest.mark.parametrize("K,M,N", [(192, 40, 72), (192, 1024, 1024)], ids=["tiles32", "tiles64"])
-def test_scales_past_the_short_tile_add(cuda, ladder, K, M, N):
+@pytest.mark.parametrize("K,M,N,tile", [(192, 40, 72, ("small", 8, 32)), (192, 1024, 1024, ("tile", 64, 64)),
+                                        (200, 509, 2041, ("tile", 64, 64)), (200, 333, 2041, ("tile", 32, 32))], ids=str)
+def test_scales_past_the_short_tile_add(cuda, ladder, K, M, N, tile):
     """Blocks whose scales leave the short tile add's range (2^46 and more, zero, 1e-38, 2^-60) before and after
     blocks inside it: a sum that a large scale has made large must keep the long rounding in the blocks that
     follow.  Against the general kernel, which is checked against the oracle above."""
     from mxq import matmul
+    assert systolic_plan(K, M, N, matmul.MXGEMMINI(), ladder)[:3] == tile
     rng = np.random.default_rng(K + M)
     ops = []
     for n, lift in ((M, 1.0), (N, 0.5)):
         P, _ = _codes(rng, K, n, scale=lift)
-        X = np.exp2(rng.integers(-3, 3, (K // 32, n))).astype(np.float32)
+        X = np.exp2(rng.integers(-3, 3, (-(-K // 32), n))).astype(np.float32)
         X[1, : n // 2] = np.float32(2.0 ** 46)
         X[1, n // 2] = np.float32(2.0 ** 63)
         X[3, 1::5] = np.float32(1e-38)
@@ -599,9 +597,8 @@ SMALL_LADDERS = {
 @pytest.mark.parametrize("K,M,N", [(1, 1, 1), (96, 1, 17), (4099, 1, 70), (2080, 3, 33), (333, 8, 130), (1000, 17, 64),
                                    (160, 70, 515), (64, 520, 2050)])
 def test_few_outputs(cuda, name, K, M, N):
-    """The kernel for few outputs, at the edges of its tiles (1, 4, 8 and 16 rows, 16 to 64 columns), rounds (of up to
-    4096 rows of K) and K tails, for every datapath it has, against the general kernel (checked against the oracle
-    above)."""
+    """The kernel for few outputs at rounds of up to 4096 rows of K and K tails, for every datapath it has, against the
+    general kernel (checked against the oracle above).  Its tiles one by one: test_every_tile_of_few_outputs."""
     from mxq import matmul
     ar_args, ladder, size = SMALL_LADDERS[name]
     ar = getattr(matmul, ar_args[0])(*ar_args[1:])
@@ -639,8 +636,9 @@ def test_few_outputs_fall_back(cuda, name):
 @pytest.mark.parametrize("K,M,N", [(64, 2048, 2048), (200, 1000, 1030), (77, 2049, 1023), (33, 1030, 2001)],
                          ids=lambda v: str(v))
 def test_tiles_of_any_shape(cuda, name, K, M, N):
-    """Grids of 64 x 64 and 32 x 64 tiles whose operands end inside a tile, a stage or a group of four columns, for
-    every datapath, against the general kernel."""
+    """Grids of 64 x 64 and 32 x 32 tiles (few outputs' tiles for some datapaths) whose operands end inside a tile, a
+    stage or a group of four columns, against the general kernel.  Ragged 64 x 64 tiles:
+    test_tiles64_whose_last_stage_is_part_full."""
     from mxq import matmul
     ar_args, ladder, size = SMALL_LADDERS[name]
     if name == "mxquant_falling_8":
@@ -653,6 +651,86 @@ def test_tiles_of_any_shape(cuda, name, K, M, N):
     got = matmul.systolic(*ops, ar, ladder, size).cpu().numpy()
     want = matmul.systolic(*ops, ar, ladder, size, force_general=True).cpu().numpy()
     assert_bits_equal(got, want, f"{name} {M}x{N}, K={K}")
+
+
+# kernel and tile -> problems, K, M, N, block size; tiles that end inside a group of four columns
+HINT_SHAPES = {("small", 8, 32): (3, 200, 300, 333, 32), ("tile", 32, 32): (2, 200, 333, 2041, 32),
+               ("tile", 64, 64): (2, 200, 509, 2041, 32), ("fast", 32, 64): (2, 200, 509, 2041, 64)}
+
+
+@pytest.mark.parametrize("tile", HINT_SHAPES, ids=str)
+def test_hints_and_epilogue_on_every_kernel(cuda, tile):
+    """Every hint and the epilogue on each kernel that takes them, some of A's columns past the datapath's bound: a skip
+    map with c_end (marked groups hold the result, +0, or what the buffer held where c_end allows it), k_end with Inf and
+    NaN past it (those tiles do not stop early), k_end with a_live (rows of A past it hold NaN: they are not read), and the
+    score step on top of k_end: against the hint-free run, which equals the general kernel's elsewhere in this file."""
+    from mxq import _lib, matmul
+    from mxq.matmul._systolic import systolic_batched
+    from mxq.nn._attention import _mask_rows, _scale_mask
+    count, K, M, N, bs = HINT_SHAPES[tile]
+    ar = matmul.MXGEMMINI()
+    rng = np.random.default_rng(K + M + N)
+    P_A, X_A = _codes(rng, K, count * M)
+    P_B, X_B = _codes(rng, K, count * N, scale=0.1)
+    X_A, X_B = (np.ascontiguousarray(x[:: bs // 32]) for x in (X_A, X_B))
+    g64, gm, gn, gk = -(-M // 64), -(-M // 32), -(-N // 32), -(-K // 32)
+    ends = rng.integers(1, K // 64 + 1, (count, g64)).astype(np.int32) * 64 - rng.integers(0, 20, (count, g64)).astype(np.int32)
+    for z in range(count):
+        for t in range(g64):
+            P_A[ends[z, t]:, z * M + 64 * t: min(z * M + 64 * t + 64, (z + 1) * M)] = 0.0
+    P_A[3, M + 70] = 600.0                                     # problem 1: a tile for the general kernel
+    lay = _lib.SystolicLayout(ld_a=count * M, batch_a=M, ld_xa=count * M, batch_xa=M,
+                              ld_b=count * N, batch_b=N, ld_xb=count * N, batch_xb=N, ld_c=N, batch_c=M * N)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()          # noqa: E731
+
+    def run(ops, epilogue=None, **hints):
+        plan = systolic_plan(K, M, N, ar, HW_FINAL, 16, bs, count, count * M, count * N, **dict.fromkeys(hints, True))
+        assert plan[:3] == tile or {"a_live", "c_end"} & set(hints) or plan[0] == tile[0] == "fast", plan
+        C = torch.full((count, M, N), 7.0, device="cuda")
+        systolic_batched([t(x) for x in ops], lay, count, K, M, N, C, ar, HW_FINAL, 16, bs, epilogue=epilogue,
+                         **{k: t(v) for k, v in hints.items()})
+        return C.cpu().numpy()
+
+    ops = (P_A, X_A, P_B, X_B)
+    want = run(ops)
+    skip = np.triu(np.ones((gm, gn), np.uint8), 1)[None].repeat(count, 0) | (rng.random((count, gm, gn)) < 0.1).astype(np.uint8)
+    full = skip.astype(bool).repeat(32, 1).repeat(32, 2)[:, :M, :N]
+    c_end = np.minimum(64 * (np.arange(g64) + 1), N).astype(np.int32)[None].repeat(count, 0)
+    past = np.zeros((count, M, N), bool)
+    for r in range(g64):
+        past[:, 64 * r: 64 * r + 64, c_end[0, r]:] = True
+    for hints in ({"skip": skip}, {"skip": skip, "k_end": ends}, {"skip": skip, "c_end": c_end}):
+        got = run(ops, **hints)
+        assert_bits_equal(got[~full], want[~full], f"groups left {list(hints)}")
+        same = (got.view(np.uint32) == want.view(np.uint32)) | (got.view(np.uint32) == 0)
+        assert (same | ((got == 7.0) & past & ("c_end" in hints)))[full].all(), f"marked groups {list(hints)}"
+    assert_bits_equal(run(ops, k_end=ends), want, "k_end")
+    wrong = np.maximum(ends - 70, 0)
+    assert_bits_equal(run(ops, k_end=wrong), want, "k_end that some tiles pass")
+    live = np.zeros((count, gk, gm), np.uint8)
+    garbage = P_A.copy()
+    for z in range(count):
+        for k in range(gk):
+            for c in range(gm):
+                piece = (slice(32 * k, 32 * k + 32), slice(z * M + 32 * c, min(z * M + 32 * c + 32, (z + 1) * M)))
+                live[z, k, c] = P_A[piece].any()
+                if 32 * k >= ends[z, c // 2]:
+                    garbage[piece] = np.nan
+    assert_bits_equal(run((garbage, X_A, P_B, X_B), k_end=ends, a_live=live), want, "a_live")
+    assert_bits_equal(run(ops, k_end=ends, a_live=live), want, "a_live, zeros past k_end")
+    bad = [x.copy() for x in ops]
+    bad[2][K - 3, 5] = np.inf
+    bad[3][-1, N + 40] = np.nan
+    bad_want = run(bad)
+    assert np.isnan(bad_want).any()
+    assert_bits_equal(run(bad, k_end=ends), bad_want, "non-finite values past k_end")
+    bias = torch.from_numpy(rng.standard_normal((1, M, N)).astype(np.float32) * 3).cuda()
+    mask, b_stride, r_stride = _mask_rows(bias, 0, count, 0)
+    epi = _lib.SystolicEpilogue(scale=0.088388, bf16=1, mask=_lib.ptr(mask), mask_b_stride=b_stride,
+                                mask_row_stride=r_stride, z0=0, z_per_b=count, m=M)
+    scored = torch.from_numpy(want).cuda()
+    _scale_mask(scored, bias, 0.088388, "bf16", 1, M, 0, count, 0)
+    assert_bits_equal(run(ops, epi, k_end=ends), scored.cpu().numpy(), "the score step")
 
 
 @pytest.mark.parametrize("M,K,ld", [(1, 1100, 4_198_405), (4, 300, (1 << 24) + 1)])
