@@ -42,7 +42,8 @@ HBM_PEAK_GBS = 8000.0
 VALU_LANE_OPS = 157.3e12 / 2
 # The emulated MAC's VALU issue on gfx950 in full-rate slots: an e4 lane step multiplies, masks the product,
 # rounds it to the lane grid (adding and subtracting a constant, two full-rate operations, or v_rndne_f32 at half
-# rate: 2 slots either way), adds exactly and rounds to nearest even at m bits (three full-rate operations) = 8.
+# rate: 2 slots either way), adds exactly and rounds to nearest even at m bits (a multiplication and an fma, two
+# full-rate operations) = 7.
 # The roof prices every MAC at that step.
 SLOTS_PER_MAC_MODEL = 7
 VALU_ROOF_TOPS = VALU_LANE_OPS / SLOTS_PER_MAC_MODEL * 2 / 1e12   # 22.47 TOP/s emulated

@@ -82,7 +82,8 @@ int mxq_version(void);
  * dominant kernel's own duration, not the whole call's).  With mxq_timer_enable(1), every later launch of a
  * timed kernel records a pair of HIP events on its stream.  mxq_timer_read waits for the pairs recorded under
  * `kernel`, returns their summed milliseconds and their number, and forgets them.  Timed kernels:
- * "systolic_fast", "systolic_general", "block_quantize", "lut_kmeans", "mx_mfma", "adder_fast", "adder_tree",
+ * "systolic_fast" (the tile kernel's and the register-staged one's), "systolic_small", "systolic_general",
+ * "block_quantize", "lut_quant", "lut_pick_codes", "mx_pack_bytes", "lut_kmeans", "mx_mfma", "adder_fast", "adder_tree",
  * "anchor_fast", "anchor_tree".  Not for use under graph capture. */
 int mxq_timer_enable(int32_t on);
 int mxq_timer_read(const char* kernel, double* total_ms, int64_t* launches);
@@ -186,9 +187,9 @@ typedef struct mxq_systolic_layout {
  *          a_live[(z * ceil(K/32) + s) * ceil(M/32) + g] != 0 unless every code of A in those rows and columns
  *          is +-0 and every block scale over them finite.  The pass then reads B only.  A byte that wrongly
  *          says 0 for a stage some tile leaves out gives wrong results: this one is a promise, not a hint.
- *          When the fast kernel runs (mxq_systolic_fast_lanes), a tile it hands to the general kernel for
- *          another reason is recomputed over the same rows when its left-out rows passed the check, so rows of
- *          A past k_end whose a_live bytes are 0 are never read: they need not hold codes or scales at all.
+ *          For lanes that mxq_systolic_fast_lanes takes, a tile handed to the general kernel for another reason
+ *          is recomputed over the same rows when its left-out rows passed the check, so rows of A past k_end whose
+ *          a_live bytes are 0 are never read: they need not hold codes or scales at all.
  *   c_end  with skip: per problem z and 64-row group t of C, a fast tile made only of skipped groups whose first
  *          column is at or past c_end[z * ceil(M/64) + t] is not stored at all (those outputs keep what the
  *          buffer held).  Attention's scores past a 64-row group's last seen key are never read: the softmax
@@ -200,9 +201,10 @@ typedef struct mxq_systolic_hints {
   const int32_t* c_end;
 } mxq_systolic_hints;
 
-/* 1 when mxq_systolic and mxq_systolic_batched run the fast kernel for these lanes and this arithmetic (any
- * other case runs the general kernel alone, which reads every row of A and computes every tile), else 0.  No
- * counterpart in the reference: a caller that leaves rows of A unwritten under k_end asks this first. */
+/* 1 when, for these lanes and this arithmetic (MXGEMMINI's e4 lanes, the last one bf16 or not), mxq_systolic_batched given
+ * k_end and a_live never reads the rows of A that a_live leaves out, and under c_end leaves tiles unstored; else 0: the
+ * wide and MXQUANT datapaths and the general kernel may read every row of A.  No counterpart in the reference: a caller
+ * that leaves rows of A unwritten under k_end asks this first. */
 int mxq_systolic_fast_lanes(const int32_t* lane_e, const int32_t* lane_m, int32_t size, const mxq_arith_spec* arith);
 
 /* Which kernel a systolic call of this shape runs, and on what tile of outputs a workgroup; no counterpart in the

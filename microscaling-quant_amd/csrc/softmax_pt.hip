@@ -36,7 +36,7 @@ constexpr int H = 2;          // 64-row groups per workgroup
 constexpr int RB = 64 * H;    // rows per workgroup
 constexpr int NT = 256 * H;   // threads per workgroup: 4 waves per row group
 // The most rows k_softmax_row takes: at 2048 keys 8192 rows take it 113 us and k_softmax_pt 204, 16,384 rows 361
-// and 206; at 256 keys 17 and 39, 32 and 42.
+// and 206; at 256 keys 17 and 39, 32 and 42 (one line for every key count: the row kernel's is later with few keys).
 constexpr int64_t kRowKernelRows = 8192;
 static_assert(H == 2, "a workgroup pairs a front and a back row group");
 

@@ -857,8 +857,6 @@ FastLanes make_fast_lanes(const int32_t* e, const int32_t* m, int size, const mx
     if (prev >= 0) fl.rescale[i] = pow2f(mi - prev);
     fl.split[i] = (float)((1u << (23 - mi)) + 1u);
     fl.magic[i] = 1.5f * pow2f(17 - mi);
-    fl.pw[i] = (float)(1u << (23 - mi));
-    fl.low[i] = 1.0f - fl.pw[i];
     prev = mi;
   }
   fl.out_scale = pow2f(-(6 + prev));

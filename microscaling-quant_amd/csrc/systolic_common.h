@@ -33,8 +33,7 @@ struct SysArgs {
   int64_t kend_groups;    // ceil(M / 64): 64-column groups of A, 64-row groups of C
   const int32_t* c_end;   // per problem and 64-row group of C: skipped tiles from this column on are not stored
   // dispatch position (blockIdx.x + tiles_x * (blockIdx.y + tiles_y * blockIdx.z)) -> fast tile
-  // (z * tiles_y + ty) * tiles_x + tx, by descending work (k_tile_order); NULL: the grid's own tile, rows last
-  // first
+  // (z * tiles_y + ty) * tiles_x + tx, by descending work (k_tile_order); NULL: the grid's own tile
   const uint32_t* order;
   // with an order and skip: bit 31 of an order entry set when its tile is skipped (tile_skipped at the fast tile
   // size, as k_tile_bucket found it), so the fast kernels read no skip bytes; the tile is the low 31 bits
@@ -117,7 +116,7 @@ struct FastLanes {
   uint32_t pmask;        // product truncation to prod_m fraction bits
   float flush_thr;       // bf16 lane: |product| below this becomes zero
   uint32_t xs_lo, xs_hi; // scale magnitudes (bit patterns) that allow the short tile add
-  float pw[32], low[32]; // P = 2^(23 - m_i) and 1 - P: fma_rne's constants
+  float pw[32], low[32]; // P = 2^(23 - m_i) and 1 - P: fma_rne's constants (kWide's lanes only)
   // MXQUANT's grids (Qtorch): the product's and the lanes'
   Qtorch prod, lane[32];
 };

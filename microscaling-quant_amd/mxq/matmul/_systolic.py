@@ -6,9 +6,10 @@ is multiplied by the scale map and added into the output by tile_add.  `size` mu
 K tail: the last reduction leaves the column after its last real product, as MXQuant's `_simulate_atw`.
 
 With MXGEMMINI or MXQUANT (or compiled(...) of them) the whole call is one HIP launch sequence on the GPU
-(include/mxq_hip.h mxq_systolic): every output element's chain is computed in order by one thread, the K
-loop staged through LDS.  A hand-made Arithmetic, or a size the kernel does not take (it needs size | 32),
-runs the reference's loop with the Arithmetic's own callables.
+(include/mxq_hip.h mxq_systolic): every output element's sums are added in the order of K.  With few outputs
+the waves of a workgroup take reductions of K in turn and their sums are added in that order.  A hand-made
+Arithmetic, or a size the kernel does not take (it needs size | 32), runs the reference's loop with the
+Arithmetic's own callables.
 """
 from typing import Optional, Sequence, Tuple
 
