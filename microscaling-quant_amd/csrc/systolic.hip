@@ -1010,7 +1010,7 @@ constexpr Shape kShapes[] = {
     // (HW_FINAL: 512 x 2048 outputs at K = 32 and 2048, then 200 x 2048)
     {Plan::kTile, 64, 6, 8, 5.1, 2.2, 61, 215, 278, {1, 1.35, 1.40, 2.39, 2.10, 2.10}},    // 13, 282; 12, 293
     {Plan::kTile, 32, 5, 4, 5.9, 0.6, 60, 55, 164, {1, 1.32, 1.36, 2.24, 1.96, 1.96}},     // 14, 286; 10, 181
-    {Plan::kSmall, 16, 6, 8, 2.4, 1.1, 22, 74, 105, {1, 0, 0, 2.00, 0, 0}},                // 28, 322; 15, 160
+    {Plan::kSmall, 16, 6, 8, 2.4, 1.1, 22, 74, 105, {1, 0, 0, 2.06, 0, 0}},                // 28, 322; 15, 160
     {Plan::kSmall, 8, 6, 8, 2.5, 1.1, 14, 43, 64, {1, 1.28, 1.28, 1.83, 1.70, 1.70}},      // 34, 369; 19, 183
     {Plan::kSmall, 8, 6, 16, 1.9, 2.5, 0, 51, 0, {1, 0, 0, 1.86, 0, 0}},                   // 74, 422; 38, 205
     {Plan::kSmall, 8, 5, 16, 2.1, 1.5, 0, 31, 0, {1, 0, 0, 1.70, 0, 0}},                   // 147, 514; 66, 214

@@ -62,3 +62,8 @@ MEASURED = {(64, 4, 4096): [(8, 64), (8, 32)], (64, 333, 2048): [(32, 32)], (64,
 @pytest.mark.parametrize("K,M,N", MEASURED, ids=str)
 def test_measured_choices(K, M, N):
     assert _plan("hw_final", K, M, N)[1:3] in MEASURED[K, M, N]
+
+
+def test_measured_choice_mxquant():
+    """MXQUANT(4, 3) under HW_FINAL, 512 x 2048 outputs of K = 2048: 32 x 32 tiles 625 us, 16-row tiles of few outputs 640."""
+    assert _plan("mxquant", 2048, 512, 2048)[:3] == ("tile", 32, 32)
