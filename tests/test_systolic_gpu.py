@@ -160,6 +160,39 @@ def test_fast_guards(cuda):
         assert_bits_equal(_run(pa, xa, pb, xb, ar, HW_FINAL), want, what)
 
 
+@pytest.mark.parametrize("what", ["nan scale", "inf scale", "scale product overflows", "huge a, tiny b", "products above 8",
+                                  "subnormal code", "off-grid codes"])
+@pytest.mark.parametrize("tile,M,N,block", [(("tile", 32, 32), 333, 2041, 32), (("tile", 64, 64), 509, 2041, 32),
+                                            (("fast", 32, 32), 509, 2041, 64)], ids=str)
+def test_guards_on_every_tile(cuda, tile, M, N, block, what):
+    """test_fast_guards' operands (which run the kernel for few outputs there) on each tile kernel, in some tiles, against
+    the general kernel."""
+    from mxq import matmul
+    K, ar = 200, matmul.MXGEMMINI()
+    assert systolic_plan(K, M, N, ar, HW_FINAL, 16, block)[:3] == tile
+    rng = np.random.default_rng(6)
+    P_A, X_A = _codes(rng, K, M)
+    P_B, X_B = _codes(rng, K, N, scale=0.1)
+    X_A, X_B = (np.ascontiguousarray(x[:: block // 32]) for x in (X_A, X_B))
+    if what == "nan scale":
+        X_A[1, 70] = np.nan
+    elif what == "inf scale":
+        X_B[2, 1500] = np.inf
+    elif what == "scale product overflows":
+        X_A[0, 100:200], X_B[0, :70] = np.float32(2.0 ** 100), np.float32(2.0 ** 100)
+    elif what == "huge a, tiny b":
+        P_A[3, 72] = np.float32(2.0 ** 110)
+        P_B[:, 700:900] = (P_B[:, 700:900] * np.float32(2.0 ** -120)).astype(np.float32)
+    elif what == "products above 8":
+        P_A[197, 305] = 448.0
+    elif what == "subnormal code":
+        P_A[7, 300] = np.float32(1e-40)
+    else:
+        P_A[:, 64:96] += np.float32(1e-3)
+    ops = (P_A, X_A, P_B, X_B)
+    assert_bits_equal(_run(*ops, ar, HW_FINAL, 16, block), _run(*ops, ar, HW_FINAL, 16, block, force_general=True), what)
+
+
 @pytest.mark.parametrize("prod_floor,edge", [(-16, 53), (-40, 41), (-126, 53)])
 def test_tile_add_scale_ranges(cuda, prod_floor, edge):
     """The fast kernel adds S * scale into C without rounding S * scale first only for blocks whose scales are
@@ -782,9 +815,20 @@ def test_other_blocks_on_the_register_staged_kernel(cuda, name, block, tile):
     """Blocks of other sizes than 32 on k_systolic_fast's three tiles, whose operands end inside a tile, a stage and a
     block: scales that leave the short tile add's range (one of them large, ahead of blocks inside it), a tile of zeros
     and codes past the fast bound, against the general kernel."""
-    from mxq import matmul
     _, ladder, size = {**SMALL_LADDERS, "e4m6_32": (None, [(4, 6)] * 32, 32)}[name]
-    K, M, N = FAST_TILES[tile]
+    _on_the_register_staged_kernel(*FAST_TILES[tile], ladder, size, block, tile)
+
+
+@pytest.mark.parametrize("name,tile,K,M,N", [("e4m4", "64x64", 202, 1024, 4096), ("e4m5_bf16_8", "64x64", 202, 1024, 4096),
+                                             ("e4m5_bf16_8", "32x64", 202, 2048, 1000), ("e4m6_32", "32x32", 330, 512, 4100)])
+def test_blocks_of_32_on_the_register_staged_kernel(cuda, name, tile, K, M, N):
+    """The ladders and shapes that k_systolic_fast takes with blocks of 32, whose scales its 32-row tiles stage in LDS."""
+    _, ladder, size = {**SMALL_LADDERS, "e4m6_32": (None, [(4, 6)] * 32, 32)}[name]
+    _on_the_register_staged_kernel(K, M, N, ladder, size, 32, tile)
+
+
+def _on_the_register_staged_kernel(K, M, N, ladder, size, block, tile):
+    from mxq import matmul
     assert systolic_plan(K, M, N, matmul.MXGEMMINI(), ladder, size, block)[:3] == ("fast", *map(int, tile.split("x")))
     g = torch.Generator(device="cuda").manual_seed(M + block)
     P = [torch.randn(K, n, generator=g, device="cuda").mul_(s).to(torch.float8_e4m3fn).float() for n, s in ((M, 1.0), (N, 0.5))]
