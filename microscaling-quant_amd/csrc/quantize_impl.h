@@ -1,8 +1,8 @@
 // Fused MX block quantization for gfx950.
 //
 // A tensor is viewed as (outer, n, inner) with the block axis n in the middle.  Three layouts:
-//   split    (block 32): eight lanes of a wavefront share one block column of VEC adjacent columns, four rows
-//            each; their maxima meet through cross-lane exchanges; the block stays in registers.
+//   split    (block 32): eight lanes of a wavefront (or 32) share one block column of VEC adjacent columns, four rows
+//            each (or one); their maxima meet through cross-lane exchanges; the block stays in registers.
 //   row      (inner == 1, block 32): eight lanes own one contiguous block, four elements each.
 //   strided  (any other block size): one thread per block column, the block read twice.
 // Kernels are specialised on the element rule and, for the OCP grid and the microxcaling step, on the

@@ -303,8 +303,8 @@ def test_trees_against_reference_fixtures(cuda, case):
                          ids=["readme", "bf16", "e4m7", "e4m9", "size32"])
 @pytest.mark.parametrize("K,M,N", [(192, 40, 72), (192, 2048, 4096)], ids=["tiles32", "tiles64"])
 def test_adder_scales_past_the_short_tile_add(cuda, size, levels, K, M, N):
-    """Blocks whose scales leave the short tile add's range before and after blocks inside it, against the general
-    kernel (checked against the oracle above)."""
+    """Scales past the range in which a tile could be added with one rounding (2^46 and more, subnormal, zero) before and
+    after blocks inside it, on both heights of tile, against the general kernel (checked against the oracle above)."""
     from mxq import matmul
     rng = np.random.default_rng(size + M)
     ops = []
